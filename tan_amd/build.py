@@ -15,7 +15,9 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-I" + os.path.join(ROOT, "include")]
 
-SOURCES = ["tan_kernels.hip", "tan_room.hip", "tan_noalloc.hip", "tan_engine.cpp", "tan_api.cpp", "tan_wav.cpp"]
+# (source, extra flags): tan_kernels.hip in its parts, the slowest to compile first
+SOURCES = [("tan_kernels.hip", [f"-DTANX_PART={k}"]) for k in (1, 2, 3, 4, 0)] + [
+    (s, []) for s in ("tan_room.hip", "tan_noalloc.hip", "tan_engine.cpp", "tan_api.cpp", "tan_wav.cpp")]
 
 
 def build_library(verbose=False, jobs=None):
@@ -26,12 +28,12 @@ def build_library(verbose=False, jobs=None):
     os.makedirs(objdir, exist_ok=True)
     out = os.path.join(LIBDIR, "libtan_mi355x.so")
     tmp = out + ".tmp"
-    srcs = [os.path.join(CSRC, s) for s in SOURCES]
-    objs = [os.path.join(objdir, os.path.basename(s) + ".o") for s in srcs]
+    srcs = [(os.path.join(CSRC, s), flags) for s, flags in SOURCES]
+    objs = [os.path.join(objdir, "".join([s] + [f.rsplit("=", 1)[-1] for f in flags]) + ".o") for s, flags in SOURCES]
 
     def compile_one(pair):
-        src, obj = pair
-        cmd = [HIPCC] + HIP_FLAGS + ["-c", "-o", obj, src]
+        (src, flags), obj = pair
+        cmd = [HIPCC] + HIP_FLAGS + flags + ["-c", "-o", obj, src]
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.check_call(cmd)

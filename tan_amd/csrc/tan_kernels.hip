@@ -23,6 +23,15 @@
 #include <map>
 #include <mutex>
 
+// This file compiles whole, or in parts of about equal compile time built in
+// parallel (TANX_PART): 0 the launchers' dispatch on the IR type, 1 + IrType
+// the convolution kernels of one IR type, 4 TANFFT, time domain, output chain.
+#ifdef TANX_PART
+#define TANX_IN(part) (TANX_PART == (part))
+#else
+#define TANX_IN(part) 1
+#endif
+
 namespace tanx {
 
 // Loads and stores through the global address space.  A pointer read from
@@ -1673,6 +1682,7 @@ __global__ __launch_bounds__(256) void k_ir_transform_rows_group(const IrArgs *_
     ir_transform_rows_part<M, NR>(a, local % chunks, local / chunks, s0, s1, tw, twn);
 }
 
+#if TANX_IN(4)
 // ---------------------------------------------------------------------------
 // TANFFT transforms, one workgroup per channel.  M is the complex FFT size
 // (N for complex directions, N/2 for real ones).
@@ -2085,10 +2095,12 @@ __global__ void k_zero(float4 *p, size_t n4)
         p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
+#endif  // TANX_IN(4)
+
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-static inline int fft_threads(int M)
+[[maybe_unused]] static inline int fft_threads(int M)
 {
     int t = M / 4;
     if (t < 64) t = 64;
@@ -2109,7 +2121,7 @@ static inline int fft_threads(int M)
 // With ev0/ev1, the launch itself records the kernel's start and end (the
 // dispatch's own timestamps), so event timing measures the kernel alone.
 template <int HT>
-static hipError_t launch_tick_t(int B, int tail_nf, const TickArgs &a, hipStream_t s, unsigned blocks,
+hipError_t launch_tick_t(int B, int tail_nf, const TickArgs &a, hipStream_t s, unsigned blocks,
                                 hipEvent_t ev0, hipEvent_t ev1)
 {
     const int tk = a.nchunk == 0 ? 0 : (is_pass(a) ? 2 : 1);
@@ -2149,33 +2161,11 @@ static hipError_t launch_tick_t(int B, int tail_nf, const TickArgs &a, hipStream
     return hipGetLastError();
 }
 
-hipError_t launch_tick(int B, int tail_nf, const TickArgs &a, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
-{
-    const unsigned blocks = (unsigned)(a.nhead + a.C * a.nchunk + a.C * a.nchB);
-    if (blocks == 0) return hipSuccess;
-    switch (a.irtype) {
-    case IR_F32: return launch_tick_t<IR_F32>(B, tail_nf, a, s, blocks, ev0, ev1);
-    case IR_F16: return launch_tick_t<IR_F16>(B, tail_nf, a, s, blocks, ev0, ev1);
-    case IR_BF16: return launch_tick_t<IR_BF16>(B, tail_nf, a, s, blocks, ev0, ev1);
-    default: return hipErrorInvalidValue;
-    }
-}
-
 template <int HT>
-static hipError_t launch_desc_t(int B, const TickArgs *d, int k, unsigned blocks, hipStream_t s)
+hipError_t launch_desc_t(int B, const TickArgs *d, int k, unsigned blocks, hipStream_t s)
 {
     TANX_SWITCH_B(B, hipLaunchKernelGGL((k_tick_desc<M, HT>), dim3(blocks), dim3(kTickThreads), 0, s, d, k));
     return hipGetLastError();
-}
-
-hipError_t launch_tick_desc(int B, int irtype, const TickArgs *d_descs, int k, unsigned blocks, hipStream_t s)
-{
-    switch (irtype) {
-    case IR_F32: return launch_desc_t<IR_F32>(B, d_descs, k, blocks, s);
-    case IR_F16: return launch_desc_t<IR_F16>(B, d_descs, k, blocks, s);
-    case IR_BF16: return launch_desc_t<IR_BF16>(B, d_descs, k, blocks, s);
-    default: return hipErrorInvalidValue;
-    }
 }
 
 template <int HT, int M>
@@ -2203,7 +2193,7 @@ static hipError_t launch_group_m(int roles, int km, const TickArgs *d, const int
 }
 
 template <int HT>
-static hipError_t launch_group_t(int B, int roles, int km, const TickArgs *d, const int *st, int nobj,
+hipError_t launch_group_t(int B, int roles, int km, const TickArgs *d, const int *st, int nobj,
                                  unsigned blocks, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
 {
     switch (B) {
@@ -2215,23 +2205,8 @@ static hipError_t launch_group_t(int B, int roles, int km, const TickArgs *d, co
     }
 }
 
-hipError_t launch_group_tick(int irtype, int B, int roles, int km, const TickArgs *d_descs, const int *d_starts,
-                             int nobj, unsigned blocks, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
-{
-    if (blocks == 0) return hipSuccess;
-    hipError_t e;
-    switch (irtype) {
-    case IR_F32: e = launch_group_t<IR_F32>(B, roles, km, d_descs, d_starts, nobj, blocks, s, ev0, ev1); break;
-    case IR_F16: e = launch_group_t<IR_F16>(B, roles, km, d_descs, d_starts, nobj, blocks, s, ev0, ev1); break;
-    case IR_BF16: e = launch_group_t<IR_BF16>(B, roles, km, d_descs, d_starts, nobj, blocks, s, ev0, ev1); break;
-    default: return hipErrorInvalidValue;
-    }
-    if (e != hipSuccess) return e;
-    return hipGetLastError();
-}
-
 // Resident workgroups of one kernel on the current device (cached per kernel)
-static unsigned resident_blocks(const void *kernel)
+[[maybe_unused]] static unsigned resident_blocks(const void *kernel)
 {
     static std::mutex mtx;
     static std::map<std::pair<int, const void *>, unsigned> cache;
@@ -2285,7 +2260,7 @@ static hipError_t launch_queue_m(int roles, int km, const TickArgs *d, const int
 }
 
 template <int HT>
-static hipError_t launch_queue_t(int B, int roles, int km, const TickArgs *d, const int *st, int nobj, int total,
+hipError_t launch_queue_t(int B, int roles, int km, const TickArgs *d, const int *st, int nobj, int total,
                                  int *next, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
 {
     switch (B) {
@@ -2297,23 +2272,8 @@ static hipError_t launch_queue_t(int B, int roles, int km, const TickArgs *d, co
     }
 }
 
-hipError_t launch_group_queue(int irtype, int B, int roles, int km, const TickArgs *d_descs, const int *d_starts,
-                              int nobj, int total, int *next, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
-{
-    if (total <= 0) return hipSuccess;
-    hipError_t e;
-    switch (irtype) {
-    case IR_F32: e = launch_queue_t<IR_F32>(B, roles, km, d_descs, d_starts, nobj, total, next, s, ev0, ev1); break;
-    case IR_F16: e = launch_queue_t<IR_F16>(B, roles, km, d_descs, d_starts, nobj, total, next, s, ev0, ev1); break;
-    case IR_BF16: e = launch_queue_t<IR_BF16>(B, roles, km, d_descs, d_starts, nobj, total, next, s, ev0, ev1); break;
-    default: return hipErrorInvalidValue;
-    }
-    if (e != hipSuccess) return e;
-    return hipGetLastError();
-}
-
 template <int HT>
-static hipError_t launch_heads_t(int B, const HeadBatchArgs &h, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
+hipError_t launch_heads_t(int B, const HeadBatchArgs &h, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
 {
     const dim3 g((unsigned)h.C), t(kTickThreads);
 #define TANX_HEADS(MM)                                                                            \
@@ -2332,7 +2292,7 @@ static hipError_t launch_heads_t(int B, const HeadBatchArgs &h, hipStream_t s, h
 }
 
 template <int HT>
-static hipError_t launch_window_t(int B, int tail_nf, const HeadBatchArgs &h, const TickArgs &a, hipStream_t s,
+hipError_t launch_window_t(int B, int tail_nf, const HeadBatchArgs &h, const TickArgs &a, hipStream_t s,
                                   hipEvent_t ev0, hipEvent_t ev1)
 {
     const dim3 grid((unsigned)(h.C + a.C * a.nchunk));
@@ -2354,6 +2314,183 @@ static hipError_t launch_window_t(int B, int tail_nf, const HeadBatchArgs &h, co
 #undef TANX_WINDOW_K
     return hipGetLastError();
 }
+
+// partition sizes of uniform blocks (64..1024) and of frames (128..4096)
+#define TANX_SWITCH_PART(B, CALL)                        \
+    switch (B) {                                         \
+    case 64: { constexpr int M = 64; CALL; } break;      \
+    case 128: { constexpr int M = 128; CALL; } break;    \
+    case 256: { constexpr int M = 256; CALL; } break;    \
+    case 512: { constexpr int M = 512; CALL; } break;    \
+    case 1024: { constexpr int M = 1024; CALL; } break;  \
+    case 2048: { constexpr int M = 2048; CALL; } break;  \
+    case 4096: { constexpr int M = 4096; CALL; } break;  \
+    default: return hipErrorInvalidValue;                \
+    }
+
+template <int HT>
+hipError_t launch_ir_transform_group_t(int B, const IrArgs *d_descs, const int *d_starts, int n, unsigned blocks,
+                                       hipStream_t s)
+{
+    const dim3 g(blocks);
+    if constexpr (HT == IR_F32) {
+        switch (B) {
+        case 64: hipLaunchKernelGGL((k_ir_transform_rows_group<64, 4>), g, dim3(256), 0, s, d_descs, d_starts, n); break;
+        case 128: hipLaunchKernelGGL((k_ir_transform_rows_group<128, 4>), g, dim3(256), 0, s, d_descs, d_starts, n); break;
+        case 256: hipLaunchKernelGGL((k_ir_transform_rows_group<256, 4>), g, dim3(256), 0, s, d_descs, d_starts, n); break;
+        case 512: hipLaunchKernelGGL((k_ir_transform_rows_group<512, 2>), g, dim3(256), 0, s, d_descs, d_starts, n); break;
+        case 1024: hipLaunchKernelGGL((k_ir_transform_group<1024, HT>), g, dim3(fft_threads(1024)), 0, s, d_descs, d_starts, n); break;
+        case 2048: hipLaunchKernelGGL((k_ir_transform_group<2048, HT>), g, dim3(fft_threads(2048)), 0, s, d_descs, d_starts, n); break;
+        case 4096: hipLaunchKernelGGL((k_ir_transform_group<4096, HT>), g, dim3(fft_threads(4096)), 0, s, d_descs, d_starts, n); break;
+        default: return hipErrorInvalidValue;
+        }
+    } else {
+        TANX_SWITCH_PART(B, hipLaunchKernelGGL((k_ir_transform_group<M, HT>), g, dim3(fft_threads(M)), 0, s, d_descs,
+                                               d_starts, n));
+    }
+    return hipGetLastError();
+}
+
+template <int HT>
+hipError_t launch_ir_transform_t(int B, int nchan, const IrArgs &a, hipStream_t s)
+{
+    if constexpr (HT == IR_F32) {
+        // short partitions: several rows per workgroup
+        const dim3 g4((unsigned)((a.P + 3) / 4), (unsigned)nchan), g2((unsigned)((a.P + 1) / 2), (unsigned)nchan);
+        const dim3 g1((unsigned)a.P, (unsigned)nchan);
+        switch (B) {
+        case 64: hipLaunchKernelGGL((k_ir_transform_rows<64, 4>), g4, dim3(256), 0, s, a); break;
+        case 128: hipLaunchKernelGGL((k_ir_transform_rows<128, 4>), g4, dim3(256), 0, s, a); break;
+        case 256: hipLaunchKernelGGL((k_ir_transform_rows<256, 4>), g4, dim3(256), 0, s, a); break;
+        case 512: hipLaunchKernelGGL((k_ir_transform_rows<512, 2>), g2, dim3(256), 0, s, a); break;
+        case 1024: hipLaunchKernelGGL((k_ir_transform<1024, HT>), g1, dim3(fft_threads(1024)), 0, s, a); break;
+        case 2048: hipLaunchKernelGGL((k_ir_transform<2048, HT>), g1, dim3(fft_threads(2048)), 0, s, a); break;
+        case 4096: hipLaunchKernelGGL((k_ir_transform<4096, HT>), g1, dim3(fft_threads(4096)), 0, s, a); break;
+        default: return hipErrorInvalidValue;
+        }
+    } else {
+        TANX_SWITCH_PART(B, hipLaunchKernelGGL((k_ir_transform<M, HT>), dim3(a.P, nchan), dim3(fft_threads(M)), 0, s, a));
+    }
+    return hipGetLastError();
+}
+
+#define TANX_SWITCH_FRAME(N, CALL)                       \
+    switch (N) {                                         \
+    case 128: { constexpr int F = 128; CALL; } break;    \
+    case 256: { constexpr int F = 256; CALL; } break;    \
+    case 512: { constexpr int F = 512; CALL; } break;    \
+    case 1024: { constexpr int F = 1024; CALL; } break;  \
+    case 2048: { constexpr int F = 2048; CALL; } break;  \
+    case 4096: { constexpr int F = 4096; CALL; } break;  \
+    default: return hipErrorInvalidValue;                \
+    }
+
+template <int HT>
+hipError_t launch_frame_t(const FrameArgs &a, hipStream_t s, hipEvent_t ev1)
+{
+    TANX_SWITCH_FRAME(a.N, hipExtLaunchKernelGGL((k_frame<F, HT>), dim3(a.C), dim3(frame_threads<F>()), 0, s, nullptr, ev1, 0, a));
+    return hipGetLastError();
+}
+
+template <int HT>
+hipError_t launch_group_frame_t(const FrameArgs *d_descs, const int *d_starts, int nobj, unsigned blocks, hipStream_t s,
+                                hipEvent_t ev0, hipEvent_t ev1)
+{
+    hipExtLaunchKernelGGL((k_group_frame<HT>), dim3(blocks), dim3(kGroupFrameThreads), 0, s, ev0, ev1, 0, d_descs,
+                          d_starts, nobj);
+    return hipGetLastError();
+}
+
+// The typed launchers of one IR type, compiled in that type's part
+#define TANX_TYPED(PRE, HT)                                                                                          \
+    PRE template hipError_t launch_tick_t<HT>(int, int, const TickArgs &, hipStream_t, unsigned, hipEvent_t,        \
+                                              hipEvent_t);                                                          \
+    PRE template hipError_t launch_desc_t<HT>(int, const TickArgs *, int, unsigned, hipStream_t);                   \
+    PRE template hipError_t launch_group_t<HT>(int, int, int, const TickArgs *, const int *, int, unsigned,         \
+                                               hipStream_t, hipEvent_t, hipEvent_t);                                \
+    PRE template hipError_t launch_queue_t<HT>(int, int, int, const TickArgs *, const int *, int, int, int *,       \
+                                               hipStream_t, hipEvent_t, hipEvent_t);                                \
+    PRE template hipError_t launch_heads_t<HT>(int, const HeadBatchArgs &, hipStream_t, hipEvent_t, hipEvent_t);    \
+    PRE template hipError_t launch_window_t<HT>(int, int, const HeadBatchArgs &, const TickArgs &, hipStream_t,     \
+                                                hipEvent_t, hipEvent_t);                                            \
+    PRE template hipError_t launch_ir_transform_group_t<HT>(int, const IrArgs *, const int *, int, unsigned,        \
+                                                            hipStream_t);                                           \
+    PRE template hipError_t launch_ir_transform_t<HT>(int, int, const IrArgs &, hipStream_t);                       \
+    PRE template hipError_t launch_frame_t<HT>(const FrameArgs &, hipStream_t, hipEvent_t);                         \
+    PRE template hipError_t launch_group_frame_t<HT>(const FrameArgs *, const int *, int, unsigned, hipStream_t,    \
+                                                     hipEvent_t, hipEvent_t);
+#if TANX_IN(1)
+TANX_TYPED(, IR_F32)
+#endif
+#if TANX_IN(2)
+TANX_TYPED(, IR_F16)
+#endif
+#if TANX_IN(3)
+TANX_TYPED(, IR_BF16)
+#endif
+
+#if TANX_IN(0)
+#ifdef TANX_PART
+TANX_TYPED(extern, IR_F32)
+TANX_TYPED(extern, IR_F16)
+TANX_TYPED(extern, IR_BF16)
+#endif
+
+hipError_t launch_tick(int B, int tail_nf, const TickArgs &a, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
+{
+    const unsigned blocks = (unsigned)(a.nhead + a.C * a.nchunk + a.C * a.nchB);
+    if (blocks == 0) return hipSuccess;
+    switch (a.irtype) {
+    case IR_F32: return launch_tick_t<IR_F32>(B, tail_nf, a, s, blocks, ev0, ev1);
+    case IR_F16: return launch_tick_t<IR_F16>(B, tail_nf, a, s, blocks, ev0, ev1);
+    case IR_BF16: return launch_tick_t<IR_BF16>(B, tail_nf, a, s, blocks, ev0, ev1);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+
+hipError_t launch_tick_desc(int B, int irtype, const TickArgs *d_descs, int k, unsigned blocks, hipStream_t s)
+{
+    switch (irtype) {
+    case IR_F32: return launch_desc_t<IR_F32>(B, d_descs, k, blocks, s);
+    case IR_F16: return launch_desc_t<IR_F16>(B, d_descs, k, blocks, s);
+    case IR_BF16: return launch_desc_t<IR_BF16>(B, d_descs, k, blocks, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+
+hipError_t launch_group_tick(int irtype, int B, int roles, int km, const TickArgs *d_descs, const int *d_starts,
+                             int nobj, unsigned blocks, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
+{
+    if (blocks == 0) return hipSuccess;
+    hipError_t e;
+    switch (irtype) {
+    case IR_F32: e = launch_group_t<IR_F32>(B, roles, km, d_descs, d_starts, nobj, blocks, s, ev0, ev1); break;
+    case IR_F16: e = launch_group_t<IR_F16>(B, roles, km, d_descs, d_starts, nobj, blocks, s, ev0, ev1); break;
+    case IR_BF16: e = launch_group_t<IR_BF16>(B, roles, km, d_descs, d_starts, nobj, blocks, s, ev0, ev1); break;
+    default: return hipErrorInvalidValue;
+    }
+    if (e != hipSuccess) return e;
+    return hipGetLastError();
+}
+
+
+hipError_t launch_group_queue(int irtype, int B, int roles, int km, const TickArgs *d_descs, const int *d_starts,
+                              int nobj, int total, int *next, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
+{
+    if (total <= 0) return hipSuccess;
+    hipError_t e;
+    switch (irtype) {
+    case IR_F32: e = launch_queue_t<IR_F32>(B, roles, km, d_descs, d_starts, nobj, total, next, s, ev0, ev1); break;
+    case IR_F16: e = launch_queue_t<IR_F16>(B, roles, km, d_descs, d_starts, nobj, total, next, s, ev0, ev1); break;
+    case IR_BF16: e = launch_queue_t<IR_BF16>(B, roles, km, d_descs, d_starts, nobj, total, next, s, ev0, ev1); break;
+    default: return hipErrorInvalidValue;
+    }
+    if (e != hipSuccess) return e;
+    return hipGetLastError();
+}
+
 
 hipError_t launch_window(int B, int tail_nf, const HeadBatchArgs &h, const TickArgs &a, hipStream_t s,
                          hipEvent_t ev0, hipEvent_t ev1)
@@ -2380,18 +2517,6 @@ hipError_t launch_heads(int B, int irtype, const HeadBatchArgs &h, hipStream_t s
     }
 }
 
-// partition sizes of uniform blocks (64..1024) and of frames (128..4096)
-#define TANX_SWITCH_PART(B, CALL)                        \
-    switch (B) {                                         \
-    case 64: { constexpr int M = 64; CALL; } break;      \
-    case 128: { constexpr int M = 128; CALL; } break;    \
-    case 256: { constexpr int M = 256; CALL; } break;    \
-    case 512: { constexpr int M = 512; CALL; } break;    \
-    case 1024: { constexpr int M = 1024; CALL; } break;  \
-    case 2048: { constexpr int M = 2048; CALL; } break;  \
-    case 4096: { constexpr int M = 4096; CALL; } break;  \
-    default: return hipErrorInvalidValue;                \
-    }
 
 int ir_transform_blocks(int B, int irtype, int P, int nchan)
 {
@@ -2404,107 +2529,50 @@ hipError_t launch_ir_transform_group(int B, int irtype, const IrArgs *d_descs, c
                                      unsigned blocks, hipStream_t s)
 {
     if (n == 0 || blocks == 0) return hipSuccess;
-    const dim3 g(blocks);
     switch (irtype) {
-    case IR_F32:
-        if (B <= 256) {
-            switch (B) {
-            case 64: hipLaunchKernelGGL((k_ir_transform_rows_group<64, 4>), g, dim3(256), 0, s, d_descs, d_starts, n); break;
-            case 128: hipLaunchKernelGGL((k_ir_transform_rows_group<128, 4>), g, dim3(256), 0, s, d_descs, d_starts, n); break;
-            case 256: hipLaunchKernelGGL((k_ir_transform_rows_group<256, 4>), g, dim3(256), 0, s, d_descs, d_starts, n); break;
-            default: return hipErrorInvalidValue;
-            }
-        } else if (B == 512) {
-            hipLaunchKernelGGL((k_ir_transform_rows_group<512, 2>), g, dim3(256), 0, s, d_descs, d_starts, n);
-        } else {
-            TANX_SWITCH_PART(B, hipLaunchKernelGGL((k_ir_transform_group<M, IR_F32>), g, dim3(fft_threads(M)), 0, s,
-                                                   d_descs, d_starts, n));
-        }
-        break;
-    case IR_F16:
-        TANX_SWITCH_PART(B, hipLaunchKernelGGL((k_ir_transform_group<M, IR_F16>), g, dim3(fft_threads(M)), 0, s,
-                                               d_descs, d_starts, n));
-        break;
-    case IR_BF16:
-        TANX_SWITCH_PART(B, hipLaunchKernelGGL((k_ir_transform_group<M, IR_BF16>), g, dim3(fft_threads(M)), 0, s,
-                                               d_descs, d_starts, n));
-        break;
-    default:
-        return hipErrorInvalidValue;
+    case IR_F32: return launch_ir_transform_group_t<IR_F32>(B, d_descs, d_starts, n, blocks, s);
+    case IR_F16: return launch_ir_transform_group_t<IR_F16>(B, d_descs, d_starts, n, blocks, s);
+    case IR_BF16: return launch_ir_transform_group_t<IR_BF16>(B, d_descs, d_starts, n, blocks, s);
+    default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_ir_transform(int B, int nchan, const IrArgs &a, hipStream_t s)
 {
     if (a.P == 0 || nchan == 0) return hipSuccess;
     switch (a.irtype) {
-    case IR_F32:
-        // short partitions: several rows per workgroup
-        if (B <= 256) {
-            const dim3 g((unsigned)((a.P + 3) / 4), (unsigned)nchan);
-            switch (B) {
-            case 64: hipLaunchKernelGGL((k_ir_transform_rows<64, 4>), g, dim3(256), 0, s, a); break;
-            case 128: hipLaunchKernelGGL((k_ir_transform_rows<128, 4>), g, dim3(256), 0, s, a); break;
-            case 256: hipLaunchKernelGGL((k_ir_transform_rows<256, 4>), g, dim3(256), 0, s, a); break;
-            default: return hipErrorInvalidValue;
-            }
-        } else if (B == 512) {
-            hipLaunchKernelGGL((k_ir_transform_rows<512, 2>), dim3((unsigned)((a.P + 1) / 2), (unsigned)nchan), dim3(256),
-                               0, s, a);
-        } else {
-            TANX_SWITCH_PART(B, hipLaunchKernelGGL((k_ir_transform<M, IR_F32>), dim3(a.P, nchan), dim3(fft_threads(M)), 0, s, a));
-        }
-        break;
-    case IR_F16:
-        TANX_SWITCH_PART(B, hipLaunchKernelGGL((k_ir_transform<M, IR_F16>), dim3(a.P, nchan), dim3(fft_threads(M)), 0, s, a));
-        break;
-    case IR_BF16:
-        TANX_SWITCH_PART(B, hipLaunchKernelGGL((k_ir_transform<M, IR_BF16>), dim3(a.P, nchan), dim3(fft_threads(M)), 0, s, a));
-        break;
-    default:
-        return hipErrorInvalidValue;
+    case IR_F32: return launch_ir_transform_t<IR_F32>(B, nchan, a, s);
+    case IR_F16: return launch_ir_transform_t<IR_F16>(B, nchan, a, s);
+    case IR_BF16: return launch_ir_transform_t<IR_BF16>(B, nchan, a, s);
+    default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
-
-#define TANX_SWITCH_FRAME(N, CALL)                       \
-    switch (N) {                                         \
-    case 128: { constexpr int F = 128; CALL; } break;    \
-    case 256: { constexpr int F = 256; CALL; } break;    \
-    case 512: { constexpr int F = 512; CALL; } break;    \
-    case 1024: { constexpr int F = 1024; CALL; } break;  \
-    case 2048: { constexpr int F = 2048; CALL; } break;  \
-    case 4096: { constexpr int F = 4096; CALL; } break;  \
-    default: return hipErrorInvalidValue;                \
-    }
 
 hipError_t launch_frame(int irtype, const FrameArgs &a, hipStream_t s, hipEvent_t ev1)
 {
     if (a.C == 0) return hipSuccess;
     switch (irtype) {
-    case IR_F32: TANX_SWITCH_FRAME(a.N, hipExtLaunchKernelGGL((k_frame<F, IR_F32>), dim3(a.C), dim3(frame_threads<F>()), 0, s, nullptr, ev1, 0, a)); break;
-    case IR_F16: TANX_SWITCH_FRAME(a.N, hipExtLaunchKernelGGL((k_frame<F, IR_F16>), dim3(a.C), dim3(frame_threads<F>()), 0, s, nullptr, ev1, 0, a)); break;
-    case IR_BF16: TANX_SWITCH_FRAME(a.N, hipExtLaunchKernelGGL((k_frame<F, IR_BF16>), dim3(a.C), dim3(frame_threads<F>()), 0, s, nullptr, ev1, 0, a)); break;
+    case IR_F32: return launch_frame_t<IR_F32>(a, s, ev1);
+    case IR_F16: return launch_frame_t<IR_F16>(a, s, ev1);
+    case IR_BF16: return launch_frame_t<IR_BF16>(a, s, ev1);
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_group_frame(int irtype, const FrameArgs *d_descs, const int *d_starts, int nobj, unsigned blocks,
                               hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
 {
     if (blocks == 0 || nobj == 0) return hipSuccess;
-    const dim3 g(blocks), t(kGroupFrameThreads);
     switch (irtype) {
-    case IR_F32: hipExtLaunchKernelGGL((k_group_frame<IR_F32>), g, t, 0, s, ev0, ev1, 0, d_descs, d_starts, nobj); break;
-    case IR_F16: hipExtLaunchKernelGGL((k_group_frame<IR_F16>), g, t, 0, s, ev0, ev1, 0, d_descs, d_starts, nobj); break;
-    case IR_BF16: hipExtLaunchKernelGGL((k_group_frame<IR_BF16>), g, t, 0, s, ev0, ev1, 0, d_descs, d_starts, nobj); break;
+    case IR_F32: return launch_group_frame_t<IR_F32>(d_descs, d_starts, nobj, blocks, s, ev0, ev1);
+    case IR_F16: return launch_group_frame_t<IR_F16>(d_descs, d_starts, nobj, blocks, s, ev0, ev1);
+    case IR_BF16: return launch_group_frame_t<IR_BF16>(d_descs, d_starts, nobj, blocks, s, ev0, ev1);
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
+#endif  // TANX_IN(0)
 
+#if TANX_IN(4)
 static hipError_t launch_fft4_pass(bool rows, int size, int channels, const Fft4Pass &p, hipStream_t s)
 {
     const unsigned tiles = (unsigned)((1ll << p.logM) / kFft4Tile);
@@ -2679,5 +2747,7 @@ hipError_t launch_zero(void *p, size_t bytes, hipStream_t s)
     hipLaunchKernelGGL(k_zero, dim3((unsigned)blocks), dim3(256), 0, s, reinterpret_cast<float4 *>(p), n4);
     return hipGetLastError();
 }
+
+#endif  // TANX_IN(4)
 
 }  // namespace tanx
