@@ -2120,15 +2120,32 @@ __global__ __launch_bounds__(64 * kDftWaves) void k_dft_mfma(const float *__rest
 // Output chain: mixer and sample converter (grid-stride, one sample per lane).
 // ---------------------------------------------------------------------------
 // Sum of the channels in channel order (the reference's order), channel c at
-// ins[c] (device pointer list) or at in + c * stride.
-__global__ void k_mix(const float *const *__restrict__ ins, const float *__restrict__ in, long long stride,
-                      int channels, long long n, float *__restrict__ out)
+// ins[c] (LIST: device pointer list) or at in + c * stride.  A block of audio
+// is a few hundred samples, so the sum is one lane's chain of loads: the
+// channels' samples are loaded kMixBatch at a time (one memory round trip)
+// and then added in order, on workgroups of one wave that spread over the
+// compute units: 2.9 instead of 8.8 us for 32 channels of 256 samples.
+constexpr int kMixBatch = 16, kMixThreads = 64;
+
+template <bool LIST>
+__global__ __launch_bounds__(kMixThreads) void k_mix(const float *const *__restrict__ ins,
+                                                     const float *__restrict__ in, long long stride, int channels,
+                                                     long long n, float *__restrict__ out)
 {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
         float acc = 0.f;
-        for (int c = 0; c < channels; c++) {
-            const float v = ins ? ins[c][i] : in[(size_t)c * stride + i];
-            acc = c == 0 ? v : acc + v;
+        for (int c0 = 0; c0 < channels; c0 += kMixBatch) {
+            float v[kMixBatch];
+            // channels past the last one load it again, unused
+#pragma unroll
+            for (int u = 0; u < kMixBatch; u++) {
+                const int c = min(c0 + u, channels - 1);
+                if constexpr (LIST) v[u] = gld(ins[c] + i);
+                else v[u] = in[(size_t)c * stride + i];
+            }
+#pragma unroll
+            for (int u = 0; u < kMixBatch; u++)
+                if (c0 + u < channels) acc = c0 + u == 0 ? v[u] : acc + v[u];
         }
         out[i] = acc;
     }
@@ -2788,7 +2805,9 @@ hipError_t launch_mix(const float *const *d_ins, const float *d_in, long long st
                       float *d_out, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_mix, dim3(io_blocks(n)), dim3(256), 0, s, d_ins, d_in, stride, channels, n, d_out);
+    const dim3 g((unsigned)std::min<long long>((n + kMixThreads - 1) / kMixThreads, 16384)), t(kMixThreads);
+    if (d_ins) hipLaunchKernelGGL((k_mix<true>), g, t, 0, s, d_ins, d_in, stride, channels, n, d_out);
+    else hipLaunchKernelGGL((k_mix<false>), g, t, 0, s, d_ins, d_in, stride, channels, n, d_out);
     return hipGetLastError();
 }
 

@@ -43,3 +43,23 @@ def test_time_domain_ragged_calls_and_tap_ranges(gpu_ctx, L, B, C, calls):
         bound = (n_ir / 8 + 4) * U * np.einsum("cnk,ck->cn", np.abs(win), np.abs(hz))
         assert np.all(np.abs(y - ref) <= bound + 1e-30), np.abs(y - ref).max()
     conv.Terminate()
+
+
+@pytest.mark.parametrize("n,channels", [(1, 1), (63, 15), (64, 16), (65, 17), (256, 32), (1000, 33)])
+def test_mix_sums_in_channel_order(gpu_ctx, n, channels):
+    import torch
+    rng = np.random.default_rng(n + channels)
+    x = rng.standard_normal((channels, n + 3)).astype(np.float32)
+    ref = x[0, :n].copy()
+    for c in range(1, channels):
+        ref = ref + x[c, :n]
+    m = T.TANMixer(gpu_ctx)
+    assert m.Init(n, channels) == T.AMF_OK
+    d = torch.from_numpy(x).cuda()
+    for inputs in (d, [d[c] for c in range(channels)]):
+        out = torch.full((n + 2,), 5.0, device="cuda")
+        assert m.Mix(inputs, out) == T.AMF_OK
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.cpu().numpy()[:n], ref)
+        assert (out[n:] == 5.0).all()
+    m.Terminate()
