@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 
 // This file compiles whole, or in parts of about equal compile time built in
 // parallel (TANX_PART): 0 the launchers' dispatch on the IR type, 1 + IrType
@@ -244,6 +245,13 @@ constexpr int kHeadPreload = 4;      // near partitions a head loads together
 // [filter (<= 2)][lane group G][row float4 H] per round, G * H = 256 * V
 template <int M>
 constexpr int tail_red_float4() { return 2 * kTickThreads * ((M / 2 > 256) ? (M / 2) / 256 : 1); }
+// the same for a pass of KM outputs and NF filters, which also folds its sums there
+template <int M, int NF, int HT, int KM>
+constexpr int pass_red_float4()
+{
+    const int folds = HT == IR_F32 ? (KM + NF - 1) * kTickThreads / 2 : 0;
+    return folds > tail_red_float4<M>() ? folds : tail_red_float4<M>();
+}
 
 // Streamed rows (IR spectra, FDL) are read once per block: nontemporal loads
 // keep them from displacing reused data in the caches.  A multi-block pass
@@ -718,255 +726,323 @@ __device__ void mac_rows(const MacView &w, float4 *red)
     }
 }
 
-// One lane group's share of a split pass: outputs [OFF, OFF + KH) over every
-// partition of the chunk, the window and accumulators of KH outputs per lane;
-// output OFF + k reads FDL row (tbase + OFF + k - i), so the loop is the
-// pass's own with base and gap moved by OFF.  Sums go out directly.
-template <int M, int NF, int HT, bool NT, int KH, int OFF>
-__device__ void tailk_half(const TickArgs &a, int c, int j)
-{
-    constexpr int H = M / 2;                     // float4 per row
-    constexpr int V = H > 256 ? H / 256 : 1;     // float4 per lane per row
-    constexpr int R = H / V;                     // lanes per row
-    constexpr int U = 4;                         // partitions loaded together (8 measured slower)
-    static_assert(KH >= 1 && KH <= kPassMax, "pass length");
-    constexpr size_t kRowBytes = (size_t)M * IrRow<HT>::kBytes;
-    const int tid = threadIdx.x;
-    const int r = tid % R;
-    const float4 *F = reinterpret_cast<const float4 *>(a.fdl) + (size_t)c * a.P * H;
-    const char *HA = reinterpret_cast<const char *>(a.tHa) + (size_t)c * a.P * kRowBytes;
-    const char *HB = NF == 2 ? reinterpret_cast<const char *>(a.tHb) + (size_t)c * a.P * kRowBytes : nullptr;
-    const float *SA = HT == IR_F32 ? nullptr : a.tSa + (size_t)c * a.P;
-    const float *SB = (HT == IR_F32 || NF == 1) ? nullptr : a.tSb + (size_t)c * a.P;
-    const int mask = a.P - 1, base = a.tbase + OFF, kn = a.kn - OFF, gap = a.kgap + OFF;
-    const int i0 = 2 + j * a.pc, i1 = min(a.P, i0 + a.pc);
-    const int p0 = i0, p1 = i1;
-    bool wantA[KH], wantB[KH];
-#pragma unroll
-    for (int k = 0; k < KH; k++) {
-        wantA[k] = k < kn && a.kTA[OFF + k] != nullptr;
-        wantB[k] = NF == 2 && k < kn && a.kTB[OFF + k] != nullptr;
-    }
-    if (kn <= 0) return;  // a pass of at most OFF outputs: none of this group's
-    const bool dc0 = (r == 0);
-    const float s0 = dc0 ? 0.f : 1.f;
-    auto frow = [&](int row, int v) { return ld_row<NT>(F + (size_t)(row & mask) * H + v * R + r); };
-    auto hrow2 = [&](const char *row, int q) { return NT ? IrRow<HT>::get2(row, q) : IrRow<HT>::getc(row, q); };
+// ---------------------------------------------------------------------------
+// Sweep of a multi-output pass: acc[k] += X_{base + k - i} H_i over
+// partitions i in [p0, p1) for KM consecutive outputs k.  Every IR row and
+// FDL row is read once and used for every output: a lane keeps the last KM
+// FDL rows in registers (win).  The loop is unrolled over kBody partitions,
+// so that every index into the window is static and the window moves once
+// per kBody partitions.
+//
+// A lane owns E complex bins of the row: one (8-byte loads, 4 KM registers
+// of window and sums) for FP32 rows, two for 16-bit rows (8-byte loads of
+// them), which leaves registers for the next U partitions' rows to be in
+// flight while U are multiplied and for 4 to 7 waves per SIMD.  Rows longer
+// than the workgroup's lanes cover are swept a slice of S bins at a time.  An
+// output costs four multiply-adds per bin and partition: the packed (DC,
+// Nyquist) element's two real products are the same four with a zero and a
+// swapped factor, chosen once per partition (mac_bin).  Bound by HBM: the
+// 12-output pass of 1,024 channels x 65,536 taps at B = 256 takes 201 us (5.3
+// TB/s of rows), 247 us with two bins per lane, two lane groups and no loads
+// in flight across a stage (167 VGPRs instead of 104).  Ordinary instead of
+// nontemporal loads: 7% slower; stages of 2 partitions: 4% slower, of 6: no
+// faster.
+// ---------------------------------------------------------------------------
+template <int E>
+struct Bins {
+    float re[E], im[E];
+};
 
-    float4 accA[KH][V], accB[KH][V], xw[KH][V];
-#pragma unroll
-    for (int k = 0; k < KH; k++)
-#pragma unroll
-        for (int v = 0; v < V; v++) {
-            accA[k][v] = make_float4(0.f, 0.f, 0.f, 0.f);
-            accB[k][v] = make_float4(0.f, 0.f, 0.f, 0.f);
-            // the window as it stands before partition p0: xw[k] = row (base + k + 1 - p0)
-            // (output k + 1 reads it at p0), loaded only where some output uses it
-            xw[k][v] = (k + 1 < KH && p0 < p1 && p0 >= k + 2 + gap) ? frow(base + k + 1 - p0, v)
-                                                                     : make_float4(0.f, 0.f, 0.f, 0.f);
+constexpr int kFold = 64;  // partitions an FP32 sum runs over before it is folded into LDS
+
+template <int M, int HT>
+struct PassGeo {
+    static constexpr int E = HT == IR_F32 ? 1 : 2;                      // bins per lane
+    static constexpr int S = M < E * kTickThreads ? M : E * kTickThreads;  // bins per slice
+    static constexpr int R = S / E;                                     // lanes per slice
+    static constexpr int G = kTickThreads / R;                          // lane groups
+};
+
+// Bins of lane r of a row's slice (NT: nontemporal)
+template <int E, bool NT>
+__device__ __forceinline__ Bins<E> ld_bins(const float2 *row, int r)
+{
+    Bins<E> b;
+    if constexpr (E == 1) {
+        v2f w;
+        if constexpr (NT) w = __builtin_nontemporal_load((const gmem_t<v2f> *)(row + r));
+        else w = *(const gmem_t<v2f> *)(row + r);
+        b.re[0] = w.x;
+        b.im[0] = w.y;
+    } else {
+        const float4 w = ld_row<NT>(reinterpret_cast<const float4 *>(row) + r);
+        b.re[0] = w.x;
+        b.im[0] = w.y;
+        b.re[1] = w.z;
+        b.im[1] = w.w;
+    }
+    return b;
+}
+
+// Lane r's bins of an IR row's slice as stored, and their values
+template <int HT>
+struct IrBins {
+    v2u raw;
+    template <bool NT>
+    __device__ __forceinline__ void load(const char *row, int r)
+    {
+        const gmem_t<v2u> *p = (const gmem_t<v2u> *)row + r;
+        raw = NT ? __builtin_nontemporal_load(p) : *p;
+    }
+    __device__ __forceinline__ Bins<2> value(float s) const
+    {
+        Bins<2> b;
+        if constexpr (HT == IR_F16) {
+            b.re[0] = half_lo(raw.x) * s;
+            b.im[0] = half_hi(raw.x) * s;
+            b.re[1] = half_lo(raw.y) * s;
+            b.im[1] = half_hi(raw.y) * s;
+        } else {
+            b.re[0] = bf_lo(raw.x) * s;
+            b.im[0] = bf_hi(raw.x) * s;
+            b.re[1] = bf_lo(raw.y) * s;
+            b.im[1] = bf_hi(raw.y) * s;
         }
-    for (int i = p0; i < p1; i += U) {
-        float4 xn[U][V], ha[U][V], hb[U][V];
+        return b;
+    }
+};
+
+template <>
+struct IrBins<IR_F32> {
+    Bins<1> raw;
+    template <bool NT>
+    __device__ __forceinline__ void load(const char *row, int r)
+    {
+        raw = ld_bins<1, NT>(reinterpret_cast<const float2 *>(row), r);
+    }
+    __device__ __forceinline__ Bins<1> value(float) const { return raw; }
+};
+
+// acc += x h for one bin: hc the factor of the cross products (h.im, 0 for
+// the packed element), hd the factor of x.im in the imaginary part (h.re;
+// packed: h.im).  The products and their order are mac4's.
+__device__ __forceinline__ void mac_bin(float &re, float &im, float xr, float xi, float hr, float hc, float hd)
+{
+    re = fmaf(xr, hr, re);
+    re = fmaf(-xi, hc, re);
+    im = fmaf(xr, hc, im);
+    im = fmaf(xi, hd, im);
+}
+
+// Rows of one channel's sweep.  Row rel (relative to output 0's block) is
+// FDL slot (base + rel) & mask for rel < 0 and row rel of `fresh` from 0 on
+// (the spectra of a call's own blocks; nullptr in a pass, which reads rows
+// before the launch's heads only); rows from `zero_from` on count as zero.
+// Both pointers are at the slice.
+struct SweepRows {
+    const float2 *F;
+    const float2 *fresh;
+    int base, mask, zero_from;
+    template <int M>
+    __device__ __forceinline__ const float2 *at(int rel) const
+    {
+        return rel < 0 || !fresh ? F + (size_t)((base + rel) & mask) * M : fresh + (size_t)rel * M;
+    }
+};
+
+// dc: the lane's first bin is the packed (DC, Nyquist) element.
+// A sum of FP32 rows is folded into LDS every kFold partitions (fold: one
+// float2 per output and thread), which keeps its rounding error below that of
+// one chain over the chunk: 64 terms and the chunk's folds.
+// NF filters: HA for outputs k < kA, HB (NF = 2) for outputs k >= kB; with
+// one filter every output is computed (the caller stores those it wants).
+template <int M, int NF, int HT, bool NT, int KM>
+__device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA, const char *HB, const float *SA,
+                                           const float *SB, int p0, int p1, int r, bool dc, int kA, int kB,
+                                           Bins<PassGeo<M, HT>::E> (&accA)[KM], Bins<PassGeo<M, HT>::E> (&accB)[KM],
+                                           float2 *fold)
+{
+    constexpr int E = PassGeo<M, HT>::E;
+    constexpr int U = 4;                                                // partitions per stage
+    constexpr int kBody = NF == 2 ? U : KM < 8 ? 8 : KM;  // partitions per loop trip
+    constexpr size_t kRowBytes = (size_t)M * IrRow<HT>::kBytes;
+    static_assert(kBody % U == 0 && kFold >= kBody && KM <= kPassMax, "pass length");
+    // entry KM - 1 + q of the window holds the row of partition i + q (row
+    // -(i + q)) for the trip starting at partition i; output k reads the
+    // entry k before it
+    Bins<E> win[KM - 1 + kBody];
+#pragma unroll
+    for (int k = 0; k < KM; k++)
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            accA[k].re[e] = accA[k].im[e] = 0.f;
+            accB[k].re[e] = accB[k].im[e] = 0.f;
+            if (k > 0) win[KM - 1 - k].re[e] = win[KM - 1 - k].im[e] = 0.f;
+        }
+    if (p0 >= p1) return;
+#pragma unroll
+    for (int k = 1; k < KM; k++)
+        if (k - p0 < rows.zero_from) win[KM - 1 - k] = ld_bins<E, NT>(rows.at<M>(k - p0), r);
+
+    struct Stage {
+        Bins<E> x[U];
+        IrBins<HT> a[U], b[NF == 2 ? U : 1];
         float sa[U], sb[U];
+    } cur, nxt;
+    // the rows of partitions i .. i + U - 1 (past the end: the last one's again)
+    auto load = [&](Stage &t, int i) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int ii = i + u;
-            sa[u] = 1.f;
-            sb[u] = 1.f;
-            if (ii < p1) {
-                sa[u] = row_scale<HT>(SA, ii);
-                if (NF == 2) sb[u] = row_scale<HT>(SB, ii);
-            }
-#pragma unroll
-            for (int v = 0; v < V; v++) {
-                if (ii < p1) {
-                    xn[u][v] = frow(base - ii, v);
-                    ha[u][v] = hrow2(HA + (size_t)ii * kRowBytes, v * R + r);
-                    if (NF == 2) hb[u][v] = hrow2(HB + (size_t)ii * kRowBytes, v * R + r);
-                }
+            const int ii = min(i + u, p1 - 1);
+            t.x[u] = ld_bins<E, NT>(rows.at<M>(-ii), r);
+            t.a[u].template load<NT>(HA + (size_t)ii * kRowBytes, r);
+            if constexpr (HT != IR_F32) t.sa[u] = gld(SA + ii);
+            if constexpr (NF == 2) {
+                t.b[u].template load<NT>(HB + (size_t)ii * kRowBytes, r);
+                if constexpr (HT != IR_F32) t.sb[u] = gld(SB + ii);
             }
         }
+    };
+    // output k's fold slot (the filters' outputs together are at most KM + 1)
+    auto slot = [&](int f, int k) { return fold + (k + f) * kTickThreads + threadIdx.x; };
+    // adds the sums into their slots (the first time: stores them), clearing
+    // them, or at the end the slots into the sums
+    auto fold_sums = [&](bool first, bool last) {
+        if constexpr (E == 1) {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int ii = i + u;
-            if (ii >= p1) break;
+            for (int f = 0; f < NF; f++)
 #pragma unroll
-            for (int v = 0; v < V; v++) {
+                for (int k = 0; k < KM; k++) {
+                    if (NF == 2 && !(f == 0 ? k < kA : k >= kB)) continue;
+                    Bins<E> &s = f == 0 ? accA[k] : accB[k];
+                    float2 t = make_float2(s.re[0], s.im[0]);
+                    if (!first) t = cadd(*slot(f, k), t);
+                    if (!last) *slot(f, k) = t;
+                    s.re[0] = last ? t.x : 0.f;
+                    s.im[0] = last ? t.y : 0.f;
+                }
+        }
+    };
+    int next_fold = p0 + kFold;
+    load(cur, p0);
+    for (int i = p0; i < p1; i += kBody) {
+        if (E == 1 && i >= next_fold) {
+            fold_sums(next_fold == p0 + kFold, false);
+            next_fold += kFold;
+        }
 #pragma unroll
-                for (int k = KH - 1; k > 0; k--) xw[k][v] = xw[k - 1][v];
-                xw[0][v] = xn[u][v];
-                const bool dc = dc0 && v == 0;
-                const float sv = v == 0 ? s0 : 1.f;
-                const float4 hA = HT == IR_F32 ? ha[u][v] : scale4(ha[u][v], sa[u]);
-                float4 hB = hA;
-                if (NF == 2) hB = HT == IR_F32 ? hb[u][v] : scale4(hb[u][v], sb[u]);
+        for (int q0 = 0; q0 < kBody; q0 += U) {
+            load(nxt, i + q0 + U);
 #pragma unroll
-                for (int k = 0; k < KH; k++) {
-                    if (ii >= k + 1 + gap) {
-                        if (wantA[k]) mac4(accA[k][v], xw[k][v], hA, sv, dc);
-                        if (NF == 2 && wantB[k]) mac4(accB[k][v], xw[k][v], hB, sv, dc);
+            for (int u = 0; u < U; u++) {
+                const int q = q0 + u;
+                if (i + q < p1) {
+                    win[KM - 1 + q] = cur.x[u];
+                    const Bins<E> hA = cur.a[u].value(HT == IR_F32 ? 1.f : cur.sa[u]);
+#pragma unroll
+                    for (int e = 0; e < E; e++) {
+                        const float hr = hA.re[e], hi = hA.im[e];
+                        const float hc = e == 0 && dc ? 0.f : hi, hd = e == 0 && dc ? hi : hr;
+#pragma unroll
+                        for (int k = 0; k < KM; k++)
+                            if (NF == 1 || k < kA) {
+                                const Bins<E> &x = win[KM - 1 + q - k];
+                                mac_bin(accA[k].re[e], accA[k].im[e], x.re[e], x.im[e], hr, hc, hd);
+                            }
+                    }
+                    if constexpr (NF == 2) {
+                        const Bins<E> hB = cur.b[u].value(HT == IR_F32 ? 1.f : cur.sb[u]);
+#pragma unroll
+                        for (int e = 0; e < E; e++) {
+                            const float hr = hB.re[e], hi = hB.im[e];
+                            const float hc = e == 0 && dc ? 0.f : hi, hd = e == 0 && dc ? hi : hr;
+#pragma unroll
+                            for (int k = 0; k < KM; k++)
+                                if (k >= kB) {
+                                    const Bins<E> &x = win[KM - 1 + q - k];
+                                    mac_bin(accB[k].re[e], accB[k].im[e], x.re[e], x.im[e], hr, hc, hd);
+                                }
+                        }
                     }
                 }
             }
+            cur = nxt;
         }
+#pragma unroll
+        for (int k = 0; k < KM - 1; k++) win[k] = win[k + kBody];
     }
-    const size_t orow = ((size_t)c * a.nchunk + j) * H;
+    if (E == 1 && next_fold > p0 + kFold) fold_sums(false, true);
+}
+
+// One output row's slice of a sweep: the lane groups' sums, added in group
+// order through red ([G][S] complex), or the one group's directly.  All
+// threads call it.
+template <int M, int HT>
+__device__ __forceinline__ void put_sums(float2 *out, int g, int r, const Bins<PassGeo<M, HT>::E> &acc, float4 *red)
+{
+    using Geo = PassGeo<M, HT>;
+    if constexpr (Geo::G == 1) {
+        if constexpr (Geo::E == 1) gst(out + r, make_float2(acc.re[0], acc.im[0]));
+        else gst(reinterpret_cast<float4 *>(out) + r, make_float4(acc.re[0], acc.im[0], acc.re[1], acc.im[1]));
+    } else {
+        static_assert(Geo::S == M && Geo::G * M * sizeof(float2) <= tail_red_float4<M>() * sizeof(float4),
+                      "pass reduction buffer");
+        float2 *sums = reinterpret_cast<float2 *>(red);
 #pragma unroll
-    for (int k = 0; k < KH; k++)
+        for (int e = 0; e < Geo::E; e++) sums[g * M + Geo::E * r + e] = make_float2(acc.re[e], acc.im[e]);
+        __syncthreads();
+        for (int k = threadIdx.x; k < M; k += kTickThreads) {
+            float2 sum = sums[k];
 #pragma unroll
-        for (int v = 0; v < V; v++) {
-            if (wantA[k]) reinterpret_cast<float4 *>(a.kTA[OFF + k])[orow + v * R + r] = accA[k][v];
-            if (NF == 2 && wantB[k]) reinterpret_cast<float4 *>(a.kTB[OFF + k])[orow + v * R + r] = accB[k][v];
+            for (int gg = 1; gg < Geo::G; gg++) sum = cadd(sum, sums[gg * M + k]);
+            gst(out + k, sum);
         }
+        __syncthreads();
+    }
 }
 
 // Multi-block pass (kn >= 1 outputs): partitions [2 + j*pc, 2 + (j+1)*pc)
 // of channel c for kn consecutive blocks.  Output k (0-based, block
 // o + g + k, o the launch's first head block, g = kgap) takes partition
-// i >= g + k + 1 with FDL row (tbase + k - i), the row partition i - k reads
-// for output 0: each lane group walks its partitions in order and keeps the
-// last kPassMax rows it loaded, so every IR row and FDL row is read once and
-// used for every output.
+// i >= g + k + 1 with FDL row (tbase + k - i): the rows before the launch's
+// heads, rel = k - i < -g.  Partitions up to g meet no such row, and for the
+// later ones the window holds zeros in place of the newer rows.
 template <int M, int NF, int HT, bool NT = true, int KM = kPassMax>
 __device__ void tailk_role(const TickArgs &a, int c, int j, float4 *red)
 {
-    constexpr int H = M / 2;                     // float4 per row
-    constexpr int V = H > 256 ? H / 256 : 1;     // float4 per lane per row
-    constexpr int R = H / V;                     // lanes per row
-    constexpr int G = kTickThreads / R;          // lane groups
-    constexpr int U = 4;                         // partitions loaded together (8 measured slower)
-    static_assert(KM >= 1 && KM <= kPassMax, "pass length");
-    constexpr size_t kRowBytes = (size_t)M * IrRow<HT>::kBytes;
-    const int tid = threadIdx.x;
-    const int g = tid / R, r = tid % R;
-    if constexpr (KM == kPassMax && G == 2 && R % 64 == 0) {
-        // 16 outputs: each lane group takes 8 of them over every partition
-        // (8 window rows and 8 accumulators per lane instead of 16, and no
-        // reduction between the groups); the second group's FDL rows are the
-        // first group's of 8 partitions before, its IR rows the same ones
-        // (ordinary loads: a row must stay in the caches for the other group)
-        if (__builtin_amdgcn_readfirstlane(g) == 0) tailk_half<M, NF, HT, false, kPassMax / 2, 0>(a, c, j);
-        else tailk_half<M, NF, HT, false, kPassMax / 2, kPassMax / 2>(a, c, j);
-        return;
-    }
-    const float4 *F = reinterpret_cast<const float4 *>(a.fdl) + (size_t)c * a.P * H;
-    const char *HA = reinterpret_cast<const char *>(a.tHa) + (size_t)c * a.P * kRowBytes;
-    const char *HB = NF == 2 ? reinterpret_cast<const char *>(a.tHb) + (size_t)c * a.P * kRowBytes : nullptr;
+    using Geo = PassGeo<M, HT>;
+    const int g = threadIdx.x / Geo::R, r = threadIdx.x % Geo::R;
     const float *SA = HT == IR_F32 ? nullptr : a.tSa + (size_t)c * a.P;
     const float *SB = (HT == IR_F32 || NF == 1) ? nullptr : a.tSb + (size_t)c * a.P;
-    const int mask = a.P - 1, base = a.tbase, kn = a.kn, gap = a.kgap;
     const int i0 = 2 + j * a.pc, i1 = min(a.P, i0 + a.pc);
-    const int span = (i1 - i0 + G - 1) / G;
-    const int p0 = min(i1, i0 + g * span), p1 = min(i1, p0 + span);
-    bool wantA[KM], wantB[KM];
-#pragma unroll
-    for (int k = 0; k < KM; k++) {
-        wantA[k] = k < kn && a.kTA[k] != nullptr;
-        wantB[k] = NF == 2 && k < kn && a.kTB[k] != nullptr;
-    }
-    const bool dc0 = (r == 0);
-    const float s0 = dc0 ? 0.f : 1.f;
-    auto frow = [&](int row, int v) { return ld_row<NT>(F + (size_t)(row & mask) * H + v * R + r); };
-    auto hrow2 = [&](const char *row, int q) { return NT ? IrRow<HT>::get2(row, q) : IrRow<HT>::getc(row, q); };
-
-    float4 accA[KM][V], accB[KM][V], xw[KM][V];
-#pragma unroll
-    for (int k = 0; k < KM; k++)
-#pragma unroll
-        for (int v = 0; v < V; v++) {
-            accA[k][v] = make_float4(0.f, 0.f, 0.f, 0.f);
-            accB[k][v] = make_float4(0.f, 0.f, 0.f, 0.f);
-            // the window as it stands before partition p0: xw[k] = row (base + k + 1 - p0)
-            // (output k + 1 reads it at p0), loaded only where some output uses it
-            xw[k][v] = (k + 1 < KM && p0 < p1 && p0 >= k + 2 + gap) ? frow(base + k + 1 - p0, v)
-                                                                     : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    for (int i = p0; i < p1; i += U) {
-        float4 xn[U][V], ha[U][V], hb[U][V];
-        float sa[U], sb[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int ii = i + u;
-            sa[u] = 1.f;
-            sb[u] = 1.f;
-            if (ii < p1) {
-                sa[u] = row_scale<HT>(SA, ii);
-                if (NF == 2) sb[u] = row_scale<HT>(SB, ii);
-            }
-#pragma unroll
-            for (int v = 0; v < V; v++) {
-                if (ii < p1) {
-                    xn[u][v] = frow(base - ii, v);
-                    ha[u][v] = hrow2(HA + (size_t)ii * kRowBytes, v * R + r);
-                    if (NF == 2) hb[u][v] = hrow2(HB + (size_t)ii * kRowBytes, v * R + r);
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int ii = i + u;
-            if (ii >= p1) break;
-#pragma unroll
-            for (int v = 0; v < V; v++) {
-#pragma unroll
-                for (int k = KM - 1; k > 0; k--) xw[k][v] = xw[k - 1][v];
-                xw[0][v] = xn[u][v];
-                const bool dc = dc0 && v == 0;
-                const float sv = v == 0 ? s0 : 1.f;
-                const float4 hA = HT == IR_F32 ? ha[u][v] : scale4(ha[u][v], sa[u]);
-                float4 hB = hA;
-                if (NF == 2) hB = HT == IR_F32 ? hb[u][v] : scale4(hb[u][v], sb[u]);
-#pragma unroll
-                for (int k = 0; k < KM; k++) {
-                    if (ii >= k + 1 + gap) {
-                        if (wantA[k]) mac4(accA[k][v], xw[k][v], hA, sv, dc);
-                        if (NF == 2 && wantB[k]) mac4(accB[k][v], xw[k][v], hB, sv, dc);
-                    }
-                }
-            }
-        }
-    }
-    // the lane groups' sums reduced through red one output at a time:
-    // [NF][G][H] float4 per round
-    const size_t orow = ((size_t)c * a.nchunk + j) * H;
-    if constexpr (G == 1) {
-#pragma unroll
-        for (int k = 0; k < KM; k++)
-#pragma unroll
-            for (int v = 0; v < V; v++) {
-                if (wantA[k]) reinterpret_cast<float4 *>(a.kTA[k])[orow + v * R + r] = accA[k][v];
-                if (NF == 2 && wantB[k]) reinterpret_cast<float4 *>(a.kTB[k])[orow + v * R + r] = accB[k][v];
-            }
-    } else {
-        static_assert(NF * G * H <= tail_red_float4<M>(), "pass reduction buffer");
-        // unrolled over the outputs so that every pointer is picked
-        // statically (an output pointer indexed at run time would put the
-        // whole argument struct in private memory); the skip is uniform
+    const int span = (i1 - i0 + Geo::G - 1) / Geo::G;
+    const int q0 = min(i1, i0 + g * span), p1 = min(i1, q0 + span), p0 = max(q0, a.kgap + 1);
+    // outputs of each filter: the first ones are A's, the last ones B's
+    int kA = 0, kB = KM;
+    if constexpr (NF == 2) {
 #pragma unroll
         for (int k = 0; k < KM; k++) {
-            if (!wantA[k] && !(NF == 2 && wantB[k])) continue;
+            if (a.kTA[k]) kA = k + 1;
+            if (a.kTB[k]) kB = min(kB, k);
+        }
+    }
+    for (int s0 = 0; s0 < M; s0 += Geo::S) {
+        const size_t at = (size_t)c * a.P * M + s0;
+        const SweepRows rows = {a.fdl + at, nullptr, a.tbase, a.P - 1, -a.kgap};
+        const char *HA = reinterpret_cast<const char *>(a.tHa) + at * IrRow<HT>::kBytes;
+        const char *HB = NF == 2 ? reinterpret_cast<const char *>(a.tHb) + at * IrRow<HT>::kBytes : nullptr;
+        Bins<Geo::E> accA[KM], accB[KM];
+        pass_sweep<M, NF, HT, NT, KM>(rows, HA, HB, SA, SB, p0, p1, r, s0 == 0 && r == 0, kA, kB, accA, accB,
+                                         reinterpret_cast<float2 *>(red));
+        if constexpr (Geo::G > 1) __syncthreads();  // red: folds before, the groups' sums after
+        // unrolled over the outputs so that every pointer is picked statically
+        // (an output pointer indexed at run time would put the whole argument
+        // struct in private memory); the skip is uniform
+        const size_t orow = ((size_t)c * a.nchunk + j) * M + s0;
 #pragma unroll
-            for (int v = 0; v < V; v++) {
-                red[(0 * G + g) * H + v * R + r] = accA[k][v];
-                if (NF == 2) red[(1 * G + g) * H + v * R + r] = accB[k][v];
-            }
-            __syncthreads();
-            // one loop per filter: a pointer chosen between the two at run
-            // time would also put the argument copy in private memory
-            auto reduce_to = [&](int f, float2 *out) {
-                for (int q = tid; q < H; q += kTickThreads) {
-                    float4 sum = red[(f * G + 0) * H + q];
-#pragma unroll
-                    for (int gg = 1; gg < G; gg++) {
-                        const float4 t = red[(f * G + gg) * H + q];
-                        sum.x += t.x; sum.y += t.y; sum.z += t.z; sum.w += t.w;
-                    }
-                    reinterpret_cast<float4 *>(out)[orow + q] = sum;
-                }
-            };
-            if (wantA[k]) reduce_to(0, a.kTA[k]);
-            if (NF == 2 && wantB[k]) reduce_to(1, a.kTB[k]);
-            __syncthreads();
+        for (int k = 0; k < KM; k++) {
+            if (a.kTA[k]) put_sums<M, HT>(a.kTA[k] + orow, g, r, accA[k], red);
+            if (NF == 2 && a.kTB[k]) put_sums<M, HT>(a.kTB[k] + orow, g, r, accB[k], red);
         }
     }
 }
@@ -1039,8 +1115,7 @@ __device__ __forceinline__ void frame_mac_block(const TickArgs &a, int t, float4
 template <int M, int NF, int HT, int TK, int KM = kPassMax>
 __global__ __launch_bounds__(kTickThreads) void k_tick(TickArgs a)
 {
-    // tail or pass reduction buffer (float4): [NF][G][H]
-    constexpr int kTailRed = tail_red_float4<M>();
+    constexpr int kTailRed = TK == 2 ? pass_red_float4<M, NF, HT, KM>() : tail_red_float4<M>();
     constexpr int kHeadBytes = sizeof(HeadSmem<M>);
     constexpr int kBytes = kHeadBytes > kTailRed * 16 ? kHeadBytes : kTailRed * 16;
     __shared__ float4 smem[(kBytes + 15) / 16];
@@ -1056,6 +1131,14 @@ __global__ __launch_bounds__(kTickThreads) void k_tick(TickArgs a)
     } else {
         frame_mac_block<M, HT>(a, b - a.nhead - a.C * a.nchunk, smem);
     }
+}
+
+// float4 of LDS the tail roles of a role set use
+template <int M, int HT, int ROLES, int KM>
+constexpr int roles_red_float4()
+{
+    return ROLES == kRolesLean ? pass_red_float4<M, 1, HT, KM>()
+           : ROLES == kRolesXfade ? pass_red_float4<M, 2, HT, KM>() : tail_red_float4<M>();
 }
 
 // Roles of one tick for block index b of one object's launch.  Role sets of
@@ -1110,8 +1193,7 @@ template <int HT, int M, int ROLES, int KM>
 __global__ __launch_bounds__(kTickThreads) void k_group_tick(const TickArgs *__restrict__ descs,
                                                              const int *__restrict__ starts, int nobj)
 {
-    // tail or pass reduction buffer (float4): [NF][G][H]
-    constexpr int kTailRed = tail_red_float4<M>();
+    constexpr int kTailRed = roles_red_float4<M, HT, ROLES, KM>();
     constexpr int kHeadBytes = sizeof(HeadSmem<M>);
     constexpr int kBytes = kHeadBytes > kTailRed * 16 ? kHeadBytes : kTailRed * 16;
     __shared__ float4 smem[(kBytes + 15) / 16];
@@ -1163,7 +1245,7 @@ __global__ __launch_bounds__(kTickThreads) void k_group_queue(const TickArgs *__
                                                               const int *__restrict__ starts, int nobj, int total,
                                                               int *__restrict__ next)
 {
-    constexpr int kTailRed = tail_red_float4<M>();
+    constexpr int kTailRed = roles_red_float4<M, HT, ROLES, KM>();
     constexpr int kHeadBytes = (ROLES == kRolesHeads ? wave_heads(M) : 1) * (int)sizeof(HeadSmem<M>);
     constexpr int kBytes = kHeadBytes > kTailRed * 16 ? kHeadBytes : kTailRed * 16;
     __shared__ float4 smem[(kBytes + 15) / 16];
@@ -1367,7 +1449,7 @@ __global__ __launch_bounds__(kTickThreads) void k_heads(HeadBatchArgs h)
 template <int M, int NF, int HT, int KM>
 __global__ __launch_bounds__(kTickThreads) void k_window(HeadBatchArgs h, TickArgs a)
 {
-    constexpr int kTailRed = tail_red_float4<M>();  // float4
+    constexpr int kTailRed = pass_red_float4<M, NF, HT, KM>();
     constexpr int kBytes = sizeof(HeadsSmem<M>) > kTailRed * 16 ? sizeof(HeadsSmem<M>) : kTailRed * 16;
     __shared__ float4 smem[(kBytes + 15) / 16];
     const int b = blockIdx.x;
