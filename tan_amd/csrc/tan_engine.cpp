@@ -382,6 +382,9 @@ struct tanx_conv {
     // frame rows), counted in the context's pass_rows while the object lives
     uint64_t rows_bytes = 0;
     long long covered = 0;
+    // the sums of blocks ticks .. covered are scheduled (porg) but not
+    // computed: process_call leaves them to the next block that needs them
+    bool deferred = false;
     long long porg[2 * kPassMax][2] = {};
     int pchunk[2 * kPassMax][2] = {};
     bool fused = true;    // device path: head and next tail in one launch
@@ -1301,6 +1304,8 @@ static void nu_block_args(tanx_conv *cv, uint64_t b_obj, bool xfade, TickArgs &a
     }
 }
 
+static int32_t ensure_sums(tanx_conv *cv);
+
 static int32_t prepare_block(tanx_conv *cv, const float *din, long long in_stride, float *dout,
                              long long out_stride, size_t n, const uint32_t *flags, bool with_tail,
                              TickArgs &a, int *tail_nf, bool *xfade_out,
@@ -1311,6 +1316,7 @@ static int32_t prepare_block(tanx_conv *cv, const float *din, long long in_strid
     if (rc != TANX_OK) return rc;
     if (nrun == 0) return TANX_WRONG_STATE;
     rc = sync_run_mask(cv);
+    if (rc == TANX_OK) rc = ensure_sums(cv);
     if (rc != TANX_OK) return rc;
 
     const uint64_t b = cv->ticks;
@@ -1528,6 +1534,159 @@ static int32_t process_block_kp(tanx_conv *cv, const float *din, long long in_st
     return TANX_OK;
 }
 
+// Blocks one CallArgs launch of this object may take: its spectra and partial
+// sums are kept where the passes keep theirs (4 kp maxchunk rows per
+// channel), of which n + (n + 1) * chunks rows per channel are used.
+static int call_blocks_max(const tanx_conv *cv) { return std::min(kPassMax, (4 * cv->kp * cv->maxchunk - 1) / 2); }
+
+// Least blocks of a device call that take process_call's three launches.  Few
+// blocks of a small object are two launches of batched heads (5 blocks of 3
+// channels x 4,096 taps: 13.4 us, 14.9 us in three launches; 6 blocks: 16.6
+// against 15.2 us), but a pass over many rows costs more than a launch (5 blocks of 64
+// channels x 65,536 taps: 30.6 against 25.4 us), and heads above
+// kHeadBatchMaxB are a launch each (4 blocks of 64 channels x 16,384 taps at
+// B = 1024: 47.2 against 26.5 us).
+static size_t call_blocks_min(const tanx_conv *cv)
+{
+    const size_t rows = (size_t)cv->C * cv->P * cv->B * (sizeof(float2) + ir_elem_bytes(cv->irtype));
+    return rows > (size_t(8) << 20) || cv->B > kHeadBatchMaxB ? 4 : 6;
+}
+
+// The pass schedule of a call taken by process_call goes on as if its blocks
+// had run through process_block_kp (which blocks share a launch, and the
+// origin of the sums a launch leaves), so that the sums of later single
+// blocks are split between pass and head alike whatever calls came before:
+// the pass of the launch with the last *queued heads.
+static void schedule_queued(tanx_conv *cv, int *queued)
+{
+    TickArgs unused{};
+    if (*queued > 0) fill_pass(cv, (long long)cv->ticks - *queued, (long long)cv->ticks, unused);
+    *queued = 0;
+}
+
+// The next n blocks of a device call of a uniform object with multi-block
+// passes, in three launches (CallArgs).  A call ends before a second
+// crossfade; *advanced is the number of blocks taken.
+static int32_t process_call(tanx_conv *cv, const float *din, long long in_stride, float *dout, long long out_stride,
+                            int n, int *advanced, int *queued)
+{
+    const size_t B = cv->B;
+    *advanced = 0;
+    CallArgs a{};
+    a.C = cv->C;
+    a.P = cv->P;
+    a.irtype = cv->irtype;
+    a.run = cv->drun;
+    const int lB = __builtin_ctz((unsigned)cv->B);
+    a.twM = tw_table(cv->ctx->tw, lB);
+    a.twN = tw_table(cv->ctx->tw, lB + 1);
+    a.fdl = cv->F;
+    a.slot = cv->pos;
+    a.xin = din;
+    a.in_stride = in_stride;
+    a.yout = dout;
+    a.out_stride = out_stride;
+    a.xprev = cv->xprev;
+    // rows the caches hold: a chunk's window is filled from rows its neighbour
+    // reads too (16 blocks of 64 channels x 65,536 taps: 29 against 35 us);
+    // larger objects stream (1,024 channels: 268 against 287 us)
+    a.cached = (size_t)cv->C * cv->P * B * (sizeof(float2) + ir_elem_bytes(cv->irtype)) <= kCachedRowsMax;
+    int xb = -1, done = 0, slot_a = cv->cur;
+    for (; done < n; done++) {
+        const bool xf_next = cv->delayed && cv->ticks == cv->switch_at;
+        if (xb >= 0 && xf_next) break;
+        if ((long long)cv->ticks > cv->covered || xf_next || *queued == kHeadBatch) schedule_queued(cv, queued);
+        int nrun = 0;
+        int32_t rc = channel_flags(cv, nullptr, B, &nrun);
+        if (rc == TANX_OK && done == 0) rc = sync_run_mask(cv);
+        if (rc != TANX_OK) return rc;
+        const bool xfade = advance_switch(cv, cv->ticks);
+        if (xfade) {
+            xb = done;
+            slot_a = cv->prev;
+            cv->delayed = false;
+            cv->xfades++;
+        }
+        cv->pos = (cv->pos + 1) % cv->P;
+        cv->crossfading = xfade;
+        cv->last_xfade = xfade;
+        cv->ticks++;
+        cv->tail_due = true;
+        tail_done(cv);
+        (*queued)++;
+        const bool armed = cv->delayed && cv->switch_at == cv->ticks;
+        if (xfade || armed || cv->B > kHeadBatchMaxB) schedule_queued(cv, queued);
+    }
+    cv->deferred = true;
+    *advanced = done;
+    a.n = done;
+    a.xb = xb >= 0 ? xb : done;
+    a.HA = cv->slot_ptr(slot_a);
+    a.SA = cv->scale_ptr(slot_a);
+    const int outs = done + (xb >= 0 ? 1 : 0);
+    if (xb >= 0) {
+        a.HB = cv->slot_ptr(cv->cur);
+        a.SB = cv->scale_ptr(cv->cur);
+    }
+    // partition chunks: one or two workgroups per compute unit (each output
+    // row of a chunk is written and read back, so calls of many blocks take
+    // fewer: 16 blocks of 64 channels 30, 35 and 42 us with 256, 512 and 1,024
+    // workgroups; 8 blocks with a crossfade 54, 52 and 55 us), of at least 16
+    // partitions, as many as the rows hold
+    const int rows = 4 * cv->kp * cv->maxchunk, groups = done > 8 ? 256 : 512;
+    int chunks = std::max(1, std::min((groups + cv->C - 1) / cv->C, cv->P / 16));
+    chunks = std::max(1, std::min(chunks, (rows - done) / outs));
+    a.pc = (cv->P + chunks - 1) / chunks;
+    a.nchunk = (cv->P + a.pc - 1) / a.pc;
+    a.X = cv->T;
+    a.T = cv->T + (size_t)cv->C * done * B;
+    hipStream_t s = cv->ctx->proc;
+    if (cv->timing) {
+        hipEvent_t e0 = nullptr, e1 = nullptr;
+        TANX_CHECK(cv->t_tail.acquire(&e0, &e1));
+        TANX_CHECK(launch_call(cv->B, a, s, e0, e1));
+        cv->t_tail.commit();
+        cv->tail_alg_bytes += tail_bytes(cv, xb >= 0 ? 2 : 1) + (uint64_t)outs * head_bytes(cv, 1);
+        cv->timed_blocks += (uint64_t)done;
+        return TANX_OK;
+    }
+    TANX_CHECK(launch_call(cv->B, a, s));
+    return TANX_OK;
+}
+
+// Computes the sums process_call left: of the blocks ticks .. covered with
+// the filters they use now (the switch state that of their scheduling), from
+// the rows before their origin.  Blocks of one filter share their origin.
+static int32_t ensure_sums(tanx_conv *cv)
+{
+    if (!cv->deferred) return TANX_OK;
+    cv->deferred = false;
+    const long long e = (long long)cv->ticks, c = cv->covered;
+    const long long sw = cv->delayed && (long long)cv->switch_at >= e && (long long)cv->switch_at <= c
+                             ? (long long)cv->switch_at : c + 1;
+    // filter 0: the current one, blocks e .. sw; filter 1: the armed one, blocks sw .. c
+    for (int f = 0; f < 2; f++) {
+        const long long from = f == 0 ? e : sw, to = f == 0 ? std::min(sw, c) : c;
+        if (from > to) continue;
+        TickArgs a = tick_common(cv);
+        a.nchunk = cv->nchunk;
+        a.pc = cv->pc;
+        a.kn = (int)(c - e) + 1;
+        a.tbase = cv->pos;  // ring slot of block e
+        a.tHa = cv->slot_ptr(f == 0 ? cv->cur : cv->upd);
+        a.tSa = cv->scale_ptr(f == 0 ? cv->cur : cv->upd);
+        for (long long b = from; b <= to; b++) {
+            const int part = f == 1 && b == sw ? 1 : 0;  // the crossfade block's second sums
+            a.kgap = (int)(e - cv->porg[cv->pring(b)][part]);
+            a.kTA[b - e] = cv->tail_slot(b, part);
+            cv->pchunk[cv->pring(b)][part] = cv->nchunk;
+        }
+        const int32_t rc = launch_timed(cv, cv->t_tail, 1, a, tail_bytes(cv, 1), cv->tail_alg_bytes);
+        if (rc != TANX_OK) return rc;
+    }
+    return TANX_OK;
+}
+
 // One block launched directly; with_tail also runs the next block's tail in
 // the same launch.
 static int32_t process_block(tanx_conv *cv, const float *din, long long in_stride, float *dout,
@@ -1685,7 +1844,23 @@ extern "C" int32_t tanx_conv_process_device(tanx_conv *cv, const float *d_in, si
         return process_device_graph(cv, d_in, in_stride, d_out, out_stride, nb, processed);
     HeadQueue hq;
     const bool fuse = cv->fused && !cv->fmode;
-    for (size_t b = 0; b < nb; b++) {
+    size_t b = 0;
+    const size_t most = (size_t)std::max(1, call_blocks_max(cv));
+    if (fuse && cv->kp > 1 && !flags && std::min(nb, most) >= call_blocks_min(cv)) {
+        // windows of equal length
+        const size_t windows = (nb + most - 1) / most, want = (nb + windows - 1) / windows;
+        int queued = 0;
+        while (b < nb) {
+            int took = 0;
+            const int32_t rc = process_call(cv, d_in + b * B, (long long)in_stride, d_out + b * B,
+                                            (long long)out_stride, (int)std::min(nb - b, want), &took, &queued);
+            if (rc != TANX_OK) return rc;
+            b += (size_t)took;
+            if (processed) *processed = b * B;
+        }
+        schedule_queued(cv, &queued);
+    }
+    for (; b < nb; b++) {
         int32_t rc = (fuse && cv->kp > 1)
                          ? process_block_kp(cv, d_in + b * B, (long long)in_stride, d_out + b * B,
                                             (long long)out_stride, B, flags, hq)

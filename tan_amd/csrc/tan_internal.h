@@ -299,6 +299,34 @@ hipError_t launch_heads(int B, int irtype, const HeadBatchArgs &h, hipStream_t s
                         hipEvent_t ev1 = nullptr);
 hipError_t launch_window(int B, int tail_nf, const HeadBatchArgs &h, const TickArgs &a, hipStream_t s,
                          hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// A call's blocks w .. w+n-1 of a uniform object (n <= kPassMax) in three
+// launches, all known at once: the blocks' spectra (k_call_spectra, into X),
+// one sweep over every partition for the n outputs (k_call_pass: partition i
+// of block w+k meets X row k - i, or FDL row w + k - i before the call) and
+// the inverse transforms (k_call_out), which also move X into the FDL ring
+// and keep the last input block.  One block of the call may crossfade.
+struct CallArgs {
+    int C, P, n;
+    int irtype;
+    const uint8_t *run;
+    const float2 *twM, *twN;
+    float2 *fdl;
+    int slot;              // ring slot of block w
+    const float *xin;      // block w + k of channel c at xin + c * in_stride + k * B
+    long long in_stride;
+    float *yout;
+    long long out_stride;
+    float *xprev;
+    float2 *X;             // [C][n][B] spectra of the call's blocks
+    float2 *T;             // partial sums [C][outputs][nchunk][B]: filter A's output k is row k,
+                           // filter B's row k + 1 (blocks xb .. n-1)
+    const void *HA, *HB;   // the blocks before the crossfade and itself; it and the blocks after (or nullptr)
+    const float *SA, *SB;
+    int xb;                // block (of the n) that crossfades, n without one
+    int nchunk, pc;        // partition chunks per channel and partitions per chunk
+    int cached;            // nonzero: the sweep reads the rows with ordinary loads
+};
+hipError_t launch_call(int B, const CallArgs &a, hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 // k_tick reading its arguments from d_descs[k] (graph replay; kn must be 1)
 hipError_t launch_tick_desc(int B, int irtype, const TickArgs *d_descs, int k, unsigned blocks, hipStream_t s);
 hipError_t launch_ir_transform(int B, int nchan, const IrArgs &a, hipStream_t s);

@@ -245,12 +245,13 @@ constexpr int kHeadPreload = 4;      // near partitions a head loads together
 // [filter (<= 2)][lane group G][row float4 H] per round, G * H = 256 * V
 template <int M>
 constexpr int tail_red_float4() { return 2 * kTickThreads * ((M / 2 > 256) ? (M / 2) / 256 : 1); }
-// the same for a pass of KM outputs and NF filters, which also folds its sums there
+// the same for a pass of KM outputs and NF filters, which also keeps its
+// first segments' sums there (sweep_outputs)
 template <int M, int NF, int HT, int KM>
 constexpr int pass_red_float4()
 {
-    const int folds = HT == IR_F32 ? (KM + NF - 1) * kTickThreads / 2 : 0;
-    return folds > tail_red_float4<M>() ? folds : tail_red_float4<M>();
+    const int both = HT == IR_F32 && M <= kTickThreads ? (KM + NF) * kTickThreads / 2 : 0;
+    return both > tail_red_float4<M>() ? both : tail_red_float4<M>();
 }
 
 // Streamed rows (IR spectra, FDL) are read once per block: nontemporal loads
@@ -753,14 +754,13 @@ struct Bins {
     float re[E], im[E];
 };
 
-constexpr int kFold = 64;  // partitions an FP32 sum runs over before it is folded into LDS
-
 template <int M, int HT>
 struct PassGeo {
     static constexpr int E = HT == IR_F32 ? 1 : 2;                      // bins per lane
     static constexpr int S = M < E * kTickThreads ? M : E * kTickThreads;  // bins per slice
     static constexpr int R = S / E;                                     // lanes per slice
     static constexpr int G = kTickThreads / R;                          // lane groups
+    static constexpr int SEG = E == 1 && M <= kTickThreads ? 2 : 1;     // segments of a group's partitions
 };
 
 // Bins of lane r of a row's slice (NT: nontemporal)
@@ -851,22 +851,18 @@ struct SweepRows {
 };
 
 // dc: the lane's first bin is the packed (DC, Nyquist) element.
-// A sum of FP32 rows is folded into LDS every kFold partitions (fold: one
-// float2 per output and thread), which keeps its rounding error below that of
-// one chain over the chunk: 64 terms and the chunk's folds.
 // NF filters: HA for outputs k < kA, HB (NF = 2) for outputs k >= kB; with
 // one filter every output is computed (the caller stores those it wants).
 template <int M, int NF, int HT, bool NT, int KM>
 __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA, const char *HB, const float *SA,
                                            const float *SB, int p0, int p1, int r, bool dc, int kA, int kB,
-                                           Bins<PassGeo<M, HT>::E> (&accA)[KM], Bins<PassGeo<M, HT>::E> (&accB)[KM],
-                                           float2 *fold)
+                                           Bins<PassGeo<M, HT>::E> (&accA)[KM], Bins<PassGeo<M, HT>::E> (&accB)[KM])
 {
     constexpr int E = PassGeo<M, HT>::E;
     constexpr int U = 4;                                                // partitions per stage
     constexpr int kBody = NF == 2 ? U : KM < 8 ? 8 : KM;  // partitions per loop trip
     constexpr size_t kRowBytes = (size_t)M * IrRow<HT>::kBytes;
-    static_assert(kBody % U == 0 && kFold >= kBody && KM <= kPassMax, "pass length");
+    static_assert(kBody % U == 0 && KM <= kPassMax, "pass length");
     // entry KM - 1 + q of the window holds the row of partition i + q (row
     // -(i + q)) for the trip starting at partition i; output k reads the
     // entry k before it
@@ -903,33 +899,8 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
             }
         }
     };
-    // output k's fold slot (the filters' outputs together are at most KM + 1)
-    auto slot = [&](int f, int k) { return fold + (k + f) * kTickThreads + threadIdx.x; };
-    // adds the sums into their slots (the first time: stores them), clearing
-    // them, or at the end the slots into the sums
-    auto fold_sums = [&](bool first, bool last) {
-        if constexpr (E == 1) {
-#pragma unroll
-            for (int f = 0; f < NF; f++)
-#pragma unroll
-                for (int k = 0; k < KM; k++) {
-                    if (NF == 2 && !(f == 0 ? k < kA : k >= kB)) continue;
-                    Bins<E> &s = f == 0 ? accA[k] : accB[k];
-                    float2 t = make_float2(s.re[0], s.im[0]);
-                    if (!first) t = cadd(*slot(f, k), t);
-                    if (!last) *slot(f, k) = t;
-                    s.re[0] = last ? t.x : 0.f;
-                    s.im[0] = last ? t.y : 0.f;
-                }
-        }
-    };
-    int next_fold = p0 + kFold;
     load(cur, p0);
     for (int i = p0; i < p1; i += kBody) {
-        if (E == 1 && i >= next_fold) {
-            fold_sums(next_fold == p0 + kFold, false);
-            next_fold += kFold;
-        }
 #pragma unroll
         for (int q0 = 0; q0 < kBody; q0 += U) {
             load(nxt, i + q0 + U);
@@ -971,34 +942,73 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
 #pragma unroll
         for (int k = 0; k < KM - 1; k++) win[k] = win[k + kBody];
     }
-    if (E == 1 && next_fold > p0 + kFold) fold_sums(false, true);
 }
 
-// One output row's slice of a sweep: the lane groups' sums, added in group
-// order through red ([G][S] complex), or the one group's directly.  All
-// threads call it.
-template <int M, int HT>
-__device__ __forceinline__ void put_sums(float2 *out, int g, int r, const Bins<PassGeo<M, HT>::E> &acc, float4 *red)
+// The outputs of partitions [i0, i1) (those from pmin on) of one channel's
+// slice: out(f, k) is filter f's output row k (at the slice) or nullptr; the
+// skip is uniform.  The range is cut into segs * G segments (segs <= SEG),
+// each summed as one chain; a lane group takes segs of them (its first one's
+// sums wait in LDS, one float2 per output and thread) and an output adds the
+// segments in order.  All threads call it.
+template <int M, int NF, int HT, bool NT, int KM, class Out>
+__device__ __forceinline__ void sweep_outputs(const SweepRows &rows, const char *HA, const char *HB, const float *SA,
+                                              const float *SB, int i0, int i1, int pmin, bool dc0, int kA, int kB,
+                                              int segs, float4 *red, Out out)
 {
     using Geo = PassGeo<M, HT>;
-    if constexpr (Geo::G == 1) {
-        if constexpr (Geo::E == 1) gst(out + r, make_float2(acc.re[0], acc.im[0]));
-        else gst(reinterpret_cast<float4 *>(out) + r, make_float4(acc.re[0], acc.im[0], acc.re[1], acc.im[1]));
-    } else {
-        static_assert(Geo::S == M && Geo::G * M * sizeof(float2) <= tail_red_float4<M>() * sizeof(float4),
-                      "pass reduction buffer");
-        float2 *sums = reinterpret_cast<float2 *>(red);
+    const int g = threadIdx.x / Geo::R, r = threadIdx.x % Geo::R;
+    const int ns = segs * Geo::G, span = (i1 - i0 + ns - 1) / ns;
+    const bool both = Geo::SEG == 2 && segs == 2;
+    float2 *sums = reinterpret_cast<float2 *>(red);                          // [G][S]
+    float2 *firsts = sums + kTickThreads;                                    // [outputs][threads]
+    // filter f's output k: the filters' outputs together are at most KM + 1
+    auto first = [&](int f, int k) { return firsts + (k + f) * kTickThreads; };
+    Bins<Geo::E> acc[2][KM];
+    for (int seg = 0; seg < segs; seg++) {
+        const int q0 = min(i1, i0 + (g * segs + seg) * span), p1 = min(i1, q0 + span);
+        pass_sweep<M, NF, HT, NT, KM>(rows, HA, HB, SA, SB, max(q0, pmin), p1, r, dc0 && r == 0, kA, kB, acc[0],
+                                      acc[1]);
+        if (both && seg == 0) {
 #pragma unroll
-        for (int e = 0; e < Geo::E; e++) sums[g * M + Geo::E * r + e] = make_float2(acc.re[e], acc.im[e]);
-        __syncthreads();
-        for (int k = threadIdx.x; k < M; k += kTickThreads) {
-            float2 sum = sums[k];
+            for (int f = 0; f < NF; f++)
 #pragma unroll
-            for (int gg = 1; gg < Geo::G; gg++) sum = cadd(sum, sums[gg * M + k]);
-            gst(out + k, sum);
+                for (int k = 0; k < KM; k++)
+                    if (NF == 1 || (f == 0 ? k < kA : k >= kB))
+                        first(f, k)[threadIdx.x] = make_float2(acc[f][k].re[0], acc[f][k].im[0]);
         }
-        __syncthreads();
     }
+    // unrolled over the outputs so that every pointer is picked statically
+    // (an output pointer indexed at run time would put the whole argument
+    // struct in private memory)
+#pragma unroll
+    for (int k = 0; k < KM; k++)
+#pragma unroll
+        for (int f = 0; f < NF; f++) {
+            float2 *o = out(f, k);
+            if (!o) continue;
+            const Bins<Geo::E> &a = acc[f][k];
+            if constexpr (Geo::G == 1) {
+                float2 v = make_float2(a.re[0], a.im[0]);
+                if (both) v = cadd(first(f, k)[threadIdx.x], v);
+                if constexpr (Geo::E == 1) gst(o + r, v);
+                else gst(reinterpret_cast<float4 *>(o) + r, make_float4(v.x, v.y, a.re[1], a.im[1]));
+            } else {
+                static_assert(Geo::S == M && Geo::G * M == kTickThreads * Geo::E, "pass reduction buffer");
+#pragma unroll
+                for (int e = 0; e < Geo::E; e++) sums[g * M + Geo::E * r + e] = make_float2(a.re[e], a.im[e]);
+                __syncthreads();
+                for (int b = threadIdx.x; b < M; b += kTickThreads) {
+                    float2 sum = both ? cadd(first(f, k)[b], sums[b]) : sums[b];
+#pragma unroll
+                    for (int gg = 1; gg < Geo::G; gg++) {
+                        if (both) sum = cadd(sum, first(f, k)[gg * Geo::R + b]);
+                        sum = cadd(sum, sums[gg * M + b]);
+                    }
+                    gst(o + b, sum);
+                }
+                __syncthreads();
+            }
+        }
 }
 
 // Multi-block pass (kn >= 1 outputs): partitions [2 + j*pc, 2 + (j+1)*pc)
@@ -1011,12 +1021,9 @@ template <int M, int NF, int HT, bool NT = true, int KM = kPassMax>
 __device__ void tailk_role(const TickArgs &a, int c, int j, float4 *red)
 {
     using Geo = PassGeo<M, HT>;
-    const int g = threadIdx.x / Geo::R, r = threadIdx.x % Geo::R;
     const float *SA = HT == IR_F32 ? nullptr : a.tSa + (size_t)c * a.P;
     const float *SB = (HT == IR_F32 || NF == 1) ? nullptr : a.tSb + (size_t)c * a.P;
     const int i0 = 2 + j * a.pc, i1 = min(a.P, i0 + a.pc);
-    const int span = (i1 - i0 + Geo::G - 1) / Geo::G;
-    const int q0 = min(i1, i0 + g * span), p1 = min(i1, q0 + span), p0 = max(q0, a.kgap + 1);
     // outputs of each filter: the first ones are A's, the last ones B's
     int kA = 0, kB = KM;
     if constexpr (NF == 2) {
@@ -1031,19 +1038,12 @@ __device__ void tailk_role(const TickArgs &a, int c, int j, float4 *red)
         const SweepRows rows = {a.fdl + at, nullptr, a.tbase, a.P - 1, -a.kgap};
         const char *HA = reinterpret_cast<const char *>(a.tHa) + at * IrRow<HT>::kBytes;
         const char *HB = NF == 2 ? reinterpret_cast<const char *>(a.tHb) + at * IrRow<HT>::kBytes : nullptr;
-        Bins<Geo::E> accA[KM], accB[KM];
-        pass_sweep<M, NF, HT, NT, KM>(rows, HA, HB, SA, SB, p0, p1, r, s0 == 0 && r == 0, kA, kB, accA, accB,
-                                         reinterpret_cast<float2 *>(red));
-        if constexpr (Geo::G > 1) __syncthreads();  // red: folds before, the groups' sums after
-        // unrolled over the outputs so that every pointer is picked statically
-        // (an output pointer indexed at run time would put the whole argument
-        // struct in private memory); the skip is uniform
         const size_t orow = ((size_t)c * a.nchunk + j) * M + s0;
-#pragma unroll
-        for (int k = 0; k < KM; k++) {
-            if (a.kTA[k]) put_sums<M, HT>(a.kTA[k] + orow, g, r, accA[k], red);
-            if (NF == 2 && a.kTB[k]) put_sums<M, HT>(a.kTB[k] + orow, g, r, accB[k], red);
-        }
+        sweep_outputs<M, NF, HT, NT, KM>(rows, HA, HB, SA, SB, i0, i1, a.kgap + 1, s0 == 0, kA, kB, Geo::SEG, red,
+                                         [&](int f, int k) {
+                                             float2 *o = f == 0 ? a.kTA[k] : a.kTB[k];
+                                             return o ? o + orow : nullptr;
+                                         });
     }
 }
 
@@ -1461,6 +1461,161 @@ __global__ __launch_bounds__(kTickThreads) void k_window(HeadBatchArgs h, TickAr
         if (!a.run[c]) return;
         if (a.cached) tailk_role<M, NF, HT, false, KM>(a, c, j, smem);
         else tailk_role<M, NF, HT, true, KM>(a, c, j, smem);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Several blocks of one call (CallArgs).  The heads of a call given a block
+// at a time are a chain: transform, multiply, inverse transform, block after
+// block.  With every input block at hand the transforms are independent
+// (one wave each up to B = 256, C * n of them), the sweep reads each IR and
+// FDL row once for all n outputs, and only three launches follow each other.
+// Calls of 16 blocks, 64 channels x 65,536 taps at B = 256: 29 us, 89 us a
+// launch per four blocks; 8 blocks of 1,024 channels x 131,072 taps with FP16
+// rows: 304 us (5.3 TB/s of rows), 577 us with two sweeps; 4 blocks of 1,024
+// channels x 65,536 taps: 188 us.
+// ---------------------------------------------------------------------------
+template <int M>
+__global__ __launch_bounds__(kTickThreads) void k_call_spectra(CallArgs a)
+{
+    constexpr int HPB = wave_heads(M), NT = HPB > 1 ? 64 : kTickThreads;
+    __shared__ float2 s0[HPB][M], s1[HPB][M], tw[M];
+    const int w = HPB > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+    const int tid = HPB > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+    const int item = blockIdx.x * HPB + w, c = item / a.n, j = item - c * a.n;
+    const bool active = c < a.C && a.run[c];
+    for (int m = threadIdx.x; m < M; m += kTickThreads) tw[m] = a.twM[m];
+    if (active) {
+        const float *cur = a.xin + (size_t)c * a.in_stride + (size_t)j * M;
+        const float *prev = j == 0 ? a.xprev + (size_t)c * M : cur - M;
+#pragma unroll
+        for (int m = tid; m < M; m += NT) {
+            const float *src = m < M / 2 ? prev + 2 * m : cur + 2 * (m - M / 2);
+            s0[w][m] = make_float2(src[0], src[1]);
+        }
+    }
+    __syncthreads();
+    if (!active) return;
+    const float2 *Z = fft_lds<M, false, NT>(s0[w], s1[w], tw);
+    float2 *row = a.X + (size_t)item * M;
+#pragma unroll
+    for (int k = tid; k < M; k += NT) row[k] = r2c_post<M>(Z, k, a.twN);
+}
+
+template <int M, int NF, int HT, bool NT, int KM>
+__global__ __launch_bounds__(kTickThreads) void k_call_pass(CallArgs a)
+{
+    using Geo = PassGeo<M, HT>;
+    __shared__ float4 red[pass_red_float4<M, NF, HT, KM>()];
+    const int c = blockIdx.x / a.nchunk, j = blockIdx.x - c * a.nchunk;
+    if (!a.run[c]) return;
+    const float *SA = HT == IR_F32 ? nullptr : a.SA + (size_t)c * a.P;
+    const float *SB = (HT == IR_F32 || NF == 1) ? nullptr : a.SB + (size_t)c * a.P;
+    const int i0 = j * a.pc, i1 = min(a.P, i0 + a.pc);
+    const int kA = NF == 2 ? a.xb + 1 : a.n, kB = NF == 2 ? a.xb : a.n;
+    // a second segment (shorter chains) costs the reads that fill its window,
+    // n - 1 rows: only for chunks that are long beside it
+    const int segs = i1 - i0 > 64 * Geo::G ? Geo::SEG : 1;
+    for (int s0 = 0; s0 < M; s0 += Geo::S) {
+        const size_t at = (size_t)c * a.P * M + s0;
+        const SweepRows rows = {a.fdl + at, a.X + (size_t)c * a.n * M + s0, a.slot, a.P - 1, a.n};
+        const char *HA = reinterpret_cast<const char *>(a.HA) + at * IrRow<HT>::kBytes;
+        const char *HB = NF == 2 ? reinterpret_cast<const char *>(a.HB) + at * IrRow<HT>::kBytes : nullptr;
+        // this chunk's row of filter f's output k
+        auto out = [&](int f, int k) -> float2 * {
+            if (!(f == 0 ? k < kA : k >= kB && k < a.n)) return nullptr;
+            return a.T + (((size_t)c * (a.n + NF - 1) + k + f) * a.nchunk + j) * M + s0;
+        };
+        sweep_outputs<M, NF, HT, NT, KM>(rows, HA, HB, SA, SB, i0, i1, 0, s0 == 0, kA, kB, segs, red, out);
+    }
+}
+
+template <int M>
+__global__ __launch_bounds__(kTickThreads) void k_call_out(CallArgs a)
+{
+    constexpr int HPB = wave_heads(M), NT = HPB > 1 ? 64 : kTickThreads;
+    constexpr int KPT = M / NT, ZP = (M / 2 + NT - 1) / NT;  // bins and output sample pairs per thread
+    constexpr int CB = 8;                                     // partial rows loaded together
+    constexpr float kScale = 1.0f / (2.0f * (float)M);
+    __shared__ float2 s0[HPB][M], s1[HPB][M], tw[M];
+    const int w = HPB > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+    const int tid = HPB > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+    const int item = blockIdx.x * HPB + w, c = item / a.n, k = item - c * a.n;
+    const bool active = c < a.C && a.run[c];
+    for (int m = threadIdx.x; m < M; m += kTickThreads) tw[m] = a.twM[m];
+    __syncthreads();
+    if (!active) return;
+    const bool two = k == a.xb;
+    const int outs = a.n + (a.xb < a.n ? 1 : 0);
+    float2 wn[KPT];
+#pragma unroll
+    for (int q = 0; q < KPT; q++) wn[q] = a.twN[tid + q * NT];
+    float2 y[ZP];
+    for (int f = 0; f < (two ? 2 : 1); f++) {
+        // the row of this block's filter: A's up to the crossfade, B's (one further) after it
+        const int o = two ? k + f : k + (k > a.xb ? 1 : 0);
+        const float2 *T = a.T + ((size_t)c * outs + o) * a.nchunk * M;
+        float2 s[KPT];
+#pragma unroll
+        for (int q = 0; q < KPT; q++) s[q] = make_float2(0.f, 0.f);
+        for (int j0 = 0; j0 < a.nchunk; j0 += CB) {
+            float2 t[CB][KPT];
+#pragma unroll
+            for (int u = 0; u < CB; u++)
+#pragma unroll
+                for (int q = 0; q < KPT; q++) t[u][q] = T[(size_t)min(j0 + u, a.nchunk - 1) * M + tid + q * NT];
+#pragma unroll
+            for (int u = 0; u < CB; u++)
+#pragma unroll
+                for (int q = 0; q < KPT; q++) {
+                    s[q].x += j0 + u < a.nchunk ? t[u][q].x : 0.f;
+                    s[q].y += j0 + u < a.nchunk ? t[u][q].y : 0.f;
+                }
+        }
+#pragma unroll
+        for (int q = 0; q < KPT; q++) s1[w][tid + q * NT] = s[q];
+        group_sync<NT>();
+#pragma unroll
+        for (int q = 0; q < KPT; q++) s0[w][tid + q * NT] = c2r_pre_w<M>(s1[w], tid + q * NT, wn[q]);
+        group_sync<NT>();
+        const float2 *z = fft_lds<M, true, NT>(s0[w], s1[w], tw);
+        const float step = (float)(1.0 / (double)M);
+#pragma unroll
+        for (int q = 0; q < ZP; q++) {
+            const int n = tid + q * NT;
+            if (n < M / 2) {
+                // second half of the 2M output samples
+                const float2 v = z[M / 2 + n];
+                const float y0 = v.x * kScale, y1 = v.y * kScale;
+                if (f == 0) {
+                    y[q] = make_float2(y0, y1);
+                } else {
+                    const int j0 = 2 * n, j1 = 2 * n + 1;
+                    y[q].x = fmaf(y0, step * (float)j0, y[q].x * (step * (float)(M - j0)));
+                    y[q].y = fmaf(y1, step * (float)j1, y[q].y * (step * (float)(M - j1)));
+                }
+            }
+        }
+        group_sync<NT>();
+    }
+    float *yo = a.yout + (size_t)c * a.out_stride + (size_t)k * M;
+#pragma unroll
+    for (int q = 0; q < ZP; q++) {
+        const int n = tid + q * NT;
+        if (n < M / 2) {
+            yo[2 * n] = y[q].x;
+            yo[2 * n + 1] = y[q].y;
+        }
+    }
+    // the block's spectrum enters the delay line, the last block's input is
+    // the next call's previous one
+    const float2 *row = a.X + (size_t)item * M;
+    float2 *to = a.fdl + ((size_t)c * a.P + ((a.slot + k) & (a.P - 1))) * M;
+#pragma unroll
+    for (int q = 0; q < KPT; q++) to[tid + q * NT] = row[tid + q * NT];
+    if (k == a.n - 1) {
+        const float *last = a.xin + (size_t)c * a.in_stride + (size_t)k * M;
+        for (int m = tid; m < M; m += NT) a.xprev[(size_t)c * M + m] = last[m];
     }
 }
 
@@ -2485,6 +2640,32 @@ hipError_t launch_window_t(int B, int tail_nf, const HeadBatchArgs &h, const Tic
     return hipGetLastError();
 }
 
+template <int HT, int M>
+static hipError_t launch_call_pass(const CallArgs &a, hipStream_t s)
+{
+    const dim3 g((unsigned)(a.C * a.nchunk)), t(kTickThreads);
+#define TANX_CALL_KM(KM)                                                                          \
+    case KM:                                                                                      \
+        if (a.HB) hipLaunchKernelGGL((k_call_pass<M, 2, HT, true, KM>), g, t, 0, s, a);           \
+        else if (a.cached) hipLaunchKernelGGL((k_call_pass<M, 1, HT, false, KM>), g, t, 0, s, a); \
+        else hipLaunchKernelGGL((k_call_pass<M, 1, HT, true, KM>), g, t, 0, s, a);                \
+        break;
+    switch (pass_km(a.n)) {
+        TANX_CALL_KM(4) TANX_CALL_KM(8) TANX_CALL_KM(12) TANX_CALL_KM(16)
+    default:
+        return hipErrorInvalidValue;
+    }
+#undef TANX_CALL_KM
+    return hipGetLastError();
+}
+
+template <int HT>
+hipError_t launch_call_pass_t(int B, const CallArgs &a, hipStream_t s)
+{
+    TANX_SWITCH_B(B, return (launch_call_pass<HT, M>(a, s)));
+    return hipErrorInvalidValue;
+}
+
 // partition sizes of uniform blocks (64..1024) and of frames (128..4096)
 #define TANX_SWITCH_PART(B, CALL)                        \
     switch (B) {                                         \
@@ -2583,6 +2764,7 @@ hipError_t launch_group_frame_t(const FrameArgs *d_descs, const int *d_starts, i
     PRE template hipError_t launch_heads_t<HT>(int, const HeadBatchArgs &, hipStream_t, hipEvent_t, hipEvent_t);    \
     PRE template hipError_t launch_window_t<HT>(int, int, const HeadBatchArgs &, const TickArgs &, hipStream_t,     \
                                                 hipEvent_t, hipEvent_t);                                            \
+    PRE template hipError_t launch_call_pass_t<HT>(int, const CallArgs &, hipStream_t);                             \
     PRE template hipError_t launch_ir_transform_group_t<HT>(int, const IrArgs *, const int *, int, unsigned,        \
                                                             hipStream_t);                                           \
     PRE template hipError_t launch_ir_transform_t<HT>(int, int, const IrArgs &, hipStream_t);                       \
@@ -2687,6 +2869,39 @@ hipError_t launch_heads(int B, int irtype, const HeadBatchArgs &h, hipStream_t s
     }
 }
 
+
+template <int M>
+static hipError_t launch_call_m(const CallArgs &a, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
+{
+    const dim3 g((unsigned)((a.C * a.n + wave_heads(M) - 1) / wave_heads(M))), t(kTickThreads);
+    hipExtLaunchKernelGGL((k_call_spectra<M>), g, t, 0, s, ev0, nullptr, 0, a);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) {
+        switch (a.irtype) {
+        case IR_F32: e = launch_call_pass_t<IR_F32>(M, a, s); break;
+        case IR_F16: e = launch_call_pass_t<IR_F16>(M, a, s); break;
+        case IR_BF16: e = launch_call_pass_t<IR_BF16>(M, a, s); break;
+        default: return hipErrorInvalidValue;
+        }
+    }
+    if (e != hipSuccess) return e;
+    hipExtLaunchKernelGGL((k_call_out<M>), g, t, 0, s, nullptr, ev1, 0, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_call(int B, const CallArgs &a, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
+{
+    if (a.n < 1 || a.n > kPassMax || a.n > a.P || a.nchunk < 1 || (a.HB == nullptr) != (a.xb >= a.n) || a.xb < 0)
+        return hipErrorInvalidValue;
+    switch (B) {
+    case 64: return launch_call_m<64>(a, s, ev0, ev1);
+    case 128: return launch_call_m<128>(a, s, ev0, ev1);
+    case 256: return launch_call_m<256>(a, s, ev0, ev1);
+    case 512: return launch_call_m<512>(a, s, ev0, ev1);
+    case 1024: return launch_call_m<1024>(a, s, ev0, ev1);
+    default: return hipErrorInvalidValue;
+    }
+}
 
 int ir_transform_blocks(int B, int irtype, int P, int nchan)
 {

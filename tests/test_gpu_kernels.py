@@ -63,3 +63,44 @@ def test_mix_sums_in_channel_order(gpu_ctx, n, channels):
         np.testing.assert_array_equal(out.cpu().numpy()[:n], ref)
         assert (out[n:] == 5.0).all()
     m.Terminate()
+
+
+# (taps, block, pass_blocks, max_tail_chunks, precision): as many blocks as
+# partitions, rows of several slices, one chunk, 16-bit rows
+@pytest.mark.parametrize("L,B,K,chunks,precision", [(16 * 64, 64, 4, 0, 0), (16 * 1024, 1024, 4, 0, 0),
+                                                    (300 * 128, 128, 8, 0, 0), (64 * 512, 512, 12, 1, 0),
+                                                    (80 * 256, 256, 16, 1, 0), (20 * 1024, 1024, 4, 2, 1),
+                                                    (20 * 128, 128, 4, 0, 2)])
+def test_calls_of_many_blocks(gpu_ctx, L, B, K, chunks, precision):
+    """Calls of 1 to 33 blocks, with a response issued before some of them
+    (its crossfade falls into the call, on its first block, or in the next
+    one), against the FP64 crossfade model."""
+    import torch
+
+    from helpers import crossfade_model, snr_db
+    calls = [4, 5, 1, 16, 8, 2, 9, 12, 1, 13, 33, 3, 17]
+    at = {0: 0, 3: 1, 4: 2, 5: 3, 7: 4, 9: 5, 10: 6}  # call -> response
+    C, nb = 3, sum(calls)
+    starts = np.cumsum([0] + calls)
+    x = T.signals.input_bank(C, nb * B, base_seed=41)
+    irs = [T.signals.ir_bank(C, L, k, base_seed=43) for k in range(len(at))]
+    conv = T.TANConvolution(gpu_ctx, ir_precision=precision, pass_blocks=K, max_tail_chunks=chunks)
+    assert conv.InitGpu(T.TAN_CONVOLUTION_METHOD_FFT_UNIFORM_PARTITIONED, L, B, C) == T.AMF_OK
+    xd = torch.from_numpy(x).cuda()
+    yd = torch.zeros_like(xd)
+    for i, n in enumerate(calls):
+        b = int(starts[i])
+        if i in at:
+            assert conv.UpdateResponseTD(irs[at[i]], L) == T.AMF_OK
+        rc, done = conv.Process(xd[:, b * B:(b + n) * B], yd[:, b * B:(b + n) * B])
+        assert rc == T.AMF_OK and done == n * B
+    conv.Synchronize()
+    conv.Terminate()
+    y = yd.cpu().numpy()
+    # every switch falls two blocks after its update (none is issued while another is armed)
+    sw = [int(starts[i]) + 2 for i in at]
+    for c in range(C):
+        ref = crossfade_model(x[c], [h[c] for h in irs], sw, B)
+        if precision == 0:
+            assert np.abs(y[c] - ref).max() <= 1e-5
+        assert snr_db(ref, y[c]) >= (120.0, 60.0, 45.0)[precision]
