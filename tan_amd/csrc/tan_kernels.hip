@@ -1921,11 +1921,258 @@ __global__ __launch_bounds__(256) void k_ir_transform_rows_group(const IrArgs *_
 
 #if TANX_IN(4)
 // ---------------------------------------------------------------------------
-// TANFFT transforms, one workgroup per channel.  M is the complex FFT size
-// (N for complex directions, N/2 for real ones).
+// TANFFT.  An N-point transform (N = 64..2,048) is run by N / 16 threads that
+// hold 16 points each in registers: two or three Stockham stages of radix 16
+// or 8, with one exchange through LDS between stages.  In every stage thread
+// t holds the points t + s N/16, s < 16, and the last stage leaves the
+// results in the same places, so global memory is read and written straight
+// from registers, coalesced.  (Radix-4 stages that go through LDS each time
+// made five of it, and two buffers: 2,000 points of 1,000 channels took 9.6
+// us as 1,000 workgroups of four waves, now one wave each; TANFFT of 12
+// channels x 2^18 points 83 to 45 us.)
 // ---------------------------------------------------------------------------
+template <bool INV>
+__device__ __forceinline__ float2 mul_ni(float2 v)  // v W_4 (forward -i, inverse +i)
+{
+    return INV ? make_float2(-v.y, v.x) : make_float2(v.y, -v.x);
+}
+template <bool INV>
+__device__ __forceinline__ float2 mul_w(float2 v, float c, float s)  // v (c - i s), inverse v (c + i s)
+{
+    return cmul(v, make_float2(c, INV ? s : -s));
+}
+
+// In-place DFT of v, natural order (R = 4, 8, 16)
+template <bool INV>
+__device__ __forceinline__ void dft4(float2 &a, float2 &b, float2 &c, float2 &d)
+{
+    const float2 s02 = cadd(a, c), d02 = csub(a, c), s13 = cadd(b, d), d13 = mul_ni<INV>(csub(b, d));
+    a = cadd(s02, s13);
+    b = cadd(d02, d13);
+    c = csub(s02, s13);
+    d = csub(d02, d13);
+}
+template <int R, bool INV>
+__device__ __forceinline__ void dft(float2 (&v)[R])
+{
+    constexpr float kC1 = 0.92387953251128675613f, kS1 = 0.38268343236508977173f, kH = 0.70710678118654752440f;
+    if constexpr (R == 8) {
+        // even and odd halves, the odd ones times W_8^k
+        dft4<INV>(v[0], v[2], v[4], v[6]);
+        dft4<INV>(v[1], v[3], v[5], v[7]);
+        const float2 o[4] = {v[1], mul_w<INV>(v[3], kH, kH), mul_ni<INV>(v[5]), mul_w<INV>(v[7], -kH, kH)};
+        const float2 e[4] = {v[0], v[2], v[4], v[6]};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            v[k] = cadd(e[k], o[k]);
+            v[k + 4] = csub(e[k], o[k]);
+        }
+    } else {
+        static_assert(R == 16, "radix");
+        // columns r (points r + 4 n), times W_16^(r k), then rows
+#pragma unroll
+        for (int r = 0; r < 4; r++) dft4<INV>(v[r], v[r + 4], v[r + 8], v[r + 12]);
+        v[5] = mul_w<INV>(v[5], kC1, kS1);    // r = 1: k = 1, 2, 3 at v[5], v[9], v[13]
+        v[9] = mul_w<INV>(v[9], kH, kH);
+        v[13] = mul_w<INV>(v[13], kS1, kC1);
+        v[6] = mul_w<INV>(v[6], kH, kH);      // r = 2
+        v[10] = mul_ni<INV>(v[10]);
+        v[14] = mul_w<INV>(v[14], -kH, kH);
+        v[7] = mul_w<INV>(v[7], kS1, kC1);    // r = 3
+        v[11] = mul_w<INV>(v[11], -kH, kH);
+        v[15] = mul_w<INV>(v[15], -kC1, -kS1);
+        float2 o[16];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            dft4<INV>(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+#pragma unroll
+            for (int m = 0; m < 4; m++) o[k + 4 * m] = v[4 * k + m];
+        }
+#pragma unroll
+        for (int k = 0; k < 16; k++) v[k] = o[k];
+    }
+}
+
+// LDS place of point i: a gap every 16 points, so that a stage's writes,
+// whose lanes lie up to 16 points apart, spread over the banks
+__device__ __forceinline__ int fft_at(int i) { return i + (i >> 4); }
+constexpr int fft_lds_size(int n) { return n + n / 16; }
+
+// Stage of radix R with p points already transformed: butterfly j of a thread
+// takes its points j + m (16 / R), times W_{pR}^{m k}, k = q mod p for q = t +
+// j N/16, and (unless it is the last) leaves output m at (q - k) R + k + m p.
+template <int N, int R, int P, bool INV>
+__device__ __forceinline__ void fft_stage(float2 (&x)[16], float2 *buf, int t, const float2 *__restrict__ tw)
+{
+    constexpr int NT = N / 16, J = 16 / R;
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const int q = t + j * NT, k = q & (P - 1);
+        float2 v[R];
+#pragma unroll
+        for (int m = 0; m < R; m++) v[m] = x[j + m * J];
+        if constexpr (P > 1) {
+#pragma unroll
+            for (int m = 1; m < R; m++) {
+                float2 w = tw[m * k * (N / (P * R))];
+                if (INV) w.y = -w.y;
+                v[m] = cmul(v[m], w);
+            }
+        }
+        dft<R, INV>(v);
+        if constexpr (P * R < N) {
+#pragma unroll
+            for (int m = 0; m < R; m++) buf[fft_at((q - k) * R + k + m * P)] = v[m];
+        } else {
+#pragma unroll
+            for (int m = 0; m < R; m++) x[j + m * J] = v[m];
+        }
+    }
+    if constexpr (P * R < N) {
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 16; s++) x[s] = buf[fft_at(t + s * NT)];
+        __syncthreads();
+    }
+}
+
+// N-point FFT of x (thread t of the transform's N / 16), through buf
+// (fft_lds_size(N) points of LDS of its own).  All threads of the workgroup
+// call it.  tw: W_N table.
+template <int N, bool INV>
+__device__ __forceinline__ void fft_regs(float2 (&x)[16], float2 *buf, int t, const float2 *__restrict__ tw)
+{
+    if constexpr (N == 64) {
+        fft_stage<N, 8, 1, INV>(x, buf, t, tw);
+        fft_stage<N, 8, 8, INV>(x, buf, t, tw);
+    } else if constexpr (N == 128) {
+        fft_stage<N, 16, 1, INV>(x, buf, t, tw);
+        fft_stage<N, 8, 16, INV>(x, buf, t, tw);
+    } else if constexpr (N == 256) {
+        fft_stage<N, 16, 1, INV>(x, buf, t, tw);
+        fft_stage<N, 16, 16, INV>(x, buf, t, tw);
+    } else if constexpr (N == 512) {
+        fft_stage<N, 8, 1, INV>(x, buf, t, tw);
+        fft_stage<N, 8, 8, INV>(x, buf, t, tw);
+        fft_stage<N, 8, 64, INV>(x, buf, t, tw);
+    } else if constexpr (N == 1024) {
+        fft_stage<N, 16, 1, INV>(x, buf, t, tw);
+        fft_stage<N, 8, 16, INV>(x, buf, t, tw);
+        fft_stage<N, 8, 128, INV>(x, buf, t, tw);
+    } else {
+        static_assert(N == 2048, "size");
+        fft_stage<N, 16, 1, INV>(x, buf, t, tw);
+        fft_stage<N, 16, 16, INV>(x, buf, t, tw);
+        fft_stage<N, 8, 256, INV>(x, buf, t, tw);
+    }
+}
+
+// Two floats of a caller's row: one 8-byte access where the rows allow it
+// (al8: the base and the channel stride are multiples of 8 bytes)
+__device__ __forceinline__ float2 ld_pair(const float *p, bool al8)
+{
+    return al8 ? *reinterpret_cast<const float2 *>(p) : make_float2(p[0], p[1]);
+}
+__device__ __forceinline__ void st_pair(float *p, float2 v, bool al8)
+{
+    if (al8) {
+        *reinterpret_cast<float2 *>(p) = v;
+    } else {
+        p[0] = v.x;
+        p[1] = v.y;
+    }
+}
+
+// Transforms of 64..2,048 complex points: workgroups of one wave (two at
+// 2,048 points), 1,024 / M channels each.  M is the complex size (N for
+// complex directions, N/2 for real ones).
+constexpr int fft_threads_of(int M) { return M / 16 > 64 ? M / 16 : 64; }
+
 template <int M>
-__global__ __launch_bounds__(M / 4 > 64 ? (M / 4 < 1024 ? M / 4 : 1024) : 64) void k_fft(FftArgs a)
+__global__ __launch_bounds__(fft_threads_of(M)) void k_fft(FftArgs a, int channels, bool al8)
+{
+    constexpr int NT = M / 16, PER = fft_threads_of(M) / NT;
+    __shared__ float2 lds[PER * fft_lds_size(M)];
+    const int t = threadIdx.x % NT, sub = threadIdx.x / NT;
+    const int c = blockIdx.x * PER + sub;
+    const bool on = c < channels;  // the others compute a copy of the last channel, not stored
+    const size_t row = (size_t)min(c, channels - 1) * a.stride;
+    const float *in = a.in + row;
+    float *out = a.out + row;
+    float2 *buf = lds + sub * fft_lds_size(M);
+    const int mode = a.mode, imoff = M + 8;
+    float2 x[16];
+    if (mode <= 2 || mode == 4) {
+#pragma unroll
+        for (int s = 0; s < 16; s++) x[s] = ld_pair(in + 2 * (t + s * NT), al8);
+    } else {
+        // packed spectrum: element 0 = (DC.re, Nyquist.re); imaginary parts of
+        // DC and Nyquist are ignored as a c2r transform does
+#pragma unroll
+        for (int s = 0; s < 16; s++) {
+            const int k = t + s * NT;
+            x[s] = mode == 3 ? ld_pair(in + 2 * k, al8) : make_float2(in[k], in[imoff + k]);
+            if (k == 0) x[s].y = mode == 3 ? in[2 * M] : in[M];
+            buf[fft_at(k)] = x[s];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 16; s++) {
+            const int k = t + s * NT;
+            const float2 w = a.twN[k], v = x[s], o = buf[fft_at((M - k) & (M - 1))];
+            // c2r_pre_w
+            if (k == 0) {
+                x[s] = make_float2(v.x + v.y, v.x - v.y);
+            } else {
+                const float er = v.x + o.x, ei = v.y - o.y;
+                const float dr = v.x - o.x, di = v.y + o.y;
+                const float orr = fmaf(dr, w.x, di * w.y), oi = fmaf(di, w.x, -(dr * w.y));
+                x[s] = make_float2(er - oi, ei + orr);
+            }
+        }
+        __syncthreads();
+    }
+    const bool inv = mode == 1 || mode == 3 || mode == 5;
+    if (inv) fft_regs<M, true>(x, buf, t, a.twM);
+    else fft_regs<M, false>(x, buf, t, a.twM);
+    if (mode == 2 || mode == 4) {
+#pragma unroll
+        for (int s = 0; s < 16; s++) buf[fft_at(t + s * NT)] = x[s];
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 16; s++) {
+            const int k = t + s * NT;
+            const float2 w = a.twN[k], z0 = x[s], zc = buf[fft_at((M - k) & (M - 1))];
+            float2 X;
+            if (k == 0) {
+                X = make_float2(z0.x + z0.y, 0.f);
+                const float ny = z0.x - z0.y;
+                if (on) {
+                    if (mode == 2) st_pair(out + 2 * M, make_float2(ny, 0.f), al8);
+                    else { out[M] = ny; out[imoff + M] = 0.f; }
+                }
+            } else {
+                // r2c_post_w
+                const float er = 0.5f * (z0.x + zc.x), ei = 0.5f * (z0.y - zc.y);
+                const float dr = z0.x - zc.x, di = z0.y + zc.y;
+                const float orr = 0.5f * di, oi = -0.5f * dr;
+                X = make_float2(er + fmaf(w.x, orr, -(w.y * oi)), ei + fmaf(w.x, oi, w.y * orr));
+            }
+            if (!on) continue;
+            if (mode == 2) st_pair(out + 2 * k, X, al8);
+            else { out[k] = X.x; out[imoff + k] = X.y; }
+        }
+        return;
+    }
+    if (!on) return;
+    const float sc = mode == 0 ? 1.f : mode == 1 ? 1.0f / (float)M : 1.0f / (2.0f * (float)M);
+#pragma unroll
+    for (int s = 0; s < 16; s++) st_pair(out + 2 * (t + s * NT), make_float2(x[s].x * sc, x[s].y * sc), al8);
+}
+
+// Fewer than 64 complex points: one workgroup per channel
+template <int M>
+__global__ __launch_bounds__(M / 4 > 64 ? (M / 4 < 1024 ? M / 4 : 1024) : 64) void k_fft_small(FftArgs a)
 {
     __shared__ float2 s0[M > 1 ? M : 2], s1[M > 1 ? M : 2], s2[M > 1 ? M : 2];
     const int c = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
@@ -1981,9 +2228,9 @@ __global__ __launch_bounds__(M / 4 > 64 ? (M / 4 < 1024 ? M / 4 : 1024) : 64) vo
 // M = M1 * M2 and n = n1 * M2 + n2, k = k1 + M1 * k2:
 //   Y[k1][n2] = W_M^(n2 k1) * sum_n1 x[n1 M2 + n2] W_M1^(n1 k1)   (columns)
 //   X[k1 + M1 k2] = sum_n2 Y[k1][n2] W_M2^(n2 k2)                  (rows)
-// Each workgroup transforms T = 4096 / size columns or rows in LDS (64 KB),
-// so global reads and writes come in runs of T consecutive elements.  The
-// twiddles between the steps are generated in FP64 and rounded once.
+// A workgroup transforms T = 4,096 / size columns or rows (fft_regs), the
+// index of the column or row running fastest over its lanes, so that both
+// sides read and write runs of T elements (64 bytes at 2^18 points).
 // ---------------------------------------------------------------------------
 struct Fft4Pass {
     const float2 *in;
@@ -1995,93 +2242,119 @@ struct Fft4Pass {
     const float2 *tw;                  // W_M1 (columns) or W_M2 (rows)
 };
 
-// exp(-+2 pi i r / 2^logn) rounded once to FP32 (sign + for the inverse)
-__device__ __forceinline__ float2 tw_fp64(unsigned long long r, int logn, bool inv)
+// exp(-+2 pi i r / 2^logn) in FP64 (sign + for the inverse)
+struct Cplx64 {
+    double re, im;
+};
+__device__ __forceinline__ Cplx64 tw_fp64(unsigned long long r, int logn, bool inv)
 {
-    double s, c;
-    sincospi(-2.0 * (double)r / (double)(1ull << logn), &s, &c);
-    return make_float2((float)c, (float)(inv ? -s : s));
+    Cplx64 w;
+    sincospi(-2.0 * (double)r / (double)(1ull << logn), &w.im, &w.re);
+    if (inv) w.im = -w.im;
+    return w;
 }
+__device__ __forceinline__ Cplx64 mul64(Cplx64 a, Cplx64 b)
+{
+    return Cplx64{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+}
+__device__ __forceinline__ float2 round64(Cplx64 w) { return make_float2((float)w.re, (float)w.im); }
 
 constexpr int kFft4Tile = 4096;  // complex elements a four-step workgroup holds
+
+// the columns of a tile an odd number of places apart in LDS
+template <int N>
+struct Fft4Geo {
+    static constexpr int T = kFft4Tile / N, NT = N / 16, kStride = fft_lds_size(N) | 1;
+};
 
 template <int M1>
 __global__ __launch_bounds__(256) void k_fft4_cols(Fft4Pass a)
 {
-    constexpr int T = kFft4Tile / M1;  // columns per workgroup
-    __shared__ float2 s0[kFft4Tile], s1[kFft4Tile];
-    const int c = blockIdx.y, tid = threadIdx.x;
+    using Geo = Fft4Geo<M1>;
+    __shared__ float2 lds[Geo::T * Geo::kStride];
+    const int c = blockIdx.y, col = threadIdx.x % Geo::T, t = threadIdx.x / Geo::T;
     const long long M2 = 1ll << (a.logM - a.logM1);
-    const long long n20 = (long long)blockIdx.x * T;
-    const float2 *x = a.in + (size_t)c * a.in_stride;
-    // column t of the tile as LDS row t; runs of T consecutive n2 per n1
-    for (int e = tid; e < kFft4Tile; e += 256) {
-        const int t = e % T, n1 = e / T;
-        s0[t * M1 + n1] = x[(size_t)n1 * M2 + n20 + t];
-    }
-    __syncthreads();
-    const float2 *z = a.inv ? fft_lds_n<M1, true>(s0, s1, T, a.tw) : fft_lds_n<M1, false>(s0, s1, T, a.tw);
-    float2 *y = a.out + (size_t)c * a.out_stride;
+    const long long n2 = (long long)blockIdx.x * Geo::T + col;
+    const float2 *in = a.in + (size_t)c * a.in_stride + n2;
+    float2 x[16];
+#pragma unroll
+    for (int s = 0; s < 16; s++) x[s] = in[(size_t)(t + s * Geo::NT) * M2];
+    if (a.inv) fft_regs<M1, true>(x, lds + col * Geo::kStride, t, a.tw);
+    else fft_regs<M1, false>(x, lds + col * Geo::kStride, t, a.tw);
+    // W_M^(n2 k1) for k1 = t, t + NT, ...: a product per output in FP64 (error
+    // below 16 rounding steps of it), rounded once; a sincospi per output was
+    // half of the kernel's time
     const unsigned long long mask = (1ull << a.logM) - 1;
-    for (int e = tid; e < kFft4Tile; e += 256) {
-        const int t = e % T, k1 = e / T;
-        const long long n2 = n20 + t;
-        const float2 w = tw_fp64(((unsigned long long)n2 * (unsigned long long)k1) & mask, a.logM, a.inv != 0);
-        y[(size_t)k1 * M2 + n2] = cmul(z[t * M1 + k1], w);
+    Cplx64 w = tw_fp64(((unsigned long long)n2 * (unsigned long long)t) & mask, a.logM, a.inv != 0);
+    const Cplx64 step = tw_fp64(((unsigned long long)n2 * (unsigned long long)Geo::NT) & mask, a.logM, a.inv != 0);
+    float2 *y = a.out + (size_t)c * a.out_stride + n2;
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+        y[(size_t)(t + s * Geo::NT) * M2] = cmul(x[s], round64(w));
+        w = mul64(w, step);
     }
 }
 
 template <int M2>
 __global__ __launch_bounds__(256) void k_fft4_rows(Fft4Pass a)
 {
-    constexpr int T = kFft4Tile / M2;  // rows per workgroup
-    __shared__ float2 s0[kFft4Tile], s1[kFft4Tile];
-    const int c = blockIdx.y, tid = threadIdx.x;
+    using Geo = Fft4Geo<M2>;
+    __shared__ float2 lds[Geo::T * Geo::kStride];
+    const int c = blockIdx.y, row = threadIdx.x % Geo::T, t = threadIdx.x / Geo::T;
     const long long M1 = 1ll << a.logM1;
-    const long long k10 = (long long)blockIdx.x * T;
-    const float2 *y = a.in + (size_t)c * a.in_stride + (size_t)k10 * M2;
-    for (int e = tid; e < kFft4Tile; e += 256) s0[e] = y[e];
-    __syncthreads();
-    const float2 *z = a.inv ? fft_lds_n<M2, true>(s0, s1, T, a.tw) : fft_lds_n<M2, false>(s0, s1, T, a.tw);
-    float2 *X = a.out + (size_t)c * a.out_stride;
-    for (int e = tid; e < kFft4Tile; e += 256) {
-        const int t = e % T, k2 = e / T;
-        const float2 v = z[t * M2 + k2];
-        X[(size_t)k2 * M1 + k10 + t] = make_float2(v.x * a.scale, v.y * a.scale);
-    }
+    const long long k1 = (long long)blockIdx.x * Geo::T + row;
+    const float2 *y = a.in + (size_t)c * a.in_stride + (size_t)k1 * M2;
+    float2 x[16];
+#pragma unroll
+    for (int s = 0; s < 16; s++) x[s] = y[t + s * Geo::NT];
+    if (a.inv) fft_regs<M2, true>(x, lds + row * Geo::kStride, t, a.tw);
+    else fft_regs<M2, false>(x, lds + row * Geo::kStride, t, a.tw);
+    float2 *X = a.out + (size_t)c * a.out_stride + k1;
+#pragma unroll
+    for (int s = 0; s < 16; s++) X[(size_t)(t + s * Geo::NT) * M1] = make_float2(x[s].x * a.scale, x[s].y * a.scale);
 }
 
 // Real forward transforms of 2M points from Z = FFT_M(z) (z[n] = x[2n] +
 // i x[2n+1]): bins 0..M into the interleaved (mode 2) or planar (mode 4,
-// imaginary parts from M + 8) layout, as k_fft writes them.
+// imaginary parts from M + 8) layout, as k_fft writes them.  A thread takes
+// kFft4Bins bins 256 apart, their W_2M^k one FP64 product after another.
+constexpr int kFft4Bins = 8;
+
 __global__ __launch_bounds__(256) void k_fft4_r2c_post(const float2 *Z, long long zs, float *out, long long os,
                                                        int logM, int mode)
 {
     const int c = blockIdx.y;
     const long long M = 1ll << logM;
-    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (k > M) return;
+    const long long k0 = (long long)blockIdx.x * (256 * kFft4Bins) + threadIdx.x;
     const float2 *z = Z + (size_t)c * zs;
     float *o = out + (size_t)c * os;
-    float2 X;
-    if (k == 0 || k == M) {
-        const float2 z0 = z[0];
-        X = make_float2(k == 0 ? z0.x + z0.y : z0.x - z0.y, 0.f);
-    } else {
-        // r2c_post with the W_2M twiddle generated in FP64
-        const float2 z0 = z[k], zc = z[M - k];
-        const float er = 0.5f * (z0.x + zc.x), ei = 0.5f * (z0.y - zc.y);
-        const float dr = z0.x - zc.x, di = z0.y + zc.y;
-        const float orr = 0.5f * di, oi = -0.5f * dr;
-        const float2 w = tw_fp64((unsigned long long)k, logM + 1, false);
-        X = make_float2(er + fmaf(w.x, orr, -(w.y * oi)), ei + fmaf(w.x, oi, w.y * orr));
-    }
-    if (mode == 2) {
-        o[2 * k] = X.x;
-        o[2 * k + 1] = X.y;
-    } else {
-        o[k] = X.x;
-        o[M + 8 + k] = X.y;
+    Cplx64 w64 = tw_fp64((unsigned long long)k0, logM + 1, false);
+    const Cplx64 step = tw_fp64(256, logM + 1, false);
+#pragma unroll
+    for (int u = 0; u < kFft4Bins; u++) {
+        const long long k = k0 + 256 * u;
+        if (k > M) return;
+        float2 X;
+        if (k == 0 || k == M) {
+            const float2 z0 = z[0];
+            X = make_float2(k == 0 ? z0.x + z0.y : z0.x - z0.y, 0.f);
+        } else {
+            // r2c_post with the W_2M twiddle generated in FP64
+            const float2 z0 = z[k], zc = z[M - k];
+            const float er = 0.5f * (z0.x + zc.x), ei = 0.5f * (z0.y - zc.y);
+            const float dr = z0.x - zc.x, di = z0.y + zc.y;
+            const float orr = 0.5f * di, oi = -0.5f * dr;
+            const float2 w = round64(w64);
+            X = make_float2(er + fmaf(w.x, orr, -(w.y * oi)), ei + fmaf(w.x, oi, w.y * orr));
+        }
+        if (mode == 2) {
+            o[2 * k] = X.x;
+            o[2 * k + 1] = X.y;
+        } else {
+            o[k] = X.x;
+            o[M + 8 + k] = X.y;
+        }
+        w64 = mul64(w64, step);
     }
 }
 
@@ -2098,22 +2371,29 @@ __global__ __launch_bounds__(256) void k_fft4_c2r_pre(const float *in, long long
 {
     const int c = blockIdx.y;
     const long long M = 1ll << logM;
-    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (k >= M) return;
+    const long long k0 = (long long)blockIdx.x * (256 * kFft4Bins) + threadIdx.x;
     const float *x = in + (size_t)c * is;
-    const float2 a = c2r_bin(x, M, k, mode);
-    float2 r;
-    if (k == 0) {
-        r = make_float2(a.x + a.y, a.x - a.y);
-    } else {
-        const float2 b = c2r_bin(x, M, M - k, mode);
-        const float er = a.x + b.x, ei = a.y - b.y;
-        const float dr = a.x - b.x, di = a.y + b.y;
-        const float2 w = tw_fp64((unsigned long long)k, logM + 1, false);
-        const float orr = fmaf(dr, w.x, di * w.y), oi = fmaf(di, w.x, -(dr * w.y));
-        r = make_float2(er - oi, ei + orr);
+    Cplx64 w64 = tw_fp64((unsigned long long)k0, logM + 1, false);
+    const Cplx64 step = tw_fp64(256, logM + 1, false);
+#pragma unroll
+    for (int u = 0; u < kFft4Bins; u++) {
+        const long long k = k0 + 256 * u;
+        if (k >= M) return;
+        const float2 a = c2r_bin(x, M, k, mode);
+        float2 r;
+        if (k == 0) {
+            r = make_float2(a.x + a.y, a.x - a.y);
+        } else {
+            const float2 b = c2r_bin(x, M, M - k, mode);
+            const float er = a.x + b.x, ei = a.y - b.y;
+            const float dr = a.x - b.x, di = a.y + b.y;
+            const float2 w = round64(w64);
+            const float orr = fmaf(dr, w.x, di * w.y), oi = fmaf(di, w.x, -(dr * w.y));
+            r = make_float2(er - oi, ei + orr);
+        }
+        A[(size_t)c * as + k] = r;
+        w64 = mul64(w64, step);
     }
-    A[(size_t)c * as + k] = r;
 }
 
 // ---------------------------------------------------------------------------
@@ -2997,7 +3277,7 @@ static hipError_t launch_fft4(int channels, const FftArgs &a, hipStream_t s)
     cols.tw = a.tw1;
     rows.tw = a.tw2;
     rows.scale = a.mode == 1 ? 1.0f / (float)M : (real && inv) ? 1.0f / (2.0f * (float)M) : 1.0f;
-    const unsigned bins = (unsigned)((M + 1 + 255) / 256);
+    const unsigned bins = (unsigned)((M + 256 * kFft4Bins) / (256 * kFft4Bins));  // bins 0..M
     hipError_t e;
     if (!real) {
         cols.in = reinterpret_cast<const float2 *>(a.in);
@@ -3045,11 +3325,18 @@ hipError_t launch_fft(int channels, const FftArgs &a, hipStream_t s)
     const bool real = a.mode >= 2;
     const int M = real ? (1 << (a.log2len - 1)) : (1 << a.log2len);
     if (M > kFftLdsMax) return launch_fft4(channels, a, s);
+    const bool al8 = ((reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.out)) & 7) == 0 && a.stride % 2 == 0;
     switch (M) {
-#define TANX_FFT_CASE(V) case V: hipLaunchKernelGGL(k_fft<V>, dim3(channels), dim3(fft_threads(V)), 0, s, a); break;
-        TANX_FFT_CASE(1) TANX_FFT_CASE(2) TANX_FFT_CASE(4) TANX_FFT_CASE(8) TANX_FFT_CASE(16)
-        TANX_FFT_CASE(32) TANX_FFT_CASE(64) TANX_FFT_CASE(128) TANX_FFT_CASE(256) TANX_FFT_CASE(512)
-        TANX_FFT_CASE(1024) TANX_FFT_CASE(2048)
+#define TANX_FFT_CASE(V) case V: hipLaunchKernelGGL(k_fft_small<V>, dim3(channels), dim3(64), 0, s, a); break;
+        TANX_FFT_CASE(1) TANX_FFT_CASE(2) TANX_FFT_CASE(4) TANX_FFT_CASE(8) TANX_FFT_CASE(16) TANX_FFT_CASE(32)
+#undef TANX_FFT_CASE
+#define TANX_FFT_CASE(V)                                                                                       \
+    case V:                                                                                                    \
+        hipLaunchKernelGGL(k_fft<V>, dim3((unsigned)((channels * (V / 16) + fft_threads_of(V) - 1) / fft_threads_of(V))), \
+                           dim3(fft_threads_of(V)), 0, s, a, channels, al8);                                   \
+        break;
+        TANX_FFT_CASE(64) TANX_FFT_CASE(128) TANX_FFT_CASE(256) TANX_FFT_CASE(512) TANX_FFT_CASE(1024)
+        TANX_FFT_CASE(2048)
 #undef TANX_FFT_CASE
     default:
         return hipErrorInvalidValue;

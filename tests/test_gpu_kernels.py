@@ -104,3 +104,44 @@ def test_calls_of_many_blocks(gpu_ctx, L, B, K, chunks, precision):
         if precision == 0:
             assert np.abs(y[c] - ref).max() <= 1e-5
         assert snr_db(ref, y[c]) >= (120.0, 60.0, 45.0)[precision]
+
+
+# sizes of each stage plan, channel counts that leave a workgroup part empty,
+# rows whose pairs of floats are not 8-byte aligned
+@pytest.mark.parametrize("log2m,C,pad,off", [(6, 17, 0, 0), (6, 3, 3, 1), (7, 9, 1, 0), (8, 5, 0, 1), (9, 3, 2, 0),
+                                             (10, 2, 5, 1), (11, 3, 1, 1)])
+@pytest.mark.parametrize("direction", range(6))
+def test_fft_row_layouts(gpu_ctx, log2m, C, pad, off, direction):
+    import torch
+    log2n = log2m if direction < 2 else log2m + 1
+    n, m = 1 << log2n, 1 << (log2n - 1)
+    rng = np.random.default_rng(100 * log2m + direction)
+    x = rng.standard_normal((C, 2 * n + pad)).astype(np.float32)
+    base = torch.zeros(C * (2 * n + pad) + off, device="cuda")
+    base[off:] = torch.from_numpy(x).cuda().reshape(-1)
+    ob = torch.full_like(base, 9.0)
+    xin = base[off:].view(C, 2 * n + pad)
+    out = ob[off:].view(C, 2 * n + pad)
+    f = T.TANFFT(gpu_ctx)
+    assert f.Init() == T.AMF_OK
+    assert f.Transform(direction, log2n, C, xin, out) == T.AMF_OK
+    got = out.cpu().numpy().astype(np.float64)
+    x64 = x.astype(np.float64)
+    if direction < 2:
+        z = x64[:, 0:2 * n:2] + 1j * x64[:, 1:2 * n:2]
+        ref = np.fft.fft(z) if direction == 0 else np.fft.ifft(z)
+        g, used = got[:, 0:2 * n:2] + 1j * got[:, 1:2 * n:2], 2 * n
+    elif direction in (2, 4):
+        ref = np.fft.rfft(x64[:, :n])
+        if direction == 2:
+            g, used = got[:, 0:n + 2:2] + 1j * got[:, 1:n + 2:2], n + 2
+        else:
+            g, used = got[:, :m + 1] + 1j * got[:, m + 8:2 * m + 9], 2 * m + 9
+            assert np.all(got[:, m + 1:m + 8] == 9.0)
+    else:
+        z = (x64[:, 0:n + 2:2] + 1j * x64[:, 1:n + 2:2] if direction == 3
+             else x64[:, :m + 1] + 1j * x64[:, m + 8:2 * m + 9])
+        z[:, 0], z[:, m] = z[:, 0].real, z[:, m].real
+        ref, g, used = np.fft.irfft(z, n), got[:, :n], n
+    assert np.abs(g - ref).max() <= 3e-7 * np.abs(ref).max() * log2n  # the bound of test_gpu_fft.py
+    assert np.all(got[:, used:] == 9.0)
