@@ -1587,10 +1587,6 @@ static int32_t process_call(tanx_conv *cv, const float *din, long long in_stride
     a.yout = dout;
     a.out_stride = out_stride;
     a.xprev = cv->xprev;
-    // rows the caches hold: a chunk's window is filled from rows its neighbour
-    // reads too (16 blocks of 64 channels x 65,536 taps: 29 against 35 us);
-    // larger objects stream (1,024 channels: 268 against 287 us)
-    a.cached = (size_t)cv->C * cv->P * B * (sizeof(float2) + ir_elem_bytes(cv->irtype)) <= kCachedRowsMax;
     int xb = -1, done = 0, slot_a = cv->cur;
     for (; done < n; done++) {
         const bool xf_next = cv->delayed && cv->ticks == cv->switch_at;
@@ -1634,10 +1630,17 @@ static int32_t process_call(tanx_conv *cv, const float *din, long long in_stride
     // workgroups; 8 blocks with a crossfade 54, 52 and 55 us), of at least 16
     // partitions, as many as the rows hold
     const int rows = 4 * cv->kp * cv->maxchunk, groups = done > 8 ? 256 : 512;
+    const bool small = (size_t)cv->C * cv->P * B * (sizeof(float2) + ir_elem_bytes(cv->irtype)) <= kCachedRowsMax;
     int chunks = std::max(1, std::min((groups + cv->C - 1) / cv->C, cv->P / 16));
+    if (small) chunks = std::max(chunks, (cv->P + 63) / 64);
     chunks = std::max(1, std::min(chunks, (rows - done) / outs));
     a.pc = (cv->P + chunks - 1) / chunks;
     a.nchunk = (cv->P + a.pc - 1) / a.pc;
+    // ordinary loads and one chain of sums per chunk while the caches hold the
+    // rows (a chunk's window is filled from rows its neighbour reads too): 16
+    // blocks of 64 channels x 65,536 taps 28 us, 35 us with streaming loads;
+    // larger objects stream (1,024 channels: 268 against 287 us)
+    a.cached = small && a.pc <= 64;
     a.X = cv->T;
     a.T = cv->T + (size_t)cv->C * done * B;
     hipStream_t s = cv->ctx->proc;

@@ -736,14 +736,14 @@ __device__ void mac_rows(const MacView &w, float4 *red)
 // per kBody partitions.
 //
 // A lane owns E complex bins of the row: one (8-byte loads, 4 KM registers
-// of window and sums) for FP32 rows, two for 16-bit rows (8-byte loads of
-// them), which leaves registers for the next U partitions' rows to be in
+// of window and sums) for FP32 rows of up to 256 bins, two for longer ones
+// and for 16-bit rows (8-byte loads of them), which leaves registers for the next U partitions' rows to be in
 // flight while U are multiplied and for 4 to 7 waves per SIMD.  Rows longer
 // than the workgroup's lanes cover are swept a slice of S bins at a time.  An
 // output costs four multiply-adds per bin and partition: the packed (DC,
 // Nyquist) element's two real products are the same four with a zero and a
 // swapped factor, chosen once per partition (mac_bin).  Bound by HBM: the
-// 12-output pass of 1,024 channels x 65,536 taps at B = 256 takes 201 us (5.3
+// 12-output pass of 1,024 channels x 65,536 taps at B = 256 takes 203 us (5.2
 // TB/s of rows), 247 us with two bins per lane, two lane groups and no loads
 // in flight across a stage (167 VGPRs instead of 104).  Ordinary instead of
 // nontemporal loads: 7% slower; stages of 2 partitions: 4% slower, of 6: no
@@ -756,11 +756,12 @@ struct Bins {
 
 template <int M, int HT>
 struct PassGeo {
-    static constexpr int E = HT == IR_F32 ? 1 : 2;                      // bins per lane
+    static constexpr int E = HT == IR_F32 && M <= kTickThreads ? 1 : 2;  // bins per lane
     static constexpr int S = M < E * kTickThreads ? M : E * kTickThreads;  // bins per slice
     static constexpr int R = S / E;                                     // lanes per slice
     static constexpr int G = kTickThreads / R;                          // lane groups
-    static constexpr int SEG = E == 1 && M <= kTickThreads ? 2 : 1;     // segments of a group's partitions
+    static constexpr int SEG = E == 1 ? 2 : 1;                          // segments of a group's partitions
+    static constexpr int U = E == 2 && HT == IR_F32 ? 2 : 4;            // partitions loaded together
 };
 
 // Bins of lane r of a row's slice (NT: nontemporal)
@@ -785,8 +786,9 @@ __device__ __forceinline__ Bins<E> ld_bins(const float2 *row, int r)
 }
 
 // Lane r's bins of an IR row's slice as stored, and their values
-template <int HT>
+template <int HT, int E>
 struct IrBins {
+    static_assert(E == 2, "16-bit rows");
     v2u raw;
     template <bool NT>
     __device__ __forceinline__ void load(const char *row, int r)
@@ -812,15 +814,15 @@ struct IrBins {
     }
 };
 
-template <>
-struct IrBins<IR_F32> {
-    Bins<1> raw;
+template <int E>
+struct IrBins<IR_F32, E> {
+    Bins<E> raw;
     template <bool NT>
     __device__ __forceinline__ void load(const char *row, int r)
     {
-        raw = ld_bins<1, NT>(reinterpret_cast<const float2 *>(row), r);
+        raw = ld_bins<E, NT>(reinterpret_cast<const float2 *>(row), r);
     }
-    __device__ __forceinline__ Bins<1> value(float) const { return raw; }
+    __device__ __forceinline__ Bins<E> value(float) const { return raw; }
 };
 
 // acc += x h for one bin: hc the factor of the cross products (h.im, 0 for
@@ -853,43 +855,54 @@ struct SweepRows {
 // dc: the lane's first bin is the packed (DC, Nyquist) element.
 // NF filters: HA for outputs k < kA, HB (NF = 2) for outputs k >= kB; with
 // one filter every output is computed (the caller stores those it wants).
-template <int M, int NF, int HT, bool NT, int KM>
+// FOLD: fold() is called once between the partitions before pf and those from pf on
+// (p0 < pf < p1), to put the sums so far aside; the trips are laid so that
+// one starts at pf and the loads in flight go on across it.
+template <int M, int NF, int HT, bool NT, int KM, bool FOLD, class Fold>
 __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA, const char *HB, const float *SA,
-                                           const float *SB, int p0, int p1, int r, bool dc, int kA, int kB,
-                                           Bins<PassGeo<M, HT>::E> (&accA)[KM], Bins<PassGeo<M, HT>::E> (&accB)[KM])
+                                           const float *SB, int p0, int pf, int p1, int r, bool dc, int kA, int kB,
+                                           Bins<PassGeo<M, HT>::E> (&accA)[KM], Bins<PassGeo<M, HT>::E> (&accB)[KM],
+                                           Fold fold)
 {
     constexpr int E = PassGeo<M, HT>::E;
-    constexpr int U = 4;                                                // partitions per stage
-    constexpr int kBody = NF == 2 ? U : KM < 8 ? 8 : KM;  // partitions per loop trip
+    constexpr int U = PassGeo<M, HT>::U;                  // partitions per stage
+    constexpr int kBody = NF == 2 ? 4 : KM < 8 ? 8 : KM;  // partitions per loop trip
     constexpr size_t kRowBytes = (size_t)M * IrRow<HT>::kBytes;
     static_assert(kBody % U == 0 && KM <= kPassMax, "pass length");
     // entry KM - 1 + q of the window holds the row of partition i + q (row
     // -(i + q)) for the trip starting at partition i; output k reads the
     // entry k before it
     Bins<E> win[KM - 1 + kBody];
+    // partitions the first trip skips
+    const int lead = FOLD && pf > p0 && pf < p1 ? (kBody - (pf - p0) % kBody) % kBody : 0;
 #pragma unroll
     for (int k = 0; k < KM; k++)
 #pragma unroll
         for (int e = 0; e < E; e++) {
             accA[k].re[e] = accA[k].im[e] = 0.f;
             accB[k].re[e] = accB[k].im[e] = 0.f;
-            if (k > 0) win[KM - 1 - k].re[e] = win[KM - 1 - k].im[e] = 0.f;
         }
-    if (p0 >= p1) return;
+    // the rows before partition p0 that its outputs reach back to
 #pragma unroll
-    for (int k = 1; k < KM; k++)
-        if (k - p0 < rows.zero_from) win[KM - 1 - k] = ld_bins<E, NT>(rows.at<M>(k - p0), r);
+    for (int t = 0; t < KM - 1 + (FOLD ? kBody : 0); t++) {
+#pragma unroll
+        for (int e = 0; e < E; e++) win[t].re[e] = win[t].im[e] = 0.f;
+        const int back = KM - 1 + lead - t;  // entry t: partition p0 - back
+        if (p0 < p1 && back > 0 && back < KM && back - p0 < rows.zero_from)
+            win[t] = ld_bins<E, NT>(rows.at<M>(back - p0), r);
+    }
+    if (p0 >= p1) return;
 
     struct Stage {
         Bins<E> x[U];
-        IrBins<HT> a[U], b[NF == 2 ? U : 1];
+        IrBins<HT, E> a[U], b[NF == 2 ? U : 1];
         float sa[U], sb[U];
     } cur, nxt;
-    // the rows of partitions i .. i + U - 1 (past the end: the last one's again)
+    // the rows of partitions i .. i + U - 1 (outside the range: its ends' again)
     auto load = [&](Stage &t, int i) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int ii = min(i + u, p1 - 1);
+            const int ii = FOLD ? max(p0, min(i + u, p1 - 1)) : min(i + u, p1 - 1);
             t.x[u] = ld_bins<E, NT>(rows.at<M>(-ii), r);
             t.a[u].template load<NT>(HA + (size_t)ii * kRowBytes, r);
             if constexpr (HT != IR_F32) t.sa[u] = gld(SA + ii);
@@ -899,15 +912,19 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
             }
         }
     };
-    load(cur, p0);
-    for (int i = p0; i < p1; i += kBody) {
+    load(cur, p0 - lead);
+    for (int i = p0 - lead; i < p1; i += kBody) {
+        if (FOLD && i == pf && i > p0) fold();
 #pragma unroll
         for (int q0 = 0; q0 < kBody; q0 += U) {
             load(nxt, i + q0 + U);
+            // the loads stay before the products (moved to their use they would not
+            // be in flight: 38 instead of 28 us in the call of 16 blocks below)
+            asm volatile("" ::: "memory");
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int q = q0 + u;
-                if (i + q < p1) {
+                if ((!FOLD || i + q >= p0) && i + q < p1) {
                     win[KM - 1 + q] = cur.x[u];
                     const Bins<E> hA = cur.a[u].value(HT == IR_F32 ? 1.f : cur.sa[u]);
 #pragma unroll
@@ -946,37 +963,41 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
 
 // The outputs of partitions [i0, i1) (those from pmin on) of one channel's
 // slice: out(f, k) is filter f's output row k (at the slice) or nullptr; the
-// skip is uniform.  The range is cut into segs * G segments (segs <= SEG),
-// each summed as one chain; a lane group takes segs of them (its first one's
+// skip is uniform.  The range is cut into SEG * G segments, each summed as
+// one chain; a lane group takes SEG of them in one sweep (its first one's
 // sums wait in LDS, one float2 per output and thread) and an output adds the
 // segments in order.  All threads call it.
-template <int M, int NF, int HT, bool NT, int KM, class Out>
+template <int M, int NF, int HT, bool NT, int KM, int SEG, class Out>
 __device__ __forceinline__ void sweep_outputs(const SweepRows &rows, const char *HA, const char *HB, const float *SA,
                                               const float *SB, int i0, int i1, int pmin, bool dc0, int kA, int kB,
-                                              int segs, float4 *red, Out out)
+                                              float4 *red, Out out)
 {
     using Geo = PassGeo<M, HT>;
-    const int g = threadIdx.x / Geo::R, r = threadIdx.x % Geo::R;
-    const int ns = segs * Geo::G, span = (i1 - i0 + ns - 1) / ns;
-    const bool both = Geo::SEG == 2 && segs == 2;
-    float2 *sums = reinterpret_cast<float2 *>(red);                          // [G][S]
-    float2 *firsts = sums + kTickThreads;                                    // [outputs][threads]
+    // a group of whole waves: its partitions are uniform over the wave
+    const int g = Geo::G == 1        ? 0
+                  : Geo::R % 64 == 0 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / Geo::R)
+                                     : (int)threadIdx.x / Geo::R;
+    const int r = threadIdx.x % Geo::R;
+    constexpr int NS = SEG * Geo::G;
+    const int span = (i1 - i0 + NS - 1) / NS;
+    float2 *sums = reinterpret_cast<float2 *>(red);  // [G][S]
+    float2 *firsts = sums + kTickThreads;            // [outputs][threads]
     // filter f's output k: the filters' outputs together are at most KM + 1
     auto first = [&](int f, int k) { return firsts + (k + f) * kTickThreads; };
     Bins<Geo::E> acc[2][KM];
-    for (int seg = 0; seg < segs; seg++) {
-        const int q0 = min(i1, i0 + (g * segs + seg) * span), p1 = min(i1, q0 + span);
-        pass_sweep<M, NF, HT, NT, KM>(rows, HA, HB, SA, SB, max(q0, pmin), p1, r, dc0 && r == 0, kA, kB, acc[0],
-                                      acc[1]);
-        if (both && seg == 0) {
+    const int q0 = min(i1, i0 + g * SEG * span), pf = min(i1, q0 + span), p1 = min(i1, q0 + SEG * span);
+    const int p0 = max(q0, pmin);
+    const bool both = SEG == 2 && p0 < pf && pf < p1;
+    pass_sweep<M, NF, HT, NT, KM, SEG == 2>(rows, HA, HB, SA, SB, p0, pf, p1, r, dc0 && r == 0, kA, kB, acc[0], acc[1], [&] {
 #pragma unroll
-            for (int f = 0; f < NF; f++)
+        for (int f = 0; f < NF; f++)
 #pragma unroll
-                for (int k = 0; k < KM; k++)
-                    if (NF == 1 || (f == 0 ? k < kA : k >= kB))
-                        first(f, k)[threadIdx.x] = make_float2(acc[f][k].re[0], acc[f][k].im[0]);
-        }
-    }
+            for (int k = 0; k < KM; k++)
+                if (NF == 1 || (f == 0 ? k < kA : k >= kB)) {
+                    first(f, k)[threadIdx.x] = make_float2(acc[f][k].re[0], acc[f][k].im[0]);
+                    acc[f][k].re[0] = acc[f][k].im[0] = 0.f;
+                }
+    });
     // unrolled over the outputs so that every pointer is picked statically
     // (an output pointer indexed at run time would put the whole argument
     // struct in private memory)
@@ -994,14 +1015,16 @@ __device__ __forceinline__ void sweep_outputs(const SweepRows &rows, const char 
                 else gst(reinterpret_cast<float4 *>(o) + r, make_float4(v.x, v.y, a.re[1], a.im[1]));
             } else {
                 static_assert(Geo::S == M && Geo::G * M == kTickThreads * Geo::E, "pass reduction buffer");
+                // (a group without a second segment: no first one, the sums as they are)
+                if (SEG == 2 && !both) first(f, k)[threadIdx.x] = make_float2(0.f, 0.f);
 #pragma unroll
                 for (int e = 0; e < Geo::E; e++) sums[g * M + Geo::E * r + e] = make_float2(a.re[e], a.im[e]);
                 __syncthreads();
                 for (int b = threadIdx.x; b < M; b += kTickThreads) {
-                    float2 sum = both ? cadd(first(f, k)[b], sums[b]) : sums[b];
+                    float2 sum = SEG == 2 ? cadd(first(f, k)[b], sums[b]) : sums[b];
 #pragma unroll
                     for (int gg = 1; gg < Geo::G; gg++) {
-                        if (both) sum = cadd(sum, first(f, k)[gg * Geo::R + b]);
+                        if constexpr (SEG == 2) sum = cadd(sum, first(f, k)[gg * Geo::R + b]);
                         sum = cadd(sum, sums[gg * M + b]);
                     }
                     gst(o + b, sum);
@@ -1039,7 +1062,7 @@ __device__ void tailk_role(const TickArgs &a, int c, int j, float4 *red)
         const char *HA = reinterpret_cast<const char *>(a.tHa) + at * IrRow<HT>::kBytes;
         const char *HB = NF == 2 ? reinterpret_cast<const char *>(a.tHb) + at * IrRow<HT>::kBytes : nullptr;
         const size_t orow = ((size_t)c * a.nchunk + j) * M + s0;
-        sweep_outputs<M, NF, HT, NT, KM>(rows, HA, HB, SA, SB, i0, i1, a.kgap + 1, s0 == 0, kA, kB, Geo::SEG, red,
+        sweep_outputs<M, NF, HT, NT, KM, Geo::SEG>(rows, HA, HB, SA, SB, i0, i1, a.kgap + 1, s0 == 0, kA, kB, red,
                                          [&](int f, int k) {
                                              float2 *o = f == 0 ? a.kTA[k] : a.kTB[k];
                                              return o ? o + orow : nullptr;
@@ -1470,10 +1493,10 @@ __global__ __launch_bounds__(kTickThreads) void k_window(HeadBatchArgs h, TickAr
 // block.  With every input block at hand the transforms are independent
 // (one wave each up to B = 256, C * n of them), the sweep reads each IR and
 // FDL row once for all n outputs, and only three launches follow each other.
-// Calls of 16 blocks, 64 channels x 65,536 taps at B = 256: 29 us, 89 us a
+// Calls of 16 blocks, 64 channels x 65,536 taps at B = 256: 28 us, 89 us a
 // launch per four blocks; 8 blocks of 1,024 channels x 131,072 taps with FP16
 // rows: 304 us (5.3 TB/s of rows), 577 us with two sweeps; 4 blocks of 1,024
-// channels x 65,536 taps: 188 us.
+// channels x 65,536 taps: 185 us, 222 us before.
 // ---------------------------------------------------------------------------
 template <int M>
 __global__ __launch_bounds__(kTickThreads) void k_call_spectra(CallArgs a)
@@ -1502,6 +1525,8 @@ __global__ __launch_bounds__(kTickThreads) void k_call_spectra(CallArgs a)
     for (int k = tid; k < M; k += NT) row[k] = r2c_post<M>(Z, k, a.twN);
 }
 
+// NT: streamed rows, a chunk's sums in two chains; otherwise (short chunks of
+// rows that the caches hold) ordinary loads and one chain
 template <int M, int NF, int HT, bool NT, int KM>
 __global__ __launch_bounds__(kTickThreads) void k_call_pass(CallArgs a)
 {
@@ -1513,9 +1538,6 @@ __global__ __launch_bounds__(kTickThreads) void k_call_pass(CallArgs a)
     const float *SB = (HT == IR_F32 || NF == 1) ? nullptr : a.SB + (size_t)c * a.P;
     const int i0 = j * a.pc, i1 = min(a.P, i0 + a.pc);
     const int kA = NF == 2 ? a.xb + 1 : a.n, kB = NF == 2 ? a.xb : a.n;
-    // a second segment (shorter chains) costs the reads that fill its window,
-    // n - 1 rows: only for chunks that are long beside it
-    const int segs = i1 - i0 > 64 * Geo::G ? Geo::SEG : 1;
     for (int s0 = 0; s0 < M; s0 += Geo::S) {
         const size_t at = (size_t)c * a.P * M + s0;
         const SweepRows rows = {a.fdl + at, a.X + (size_t)c * a.n * M + s0, a.slot, a.P - 1, a.n};
@@ -1526,7 +1548,8 @@ __global__ __launch_bounds__(kTickThreads) void k_call_pass(CallArgs a)
             if (!(f == 0 ? k < kA : k >= kB && k < a.n)) return nullptr;
             return a.T + (((size_t)c * (a.n + NF - 1) + k + f) * a.nchunk + j) * M + s0;
         };
-        sweep_outputs<M, NF, HT, NT, KM>(rows, HA, HB, SA, SB, i0, i1, 0, s0 == 0, kA, kB, segs, red, out);
+        sweep_outputs<M, NF, HT, NT, KM, NT ? Geo::SEG : 1>(rows, HA, HB, SA, SB, i0, i1, 0, s0 == 0, kA, kB, red,
+                                                            out);
     }
 }
 
