@@ -2429,8 +2429,8 @@ __global__ __launch_bounds__(256) void k_fft4_c2r_pre(const float *in, long long
 // floats for 8 and was bound by LDS.  The window and the filter are placed in
 // LDS so that a step's reads are aligned whatever tap the sum starts at.
 // Measured per block, before and after: 512 channels x 512 taps, B = 256:
-// 11.6 and 8.7 us (one wave per SIMD: its LDS latency); 2,048 channels: 33.2
-// and 15.1 us; 256 channels x 4,096 taps, B = 1024: 161 and 55 us (20 TFLOP/s).
+// 11.9 and 7.9 us (two waves per SIMD: LDS latency); 2,048 channels: 33.0 and
+// 15.6 us; 256 channels x 4,096 taps, B = 1024: 160 and 58 us (18 TFLOP/s).
 // Staging everything as one list with eight loads in flight per lane was no
 // faster (the address selects cost what the round trips saved).
 // ---------------------------------------------------------------------------
@@ -2531,19 +2531,42 @@ __global__ __launch_bounds__(256) void k_td(TdArgs a)
     float *yo = a.yout + (size_t)c * a.out_stride;
     const float step = (float)(1.0 / (double)a.B);
     const float *w0 = w + len - 1 - f0;
-    for (int j0 = R * tid; j0 < n; j0 += R * nt) {
-        float ya[R];
-        td_dot<R>(w0, ha, taps, j0, ya);
-        if (a.Hb) {
-            float yb[R];
-            td_dot<R>(w0, hb, taps, j0, yb);
+    // the lanes beyond those that the n outputs need share the taps: slice s of
+    // the 2^ls slices (of at least 128 taps) sums taps from s * per on, which
+    // shortens the lanes' chains (7 channels x 1,070 taps, B = 64: 20.9 to 8.3 us)
+    const int lanes = (n + R - 1) / R;
+    int ls = 0;
+    while (ls < 3 && (lanes << (ls + 1)) <= nt && (taps >> (ls + 1)) >= 128) ls++;
+    const int per = ((taps + 7) / 8 + (1 << ls) - 1) / (1 << ls) * 8;
+    float *part = hb + (a.Hb ? len : 0);  // [2 filters][slices][n] partial sums
+    const int sl = ls == 0 ? 0 : tid / lanes, k0 = min(taps, sl * per), cnt = min(per, taps - k0);
+    for (int j0 = R * (tid - sl * lanes); j0 < n && sl < (1 << ls); j0 += R * (ls == 0 ? nt : lanes)) {
+        float ya[R], yb[R];
+        td_dot<R>(w0 - k0, ha + k0, cnt, j0, ya);
+        if (a.Hb) td_dot<R>(w0 - k0, hb + k0, cnt, j0, yb);
 #pragma unroll
-            for (int o = 0; o < R; o++)
-                ya[o] = yb[o] * (step * (float)(j0 + o)) + ya[o] * (step * (float)(a.B - (j0 + o)));
+        for (int o = 0; o < R; o++) {
+            if (j0 + o >= n) continue;
+            if (ls > 0) {
+                part[sl * n + j0 + o] = ya[o];
+                if (a.Hb) part[((1 << ls) + sl) * n + j0 + o] = yb[o];
+            } else {
+                if (a.Hb) ya[o] = yb[o] * (step * (float)(j0 + o)) + ya[o] * (step * (float)(a.B - (j0 + o)));
+                yo[j0 + o] = ya[o];
+            }
         }
-#pragma unroll
-        for (int o = 0; o < R; o++)
-            if (j0 + o < n) yo[j0 + o] = ya[o];
+    }
+    if (ls > 0) {
+        __syncthreads();
+        for (int j = tid; j < n; j += nt) {
+            float ya = part[j], yb = a.Hb ? part[(n << ls) + j] : 0.f;
+            for (int s = 1; s < (1 << ls); s++) {
+                ya += part[s * n + j];
+                if (a.Hb) yb += part[(n << ls) + s * n + j];
+            }
+            if (a.Hb) ya = yb * (step * (float)j) + ya * (step * (float)(a.B - j));
+            yo[j] = ya;
+        }
     }
     // the new samples enter the history (this workgroup alone owns channel c)
     float *hw = a.hist + (size_t)c * len;
@@ -3371,7 +3394,10 @@ hipError_t launch_td(const TdArgs &a, hipStream_t s, hipEvent_t ev0, hipEvent_t 
 {
     if (a.C == 0 || a.n == 0) return hipSuccess;
     if (a.len > kMaxTdLen || a.n > a.B) return hipErrorInvalidValue;
-    const size_t smem = sizeof(float) * ((size_t)a.len + a.B + kTdPad + 2 * (size_t)a.len);
+    // window, one or two filters, and the slices' partial sums (at most 256 R
+    // per filter: 8 slices of the outputs that fill the workgroup)
+    const size_t filters = a.Hb ? 2 : 1;
+    const size_t smem = sizeof(float) * ((size_t)a.len + a.B + kTdPad + filters * ((size_t)a.len + 1024));
     // four outputs per lane once their waves cover the chip's 1,024 SIMDs, two below
     const long long waves4 = (long long)a.C * ((a.n + 255) / 256);
     if (waves4 >= 1024) hipExtLaunchKernelGGL((k_td<4>), dim3(a.C), dim3(256), smem, s, ev0, ev1, 0, a);
