@@ -3263,7 +3263,7 @@ static int32_t room_launch(tanx_ctx *ctx, uint32_t count, const tanx_room *rooms
     const size_t nears = 2 * (size_t)count;
     std::vector<RoomEar> ears(nears);
     long long max_early = 0;
-    int max_windows = 0;
+    int max_late = 0;
     for (uint32_t k = 0; k < count; k++) {
         long long images = 0;
         const int32_t rc = room_ears(&rooms[k], &sources[k], &listeners[k], fs, len, flags, max_bounces,
@@ -3274,9 +3274,10 @@ static int32_t room_launch(tanx_ctx *ctx, uint32_t count, const tanx_room *rooms
             long long box = 1;
             for (int a = 0; a < 3; a++) box *= E.hi[a] >= E.lo[a] ? (long long)(E.hi[a] - E.lo[a] + 1) : 0;
             max_early = std::max(max_early, box);
-            max_windows = std::max(max_windows, (len - E.wstart + kRoomWindow - 1) / kRoomWindow);
         }
     }
+    room_late_plan(ears.data(), nears, len);
+    for (const RoomEar &E : ears) max_late = std::max(max_late, E.late_total);
     const size_t ints = nears * (size_t)len;
     if (ints > ctx->room_acc_ints || nears > ctx->room_ears_cap) {
         // buffers in use by earlier calls on the stream: let them finish
@@ -3308,7 +3309,7 @@ static int32_t room_launch(tanx_ctx *ctx, uint32_t count, const tanx_room *rooms
                               hipMemcpyHostToDevice, ctx->proc));
     TANX_CHECK(hipEventRecord(ctx->room_ev, ctx->proc));
     ctx->room_ev_live = true;
-    TANX_CHECK(launch_room(ctx->room_ears_dev, (int)nears, max_early, max_windows, len, ctx->room_acc, d_out,
+    TANX_CHECK(launch_room(ctx->room_ears_dev, (int)nears, max_early, max_late, len, ctx->room_acc, d_out,
                            (long long)out_stride, ctx->proc));
     return TANX_OK;
 }

@@ -375,18 +375,23 @@ struct RoomEar {
     // head-filtered images): lo[k] .. hi[k] per axis
     int lo[3], hi[3];
     int wstart;        // first output sample summed by windows: min(hrtf_len, len)
+    // workgroups of the late windows: late_groups(E, w) for window w, in all
+    float late_scale;
+    int late_total;
 };
-constexpr int kRoomWindow = 2048;  // output samples per late-image window (8 KB of LDS)
+constexpr int kRoomWindow = 8192;  // output samples per late-image window (32 KB of LDS)
 // RoomEar of the left (out[0]) and right (out[1]) ear; AMF_RESULT value.
 int32_t room_ears(const tanx_room *room, const tanx_source *source, const tanx_listener *ears, int fs, int len,
                   uint32_t flags, int max_bounces, RoomEar out[2], long long *images);
+// Sets late_scale and late_total of one call's ears.
+void room_late_plan(RoomEar *ears, size_t nears, int len);
 // Sums the images of ears[e] (wrapping 32-bit integer sums of the
 // fixed-point contributions) into row e of out (out + e * out_stride, len
 // floats).  Early images go into acc[e * len ...] with global atomics, late
 // ones through per-window LDS sums added into acc; acc is left cleared.
-// max_early: the largest early-box image count over the ears; max_windows:
-// the largest number of late windows.
-hipError_t launch_room(const RoomEar *d_ears, int nears, long long max_early, int max_windows, int len,
+// max_early: the largest early-box image count over the ears; max_late: the
+// largest late_total.
+hipError_t launch_room(const RoomEar *d_ears, int nears, long long max_early, int max_late, int len,
                        unsigned *acc, float *out, long long out_stride, hipStream_t s);
 
 // Allocation-free group launches (tanx_group_process_device_noalloc): the

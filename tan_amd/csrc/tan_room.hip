@@ -176,6 +176,16 @@ __device__ __forceinline__ ImageParams image_params(const RoomEar &E)
     return p;
 }
 
+// d / 340, the IEEE quotient's bits (checked for every float from 2^-31 to
+// 2^37; the few below round to sample 0 either way): the quotient by the
+// rounded reciprocal, corrected by its remainder (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990).
+__device__ __forceinline__ float div340(float d)
+{
+    const float rc = 1.0f / 340.0f, q = d * rc;
+    return fmaf(fmaf(-340.0f, q, d), rc, q);
+}
+
 // Late images of one window of kRoomWindow output samples [w0, w0 +
 // kRoomWindow), w0 = wstart + window * kRoomWindow, and one slice of the
 // image lattice's rows (iy, iz): the images arriving in the window lie in a
@@ -185,41 +195,80 @@ __device__ __forceinline__ ImageParams image_params(const RoomEar &E)
 // candidate is then evaluated exactly), and adds the single-tap
 // contributions arriving in the window to an LDS sum.  The workgroup then
 // adds its nonzero sums to acc: one atomic per bin instead of one per image.
-constexpr int kPowTable = 512;  // damping powers 0..511 per wall in LDS
+//
+// Bound by instruction issue.  A window is as long as the LDS of three
+// workgroups per compute unit allows: a row's setup and its shell's
+// boundary cells are shared by more images (with 2,048 samples a run was
+// three cells of which half arrived outside the window), and what an image
+// needs from its ix alone (the squared x distance, the two x walls' powers)
+// is read from a table.  32 listeners (64 ears) of 65,536 taps: 0.54 ms, 1.59 ms
+// with 2,048-sample windows of equal slices and every factor from its ix.
+constexpr int kPowTable = 512;   // damping powers 0..511 per y and z wall in LDS
+constexpr int kCellTable = 512;  // cells ix of the x axis in LDS
+constexpr int kLateThreads = 512;
 
-__global__ void __launch_bounds__(256) k_room_late(const RoomEar *__restrict__ ears, unsigned *__restrict__ acc,
-                                                   int len, int slices)
+// Workgroups of one ear's window: its share of the images (the shell's volume
+// over the room's, late_scale), which grow with the square of the time, so that the outer
+// windows do not end long after the others; at least a row per thread.  The
+// same float steps on the host and the device.
+__host__ __device__ inline int late_groups(const RoomEar &E, int window)
+{
+    const float s0 = (float)(E.wstart + window * kRoomWindow), s1 = s0 + (float)kRoomWindow;
+    const float share = E.late_scale * (s1 * s1 * s1 - s0 * s0 * s0);
+    const long long rows = (long long)(2 * E.n[1] + 1) * (2 * E.n[2] + 1);
+    const int most = (int)(rows / kLateThreads < 1 ? 1 : rows / kLateThreads > 256 ? 256 : rows / kLateThreads);
+    const int want = share < 256.0f ? 1 + (int)share : 256;
+    return want < most ? want : most;
+}
+
+__global__ void __launch_bounds__(kLateThreads) k_room_late(const RoomEar *__restrict__ ears,
+                                                            unsigned *__restrict__ acc, int len)
 {
     __shared__ unsigned sum[kRoomWindow];
-    __shared__ float pw[6][kPowTable];  // pw[k][e] = ipow(damp[k], e): the same bits as ipow
+    __shared__ float pw[4][kPowTable];  // pw[k][e] = ipow(damp[k + 2], e): the same bits as ipow
+    __shared__ float2 cell[kCellTable];  // ix + n0: dx * dx and the two x walls' powers, as image_eval has them
     const RoomEar &E = ears[blockIdx.y];
-    const int window = (int)blockIdx.x / slices, slice = (int)blockIdx.x % slices;
+    if ((int)blockIdx.x >= E.late_total) return;  // uniform over the workgroup, as what follows
+    int window = 0, slice = (int)blockIdx.x, slices = late_groups(E, 0);
+    while (slice >= slices) {
+        slice -= slices;
+        slices = late_groups(E, ++window);
+    }
     const int w0 = E.wstart + window * kRoomWindow;
-    if (w0 >= len) return;  // uniform over the workgroup
     const int w1 = min(w0 + kRoomWindow, len);
     const ImageParams P = image_params(E);
     const int n0 = E.n[0], n1 = E.n[1], n2 = E.n[2];
+    const float W = P.dim[0], hx = P.head[0];
+    auto cell_of = [&](int ix) {
+        int rf, lf;
+        bounces(ix, rf, lf);
+        const float dx = image_pos(ix, W, P.src[0]) - hx;
+        return make_float2(dx * dx, ipow(P.damp[0], rf) * ipow(P.damp[1], lf));
+    };
     // reflection counts are at most n per axis
-    const bool tables = max(n0, max(n1, n2)) < kPowTable;
+    const bool tables = max(n1, n2) < kPowTable, cells = 2 * n0 + 1 <= kCellTable;
     for (int i = threadIdx.x; i < kRoomWindow; i += blockDim.x) sum[i] = 0u;
     if (tables) {
-        const int ne = max(n0, max(n1, n2)) + 1;
-        for (int i = threadIdx.x; i < 6 * ne; i += blockDim.x) pw[i / ne][i % ne] = ipow(P.damp[i / ne], i % ne);
+        const int ne = max(n1, n2) + 1;
+        for (int i = threadIdx.x; i < 4 * ne; i += blockDim.x) pw[i / ne][i % ne] = ipow(P.damp[i / ne + 2], i % ne);
     }
+    if (cells)
+        for (int i = threadIdx.x; i < 2 * n0 + 1; i += blockDim.x) cell[i] = cell_of(i - n0);
     __syncthreads();
-    auto power = [&](int k, int e) { return tables ? pw[k][e] : ipow(P.damp[k], e); };
+    auto power = [&](int k, int e) { return tables ? pw[k - 2][e] : ipow(P.damp[k], e); };
 
     const float m = 0.05f;
     const float dlo = fmaxf(0.0f, (float)(w0 - 1) * 340.0f / (float)P.fs - m);
     const float dhi = (float)w1 * 340.0f / (float)P.fs + m;
     const int wy = 2 * n1 + 1, rows = wy * (2 * n2 + 1);
-    const float W = P.dim[0], hx = P.head[0];
+    const float fs = (float)P.fs, gd = P.max_gain * P.d_min;
+    const int late0 = max(w0, P.hrtf_len), late1 = min(w1, P.len);
     for (int r = slice + slices * (int)threadIdx.x; r < rows; r += slices * (int)blockDim.x) {
         const int iy = r % wy - n1;
         const int iz = r / wy - n2;
         const float dy = image_pos(iy, P.dim[1], P.src[1]) - P.head[1];
         const float dz = image_pos(iz, P.dim[2], P.src[2]) - P.head[2];
-        const float D2 = dy * dy + dz * dz;
+        const float dy2 = dy * dy, dz2 = dz * dz, D2 = dy2 + dz2;
         if (D2 > dhi * dhi) continue;
         const float xh = sqrtf(fmaxf(0.0f, dhi * dhi - D2)) + m;
         const float xl = fmaxf(0.0f, sqrtf(fmaxf(0.0f, dlo * dlo - D2)) - m);
@@ -240,23 +289,19 @@ __global__ void __launch_bounds__(256) k_room_late(const RoomEar *__restrict__ e
         bounces(iy, tp, bt);
         bounces(iz, fr, bk);
         const float pT = power(2, tp), pB = power(3, bt), pF = power(4, fr), pK = power(5, bk);
-        for (int pass = 0; pass < 2; pass++) {
-            const int lo = pass ? b0 : a0, hi = pass ? b1 : a1;
-            for (int ix = lo; ix <= hi; ix++) {
-                if (P.suppress_direct && ix == 0 && iy == 0 && iz == 0) continue;
-                int rf, lf;
-                bounces(ix, rf, lf);
-                const float amp = power(0, rf) * power(1, lf) * pT * pB * pF * pK;
-                const float dx = image_pos(ix, W, P.src[0]) - hx;
-                const float d = sqrtf(dx * dx + dy * dy + dz * dz);
-                const int q = f2i_sat((d / 340.0f) * (float)P.fs);
-                // late (one tap): arrival 1 + q in [hrtf_len, len), and in the window
-                if (q < 0 || q >= P.len - 1) continue;
-                const int fi = q + 1;
-                if (fi < P.hrtf_len || fi < w0 || fi >= w1) continue;
-                const float dr = (d <= P.d_min) ? P.max_gain : P.max_gain * P.d_min / d;
-                atomicAdd(&sum[fi - w0], (unsigned)f2i_sat(kRoomFixedOne * amp * dr));
-            }
+        // both intervals in one loop: cell k is a0 + k, from na on b0 + k - na
+        const int na = max(0, a1 - a0 + 1), nc = na + max(0, b1 - b0 + 1), skip = b0 - a0 - na;
+        for (int k = 0; k < nc; k++) {
+            const int ix = a0 + k + (k < na ? 0 : skip);
+            const float2 cx = cells ? cell[ix + n0] : cell_of(ix);
+            const float d = sqrtf(cx.x + dy2 + dz2);
+            const int q = f2i_sat(div340(d) * fs);
+            // late (one tap): arrival 1 + q in [hrtf_len, len), and in the window
+            if (q < late0 - 1 || q >= late1 - 1) continue;
+            if (P.suppress_direct && ix == 0 && iy == 0 && iz == 0) continue;
+            const float amp = cx.y * pT * pB * pF * pK;
+            const float dr = (d <= P.d_min) ? P.max_gain : gd / d;
+            atomicAdd(&sum[q + 1 - w0], (unsigned)f2i_sat(kRoomFixedOne * amp * dr));
         }
     }
     __syncthreads();
@@ -380,23 +425,42 @@ int32_t room_ears(const tanx_room *room, const tanx_source *source, const tanx_l
     return TANX_OK;
 }
 
-hipError_t launch_room(const RoomEar *d_ears, int nears, long long max_early, int max_windows, int len,
+// Late images per workgroup: a 2,048th of all of the call's, between 4,096
+// (below, clearing and adding a window's sums outweighs them: 2 ears of
+// 65,536 taps 57 us, 79 us with 16,384) and 32,768 (above, the last
+// workgroups end late: 64 ears 535 us, 640 us with 8,192).
+void room_late_plan(RoomEar *ears, size_t nears, int len)
+{
+    auto images = [&](const RoomEar &E) {  // images within one sample's cube
+        const double step = 340.0 / (double)E.fs;
+        return 4.0 / 3.0 * 3.141592653589793 * step * step * step / ((double)E.dim[0] * E.dim[1] * E.dim[2]);
+    };
+    double all = 0.0;
+    for (size_t k = 0; k < nears; k++)
+        all += images(ears[k]) * ((double)len * len * len - (double)ears[k].wstart * ears[k].wstart * ears[k].wstart);
+    const double per = std::fmin(std::fmax(all / 2048.0, 4096.0), 32768.0);
+    for (size_t k = 0; k < nears; k++) {
+        RoomEar &E = ears[k];
+        E.late_scale = (float)(images(E) / per);
+        E.late_total = 0;
+        for (int w = 0; E.wstart + (long long)w * kRoomWindow < len; w++) E.late_total += late_groups(E, w);
+    }
+}
+
+hipError_t launch_room(const RoomEar *d_ears, int nears, long long max_early, int max_late, int len,
                        unsigned *acc, float *out, long long out_stride, hipStream_t s)
 {
     if (nears <= 0 || len <= 0) return hipSuccess;
     const long long blocks = (max_early + 255) / 256;
-    if (blocks > 0x7fffffffLL || nears > 65535 || max_windows < 0) return hipErrorInvalidValue;
+    if (blocks > 0x7fffffffLL || nears > 65535 || max_late < 0) return hipErrorInvalidValue;
     if (blocks > 0) {
         hipLaunchKernelGGL(k_room_early, dim3((unsigned)blocks, (unsigned)nears), dim3(256), 0, s, d_ears, acc, len);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    if (max_windows > 0) {
-        // row slices per window: about 2,048 workgroups in all, at most 32 slices
-        long long per = 2048LL / ((long long)max_windows * nears);
-        const int slices = (int)(per < 1 ? 1 : per > 32 ? 32 : per);
-        hipLaunchKernelGGL(k_room_late, dim3((unsigned)(max_windows * slices), (unsigned)nears), dim3(256), 0, s,
-                           d_ears, acc, len, slices);
+    if (max_late > 0) {
+        hipLaunchKernelGGL(k_room_late, dim3((unsigned)max_late, (unsigned)nears), dim3(kLateThreads), 0, s, d_ears,
+                           acc, len);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -145,3 +145,22 @@ def test_fft_row_layouts(gpu_ctx, log2m, C, pad, off, direction):
         ref, g, used = np.fft.irfft(z, n), got[:, :n], n
     assert np.abs(g - ref).max() <= 3e-7 * np.abs(ref).max() * log2n  # the bound of test_gpu_fft.py
     assert np.all(got[:, used:] == 9.0)
+
+
+# more cells along x than the table holds; more reflections along y or z than
+# the power tables hold; one window and several, ending inside one
+@pytest.mark.parametrize("dims,n", [((0.4, 30.0, 40.0), 17000), ((30.0, 0.2, 40.0), 16500), ((40.0, 30.0, 0.2), 9001),
+                                    ((3.0, 2.5, 4.0), 8193)])
+def test_room_tables_and_windows(gpu_ctx, dims, n):
+    import oracle_lib as O
+    from tan_amd import room as R
+    room = R.make_room(*dims, 0.8, damp_top=0.4)
+    src = R.MonoSource(*[0.3 * d for d in dims])
+    lst = R.make_listener(tuple(0.6 * d for d in dims), 0.16, 20.0)
+    left, right = np.zeros(n, np.float32), np.zeros(n, np.float32)
+    assert R.generateRoomResponse(gpu_ctx, room, src, lst, 48000, n, left, right) == T.AMF_OK
+    rc, oleft, oright = O.room_response(room, src, lst, 48000, n, 0, 0)
+    assert rc == 0
+    np.testing.assert_array_equal(left, oleft)
+    np.testing.assert_array_equal(right, oright)
+    assert np.count_nonzero(left) > 0
