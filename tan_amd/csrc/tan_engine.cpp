@@ -2353,8 +2353,12 @@ static int32_t group_run(tanx_ctx *ctx, int irtype, uint32_t n, tanx_conv *const
                 lo = mid;
             }
         }
-        // the staging pieces are copied in one transfer at their offsets
-        TANX_CHECK(hipMemcpyAsync(g.dev, g.host, g.total(), hipMemcpyHostToDevice, ctx->proc));
+        // the staging pieces are copied at their offsets, the frame pieces
+        // only when some object ends a frame (pinned staging by a kernel, the
+        // allocation-free call's pageable one by a transfer)
+        const size_t bytes = nframe > 0 ? g.total() : g.desc_bytes + g.start_bytes;
+        if (staged) TANX_CHECK(launch_fetch(g.host, g.dev, bytes, ctx->proc));
+        else TANX_CHECK(hipMemcpyAsync(g.dev, g.host, bytes, hipMemcpyHostToDevice, ctx->proc));
         if (staged) TANX_CHECK(hipEventRecord(staged, ctx->proc));
         hipEvent_t t0 = nullptr, t1 = nullptr;
         if (ctx->gtiming) {
@@ -2366,8 +2370,36 @@ static int32_t group_run(tanx_ctx *ctx, int irtype, uint32_t n, tanx_conv *const
             if (!ctx->q_next) TANX_CHECK(hipMalloc(&ctx->q_next, kKinds * kClasses * sizeof(int)));
             TANX_CHECK(launch_zero(ctx->q_next, align16((size_t)nl * sizeof(int)), ctx->proc));
         }
+        // heads-only launches of more than one block size become one, the last
+        HeadSets heads{};
+        int sets = 0;
+        for (int i = 0; i < nl; i++) sets += launches[i].roles == kRolesHeads;
+        const bool merge = sets > 1 && !queue;
+        if (merge) {
+            int end = 0, at = 0;
+            for (int k = 0, i = 0; k < kClasses; k++) {
+                // a class's heads launch is the last of its launches
+                while (i < nl && (launches[i].B < (64 << k) || (launches[i].B == (64 << k) && launches[i].roles != kRolesHeads))) i++;
+                if (i < nl && launches[i].B == (64 << k)) {
+                    heads.d[k] = reinterpret_cast<const TickArgs *>(g.dev) + launches[i].first;
+                    heads.st[k] = reinterpret_cast<const int *>(g.dev + g.desc_bytes) + launches[i].first;
+                    heads.n[k] = (int)launches[i].count;
+                    end += launches[i].total;
+                }
+                heads.end[k] = end;
+            }
+            for (int i = 0; i < nl; i++)
+                if (launches[i].roles != kRolesHeads) launches[at++] = launches[i];
+            launches[at] = Launch{};
+            launches[at].roles = kRolesHeads;
+            nl = at + 1;
+        }
         for (int i = 0; i < nl; i++) {
             const Launch &l = launches[i];
+            if (merge && l.roles == kRolesHeads) {
+                TANX_CHECK(launch_group_heads(irtype, heads, ctx->proc, i == 0 ? t0 : nullptr, t1));
+                continue;
+            }
             const TickArgs *dd = reinterpret_cast<const TickArgs *>(g.dev) + l.first;
             const int *ds = reinterpret_cast<const int *>(g.dev + g.desc_bytes) + l.first;
             // the first launch stamps the start event, the last one the end
@@ -2491,7 +2523,7 @@ extern "C" int32_t tanx_group_update_td_device(uint32_t n, tanx_conv *const *con
         }
         for (const Launch &l : launches)
             if (l.blocks > INT32_MAX) return TANX_INVALID_ARG;
-        TANX_CHECK(hipMemcpyAsync(ctx->g_dev, host, db + sb, hipMemcpyHostToDevice, ctx->proc));
+        TANX_CHECK(launch_fetch(host, ctx->g_dev, db + sb, ctx->proc));
         TANX_CHECK(hipEventRecord(ctx->g_ev[slot], ctx->proc));
         for (const Launch &l : launches)
             TANX_CHECK(launch_ir_transform_group(l.B, l.irtype, reinterpret_cast<const IrArgs *>(ctx->g_dev) + l.first,

@@ -246,6 +246,17 @@ hipError_t launch_ir_transform_group(int B, int irtype, const IrArgs *d_descs, c
 hipError_t launch_group_tick(int irtype, int B, int roles, int km, const TickArgs *d_descs, const int *d_starts,
                              int nobj, unsigned blocks, hipStream_t s, hipEvent_t ev0 = nullptr,
                              hipEvent_t ev1 = nullptr);
+// The heads-only launches of several block sizes (64 << k) as one launch: set
+// k's objects at d[k] with block offsets st[k], its workgroups before end[k]
+// (those of the sets before it included; an empty set ends where the one
+// before it does).
+struct HeadSets {
+    const TickArgs *d[4];
+    const int *st[4];
+    int n[4], end[4];
+};
+hipError_t launch_group_heads(int irtype, const HeadSets &h, hipStream_t s, hipEvent_t ev0 = nullptr,
+                              hipEvent_t ev1 = nullptr);
 // Work-queue form of launch_group_tick: `total` workgroup items taken in
 // order from *next (zero before the launch) by the device's resident
 // workgroups of the kernel.
@@ -352,6 +363,8 @@ hipError_t launch_convert(const void *in, long long in_step, long long in_off, i
                           long long out_step, long long out_off, int out_type, long long n, float gain, int *d_flag,
                           hipStream_t s);
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t s);
+// copies whole 16-byte pieces of pinned host memory (device-visible) into device memory
+hipError_t launch_fetch(const void *host, void *dev, size_t bytes, hipStream_t s);
 
 // Room responses by image sources (GenerateRoomResponse.cl).  One RoomEar
 // per response row: the kernel arguments the reference's host code derives

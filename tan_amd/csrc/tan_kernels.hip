@@ -1257,6 +1257,40 @@ __global__ __launch_bounds__(kTickThreads, 4) void k_group_heads(const TickArgs 
     head_block<M, HT, true>(a, b - starts[lo], sm);
 }
 
+// The heads of all block sizes in one launch.  At a few hundred channels a
+// heads-only launch is one chain of memory round trips and FFT stages long
+// (about 10 us) whatever its size, so three of them in a row cost three
+// chains: 4 ticks of 512 mono streams of three block sizes 247 to 200 us, of 60
+// streams 122 to 82 us.
+template <int HT, int K>
+__device__ __forceinline__ void head_set_block(const HeadSets &h, int b, float4 *smem)
+{
+    constexpr int M = 64 << K;
+    const int *starts = h.st[K];
+    int lo = 0, hi = h.n[K] - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (starts[mid] <= b) lo = mid;
+        else hi = mid - 1;
+    }
+    const TickArgs a = h.d[K][lo];
+    if (a.B != M) return;
+    head_block<M, HT, true>(a, b - starts[lo], reinterpret_cast<HeadSmem<M> *>(smem));
+}
+
+template <int HT>
+__global__ __launch_bounds__(kTickThreads, 4) void k_group_heads_all(HeadSets h)
+{
+    constexpr size_t kBytes = wave_heads(256) * sizeof(HeadSmem<256>) > sizeof(HeadSmem<512>)
+                                  ? wave_heads(256) * sizeof(HeadSmem<256>) : sizeof(HeadSmem<512>);
+    __shared__ float4 smem[kBytes / 16];
+    const int b = blockIdx.x;
+    if (b < h.end[0]) head_set_block<HT, 0>(h, b, smem);
+    else if (b < h.end[1]) head_set_block<HT, 1>(h, b - h.end[0], smem);
+    else if (b < h.end[2]) head_set_block<HT, 2>(h, b - h.end[1], smem);
+    else head_set_block<HT, 3>(h, b - h.end[2], smem);
+}
+
 // Work-queue form of a group launch: a grid of the device's resident
 // workgroups takes the launch's workgroup items [0, total) in order from
 // *next (zero before the launch) and runs each one as k_group_tick or, for
@@ -2986,6 +3020,13 @@ static hipError_t launch_call_pass(const CallArgs &a, hipStream_t s)
 }
 
 template <int HT>
+hipError_t launch_group_heads_t(const HeadSets &h, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
+{
+    hipExtLaunchKernelGGL((k_group_heads_all<HT>), dim3((unsigned)h.end[3]), dim3(kTickThreads), 0, s, ev0, ev1, 0, h);
+    return hipGetLastError();
+}
+
+template <int HT>
 hipError_t launch_call_pass_t(int B, const CallArgs &a, hipStream_t s)
 {
     TANX_SWITCH_B(B, return (launch_call_pass<HT, M>(a, s)));
@@ -3090,6 +3131,7 @@ hipError_t launch_group_frame_t(const FrameArgs *d_descs, const int *d_starts, i
     PRE template hipError_t launch_heads_t<HT>(int, const HeadBatchArgs &, hipStream_t, hipEvent_t, hipEvent_t);    \
     PRE template hipError_t launch_window_t<HT>(int, int, const HeadBatchArgs &, const TickArgs &, hipStream_t,     \
                                                 hipEvent_t, hipEvent_t);                                            \
+    PRE template hipError_t launch_group_heads_t<HT>(const HeadSets &, hipStream_t, hipEvent_t, hipEvent_t);        \
     PRE template hipError_t launch_call_pass_t<HT>(int, const CallArgs &, hipStream_t);                             \
     PRE template hipError_t launch_ir_transform_group_t<HT>(int, const IrArgs *, const int *, int, unsigned,        \
                                                             hipStream_t);                                           \
@@ -3108,6 +3150,27 @@ TANX_TYPED(, IR_BF16)
 #endif
 
 #if TANX_IN(0)
+// Pinned host memory to the device, read by the kernel itself: in stream
+// order like any launch, where a copy through the DMA engines left the stream
+// idle before and after it (512 mono streams, 4 ticks with 210 KB of descriptors
+// each: 315 to 247 us).
+__global__ __launch_bounds__(kTickThreads) void k_fetch(const float4 *__restrict__ src, float4 *__restrict__ dst, int n4)
+{
+    const int i = blockIdx.x * kTickThreads + threadIdx.x;
+    if (i < n4) dst[i] = src[i];
+}
+
+hipError_t launch_fetch(const void *host, void *dev, size_t bytes, hipStream_t s)
+{
+    if (bytes == 0) return hipSuccess;
+    if (bytes % 16 != 0 || bytes / 16 > 0x7fffffff || ((reinterpret_cast<uintptr_t>(host) | reinterpret_cast<uintptr_t>(dev)) & 15))
+        return hipErrorInvalidValue;
+    const int n4 = (int)(bytes / 16);
+    hipLaunchKernelGGL(k_fetch, dim3((unsigned)((n4 + kTickThreads - 1) / kTickThreads)), dim3(kTickThreads), 0, s,
+                       static_cast<const float4 *>(host), static_cast<float4 *>(dev), n4);
+    return hipGetLastError();
+}
+
 #ifdef TANX_PART
 TANX_TYPED(extern, IR_F32)
 TANX_TYPED(extern, IR_F16)
@@ -3195,6 +3258,17 @@ hipError_t launch_heads(int B, int irtype, const HeadBatchArgs &h, hipStream_t s
     }
 }
 
+
+hipError_t launch_group_heads(int irtype, const HeadSets &h, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
+{
+    if (h.end[3] <= 0) return hipSuccess;
+    switch (irtype) {
+    case IR_F32: return launch_group_heads_t<IR_F32>(h, s, ev0, ev1);
+    case IR_F16: return launch_group_heads_t<IR_F16>(h, s, ev0, ev1);
+    case IR_BF16: return launch_group_heads_t<IR_BF16>(h, s, ev0, ev1);
+    default: return hipErrorInvalidValue;
+    }
+}
 
 template <int M>
 static hipError_t launch_call_m(const CallArgs &a, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
