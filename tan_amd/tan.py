@@ -83,6 +83,14 @@ def _host_rows(arrs, channels, length=None, writable=False):
     """Row-pointer array for host float32 data: a 2-D array or a list of 1-D arrays.
 
     Returns (pointer array, keepalive list)."""
+    if (isinstance(arrs, np.ndarray) and arrs.ndim == 2 and arrs.dtype == np.float32 and arrs.strides[1] == 4
+            and 0 < channels <= arrs.shape[0]):
+        # rows of one array: their addresses at once (a row view and its pointer
+        # each cost about 2 us, 92 of 98 us per block at 23 channels of B = 128)
+        if length is not None and arrs.shape[1] < length:
+            raise ValueError("channel array shorter than the requested length")
+        at = arrs.ctypes.data + arrs.strides[0] * np.arange(channels, dtype=np.int64)
+        return (_f32p * channels).from_buffer(at), [arrs, at]
     if isinstance(arrs, np.ndarray) and arrs.ndim == 2:
         rows = [arrs[i] for i in range(arrs.shape[0])]
     else:
