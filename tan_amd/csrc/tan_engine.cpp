@@ -1657,6 +1657,107 @@ static int32_t process_call(tanx_conv *cv, const float *din, long long in_stride
     return TANX_OK;
 }
 
+// Least blocks process_call_nu's launches are worth: few channels are a chain
+// of launches a block at a time (4 blocks of 1 channel x 60,000 taps 22.3 to
+// 19.6 us, 5 of 3 channels x 20,000 32.0 to 23.1), many are bound by their
+// rows either way (4 blocks of 255 channels at B = 512: 91.6 against 92.8; 12
+// of 255 channels x 200,000 taps 221 to 185).
+static int nu_call_min(const tanx_conv *cv) { return cv->C <= 64 ? 4 : 6; }
+
+// Blocks a call of a non-uniform object may take together from here: within
+// one frame (a frame kernel runs after its last block), no switch under way,
+// and a spectrum and at least one partial-sum row per block in the tails'
+// place (4 maxchunk rows per channel).
+static int nu_call_blocks(const tanx_conv *cv)
+{
+    if (!cv->nu || cv->pending || cv->ready || cv->delayed) return 0;
+    const int left = cv->M - (int)((cv->ticks + (uint64_t)cv->nu_shift) % (uint64_t)cv->M);
+    return std::min(std::min(left, kPassMax), 2 * cv->maxchunk);
+}
+
+// The next n (<= nu_call_blocks) blocks of a device call of a non-uniform
+// object: the frame slices of the n blocks in one launch, the first frame's
+// taps as process_call's three, then the frame kernel if a frame ends.  A
+// block at a time is a launch each, bound by its chain of transforms: 16
+// blocks of 63 channels x 250,007 taps at B = 128 take 67 us, 138 before.
+static int32_t process_call_nu(tanx_conv *cv, const float *din, long long in_stride, float *dout, long long out_stride,
+                               int n)
+{
+    const size_t B = cv->B;
+    hipStream_t s = cv->ctx->proc;
+    CallArgs a{};
+    FrameSliceArgs f{};
+    FrameArgs fa;
+    bool frame_due = false;
+    uint64_t alg = 0;
+    const int lB = __builtin_ctz((unsigned)cv->B);
+    a.C = cv->C;
+    a.P = cv->P;
+    a.irtype = cv->irtype;
+    a.run = cv->drun;
+    a.twM = tw_table(cv->ctx->tw, lB);
+    a.twN = tw_table(cv->ctx->tw, lB + 1);
+    a.fdl = cv->F;
+    a.slot = cv->pos;
+    a.xin = din;
+    a.in_stride = in_stride;
+    a.yout = dout;
+    a.out_stride = out_stride;
+    a.xprev = cv->xprev;
+    a.n = a.xb = n;
+    a.HA = cv->slot_ptr(cv->cur);
+    a.SA = cv->scale_ptr(cv->cur);
+    for (int j = 0; j < n; j++) {
+        int nrun = 0;
+        int32_t rc = channel_flags(cv, nullptr, B, &nrun);
+        if (rc == TANX_OK && j == 0) rc = sync_run_mask(cv);
+        if (rc != TANX_OK) return rc;
+        TickArgs t = tick_common(cv);
+        cv->pos = (cv->pos + 1) % cv->P;
+        cv->crossfading = false;
+        cv->last_xfade = false;
+        nu_block_args(cv, cv->ticks, false, t, fa, &frame_due);
+        if (j == 0) {
+            a.zA = t.zA ? t.zA + t.zoff : nullptr;
+            a.zstride = t.N;
+            a.xring = t.xring;
+            a.xslot = t.xslot;
+            a.xmask = 2 * t.M - 1;
+            f.a = t;
+        }
+        f.fbase[j] = t.fbase;
+        f.bslice[j] = t.bslice;
+        f.out[j] = t.bTa;
+        alg += head_bytes(cv, 1) + frame_mac_bytes(cv, 1);
+        cv->ticks++;
+        cv->tail_due = true;
+        tail_done(cv);
+    }
+    cv->deferred = true;
+    f.n = n;
+    int chunks = std::max(1, std::min((512 + cv->C - 1) / cv->C, cv->P / 8));
+    chunks = std::max(1, std::min(chunks, (4 * cv->maxchunk - n) / n));
+    a.pc = (cv->P + chunks - 1) / chunks;
+    a.nchunk = (cv->P + a.pc - 1) / a.pc;
+    a.cached = a.pc <= 64;
+    a.X = cv->T;
+    a.T = cv->T + (size_t)cv->C * n * B;
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (cv->timing) TANX_CHECK(cv->t_head.acquire(&e0, &e1));
+    if (f.a.nchB > 0) TANX_CHECK(launch_frame_slices(cv->B, f, s));
+    TANX_CHECK(launch_call(cv->B, a, s, e0, frame_due ? nullptr : e1));
+    if (frame_due) {
+        TANX_CHECK(launch_frame(cv->irtype, fa, s, e1));
+        alg += frame_kernel_bytes(cv, 1);
+    }
+    if (cv->timing) {
+        cv->t_head.commit();
+        cv->head_alg_bytes += alg;
+        cv->timed_blocks += (uint64_t)n;
+    }
+    return TANX_OK;
+}
+
 // Computes the sums process_call left: of the blocks ticks .. covered with
 // the filters they use now (the switch state that of their scheduling), from
 // the rows before their origin.  Blocks of one filter share their origin.
@@ -1664,6 +1765,15 @@ static int32_t ensure_sums(tanx_conv *cv)
 {
     if (!cv->deferred) return TANX_OK;
     cv->deferred = false;
+    if (cv->kp <= 1) {
+        // a non-uniform object's tail for its next block, into the buffer that
+        // the next head reads
+        TickArgs a = tick_common(cv);
+        cv->tread ^= 1;
+        const int nf = fill_tail(cv, a);
+        cv->tread ^= 1;
+        return launch_timed(cv, cv->t_tail, nf, a, tail_bytes(cv, nf), cv->tail_alg_bytes);
+    }
     const long long e = (long long)cv->ticks, c = cv->covered;
     const long long sw = cv->delayed && (long long)cv->switch_at >= e && (long long)cv->switch_at <= c
                              ? (long long)cv->switch_at : c + 1;
@@ -1866,6 +1976,17 @@ extern "C" int32_t tanx_conv_process_device(tanx_conv *cv, const float *d_in, si
         schedule_queued(cv, &queued);
     }
     for (; b < nb; b++) {
+        if (fuse && cv->nu && !flags) {
+            const int take = (int)std::min<size_t>(nb - b, (size_t)nu_call_blocks(cv));
+            if (take >= nu_call_min(cv)) {
+                const int32_t rc = process_call_nu(cv, d_in + b * B, (long long)in_stride, d_out + b * B,
+                                                   (long long)out_stride, take);
+                if (rc != TANX_OK) return rc;
+                b += (size_t)take - 1;
+                if (processed) *processed = (b + 1) * B;
+                continue;
+            }
+        }
         int32_t rc = (fuse && cv->kp > 1)
                          ? process_block_kp(cv, d_in + b * B, (long long)in_stride, d_out + b * B,
                                             (long long)out_stride, B, flags, hq)

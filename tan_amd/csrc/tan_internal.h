@@ -336,7 +336,23 @@ struct CallArgs {
     int xb;                // block (of the n) that crossfades, n without one
     int nchunk, pc;        // partition chunks per channel and partitions per chunk
     int cached;            // nonzero: the sweep reads the rows with ordinary loads
+    // non-uniform objects: frame output added to block k's samples (channel c
+    // at zA + c * zstride + k * B, or nullptr), and the input ring (or
+    // nullptr): block w + k into slot (xslot + k) & xmask
+    const float *zA;
+    int zstride;
+    float *xring;
+    int xslot, xmask;
 };
+// Frame multiply-accumulate slices of consecutive blocks (their TickArgs'
+// frame roles, one filter) in one launch.
+struct FrameSliceArgs {
+    TickArgs a;            // the object's fields and the filter
+    int n;
+    int fbase[kPassMax], bslice[kPassMax];
+    float2 *out[kPassMax];
+};
+hipError_t launch_frame_slices(int B, const FrameSliceArgs &f, hipStream_t s);
 hipError_t launch_call(int B, const CallArgs &a, hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 // k_tick reading its arguments from d_descs[k] (graph replay; kn must be 1)
 hipError_t launch_tick_desc(int B, int irtype, const TickArgs *d_descs, int k, unsigned blocks, hipStream_t s);

@@ -1097,14 +1097,15 @@ __device__ void tail_role(const TickArgs &a, int c, int j, float4 *red)
 // Frame multiply-accumulate of a non-uniform object: bin slice a.bslice of
 // frame partitions [2 + k*pcB, 2 + (k+1)*pcB) for channel c.
 template <int M, int NF, int HT>
-__device__ void frame_mac_role(const TickArgs &a, int c, int k, float4 *red)
+__device__ void frame_mac_role(const TickArgs &a, int c, int k, int fbase, int bslice, float2 *outA, float2 *outB,
+                               float4 *red)
 {
     const size_t rowB = (size_t)a.N * IrRow<HT>::kBytes;
-    const size_t off = (size_t)a.bslice * M;  // complex elements
+    const size_t off = (size_t)bslice * M;  // complex elements
     MacView w;
     w.F = reinterpret_cast<const float4 *>(a.fb + (size_t)c * a.RB * a.N + off);
     w.fstride = a.N / 2;
-    w.base = a.fbase;
+    w.base = fbase;
     w.mask = a.RB - 1;
     w.HA = reinterpret_cast<const char *>(a.bHa) + (size_t)c * a.PB * rowB + off * IrRow<HT>::kBytes;
     w.HB = NF == 2 ? reinterpret_cast<const char *>(a.bHb) + (size_t)c * a.PB * rowB + off * IrRow<HT>::kBytes
@@ -1114,9 +1115,9 @@ __device__ void frame_mac_role(const TickArgs &a, int c, int k, float4 *red)
     w.SB = (HT == IR_F32 || NF == 1) ? nullptr : a.bSb + (size_t)c * a.PB;
     w.i0 = 2 + k * a.pcB;
     w.i1 = min(a.PB, w.i0 + a.pcB);
-    w.dc = a.bslice == 0;
-    w.TA = reinterpret_cast<float4 *>(a.bTa + ((size_t)c * a.nchB + k) * a.N + off);
-    w.TB = NF == 2 ? reinterpret_cast<float4 *>(a.bTb + ((size_t)c * a.nchB + k) * a.N + off) : nullptr;
+    w.dc = bslice == 0;
+    w.TA = reinterpret_cast<float4 *>(outA + ((size_t)c * a.nchB + k) * a.N + off);
+    w.TB = NF == 2 ? reinterpret_cast<float4 *>(outB + ((size_t)c * a.nchB + k) * a.N + off) : nullptr;
     mac_rows<M, NF, HT>(w, red);
 }
 
@@ -1127,8 +1128,20 @@ __device__ __forceinline__ void frame_mac_block(const TickArgs &a, int t, float4
     if (t >= a.C * a.nchB) return;
     const int c = t / a.nchB, k = t % a.nchB;
     if (!a.run[c]) return;
-    if (a.bHb) frame_mac_role<M, 2, HT>(a, c, k, smem);
-    else frame_mac_role<M, 1, HT>(a, c, k, smem);
+    if (a.bHb) frame_mac_role<M, 2, HT>(a, c, k, a.fbase, a.bslice, a.bTa, a.bTb, smem);
+    else frame_mac_role<M, 1, HT>(a, c, k, a.fbase, a.bslice, a.bTa, a.bTb, smem);
+}
+
+// The slices of n blocks: they read frames completed before the first of
+// them, so they need not wait for one another's blocks.
+template <int M, int HT>
+__global__ __launch_bounds__(kTickThreads) void k_frame_slices(FrameSliceArgs f)
+{
+    __shared__ float4 smem[tail_red_float4<M>()];
+    const int per = f.a.C * f.a.nchB, j = blockIdx.x / per, t = blockIdx.x - j * per;
+    const int c = t / f.a.nchB, k = t - c * f.a.nchB;
+    if (!f.a.run[c]) return;
+    frame_mac_role<M, 1, HT>(f.a, c, k, f.fbase[j], f.bslice[j], f.out[j], nullptr, smem);
 }
 
 // TK: 0 = a launch without tail blocks (head and frame roles only),
@@ -1644,7 +1657,11 @@ __global__ __launch_bounds__(kTickThreads) void k_call_out(CallArgs a)
                 // second half of the 2M output samples
                 const float2 v = z[M / 2 + n];
                 const float y0 = v.x * kScale, y1 = v.y * kScale;
-                if (f == 0) {
+                if (f == 0 && a.zA) {
+                    // (non-uniform objects: no crossfade in a call)
+                    const float *z0 = a.zA + (size_t)c * a.zstride + (size_t)k * M + 2 * n;
+                    y[q] = make_float2(fmaf(v.x, kScale, z0[0]), fmaf(v.y, kScale, z0[1]));
+                } else if (f == 0) {
                     y[q] = make_float2(y0, y1);
                 } else {
                     const int j0 = 2 * n, j1 = 2 * n + 1;
@@ -1670,9 +1687,12 @@ __global__ __launch_bounds__(kTickThreads) void k_call_out(CallArgs a)
     float2 *to = a.fdl + ((size_t)c * a.P + ((a.slot + k) & (a.P - 1))) * M;
 #pragma unroll
     for (int q = 0; q < KPT; q++) to[tid + q * NT] = row[tid + q * NT];
-    if (k == a.n - 1) {
-        const float *last = a.xin + (size_t)c * a.in_stride + (size_t)k * M;
-        for (int m = tid; m < M; m += NT) a.xprev[(size_t)c * M + m] = last[m];
+    const float *xi = a.xin + (size_t)c * a.in_stride + (size_t)k * M;
+    if (k == a.n - 1)
+        for (int m = tid; m < M; m += NT) a.xprev[(size_t)c * M + m] = xi[m];
+    if (a.xring) {
+        float *xr = a.xring + ((size_t)c * (a.xmask + 1) + ((a.xslot + k) & a.xmask)) * M;
+        for (int m = tid; m < M; m += NT) xr[m] = xi[m];
     }
 }
 
@@ -3033,6 +3053,14 @@ hipError_t launch_call_pass_t(int B, const CallArgs &a, hipStream_t s)
     return hipErrorInvalidValue;
 }
 
+template <int HT>
+hipError_t launch_frame_slices_t(int B, const FrameSliceArgs &f, hipStream_t s)
+{
+    const dim3 g((unsigned)(f.n * f.a.C * f.a.nchB)), t(kTickThreads);
+    TANX_SWITCH_B(B, hipLaunchKernelGGL((k_frame_slices<M, HT>), g, t, 0, s, f));
+    return hipGetLastError();
+}
+
 // partition sizes of uniform blocks (64..1024) and of frames (128..4096)
 #define TANX_SWITCH_PART(B, CALL)                        \
     switch (B) {                                         \
@@ -3131,6 +3159,7 @@ hipError_t launch_group_frame_t(const FrameArgs *d_descs, const int *d_starts, i
     PRE template hipError_t launch_heads_t<HT>(int, const HeadBatchArgs &, hipStream_t, hipEvent_t, hipEvent_t);    \
     PRE template hipError_t launch_window_t<HT>(int, int, const HeadBatchArgs &, const TickArgs &, hipStream_t,     \
                                                 hipEvent_t, hipEvent_t);                                            \
+    PRE template hipError_t launch_frame_slices_t<HT>(int, const FrameSliceArgs &, hipStream_t);                    \
     PRE template hipError_t launch_group_heads_t<HT>(const HeadSets &, hipStream_t, hipEvent_t, hipEvent_t);        \
     PRE template hipError_t launch_call_pass_t<HT>(int, const CallArgs &, hipStream_t);                             \
     PRE template hipError_t launch_ir_transform_group_t<HT>(int, const IrArgs *, const int *, int, unsigned,        \
@@ -3266,6 +3295,17 @@ hipError_t launch_group_heads(int irtype, const HeadSets &h, hipStream_t s, hipE
     case IR_F32: return launch_group_heads_t<IR_F32>(h, s, ev0, ev1);
     case IR_F16: return launch_group_heads_t<IR_F16>(h, s, ev0, ev1);
     case IR_BF16: return launch_group_heads_t<IR_BF16>(h, s, ev0, ev1);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launch_frame_slices(int B, const FrameSliceArgs &f, hipStream_t s)
+{
+    if (f.n < 1 || f.n > kPassMax || f.a.C < 1 || f.a.nchB < 1) return hipErrorInvalidValue;
+    switch (f.a.irtype) {
+    case IR_F32: return launch_frame_slices_t<IR_F32>(B, f, s);
+    case IR_F16: return launch_frame_slices_t<IR_F16>(B, f, s);
+    case IR_BF16: return launch_frame_slices_t<IR_BF16>(B, f, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -164,3 +164,35 @@ def test_room_tables_and_windows(gpu_ctx, dims, n):
     np.testing.assert_array_equal(left, oleft)
     np.testing.assert_array_equal(right, oright)
     assert np.count_nonzero(left) > 0
+
+
+# frames of 16, 8 and 64 blocks, a shifted frame clock, one tail chunk, 16-bit rows
+@pytest.mark.parametrize("L,B,mult,phase,precision,chunks", [(16384, 64, 16, 0, 0, 0), (20000, 128, 8, 3, 0, 0),
+                                                             (9000, 64, 64, 5, 1, 1), (40000, 256, 16, 0, 2, 0),
+                                                             (250007, 128, 0, 0, 0, 0), (30000, 1024, 4, 1, 0, 0)])
+def test_nonuniform_calls_of_many_blocks(gpu_ctx, L, B, mult, phase, precision, chunks):
+    """Calls that cross frame ends and switches equal one block per call (the
+    sums of a block are added in another order)."""
+    import torch
+    calls = [1, 20, 5, 3, 40, 16, 1, 1, 33, 4, 7, 64, 2, 50]
+    C, nb = 3, sum(calls)
+    starts = np.cumsum([0] + calls)
+    ups = {int(starts[i]): T.signals.ir_bank(C, L, k, base_seed=61) for k, i in enumerate((0, 4, 8, 11))}
+    x = torch.from_numpy(T.signals.input_bank(C, nb * B, base_seed=70)).cuda()
+    ys = []
+    for sizes in (calls, [1] * nb):
+        conv = T.TANConvolution(gpu_ctx, ir_precision=precision, nu_multiple=mult, nu_phase=phase,
+                                max_tail_chunks=chunks)
+        assert conv.InitGpu(T.TAN_CONVOLUTION_METHOD_FFT_PARTITIONED_NONUNIFORM, L, B, C) == T.AMF_OK
+        y, t = torch.zeros_like(x), 0
+        for n in sizes:
+            if t in ups:
+                assert conv.UpdateResponseTD(ups[t], L) == T.AMF_OK
+            rc, done = conv.Process(x[:, t * B:(t + n) * B], y[:, t * B:(t + n) * B])
+            assert rc == T.AMF_OK and done == n * B
+            t += n
+        conv.Synchronize()
+        conv.Terminate()
+        ys.append(y.cpu().numpy())
+    assert np.abs(ys[1]).max() > 1.0
+    assert np.abs(ys[0].astype(np.float64) - ys[1]).max() <= 2e-6  # outputs up to 3, as in test_gpu_passes.py
