@@ -1975,6 +1975,12 @@ extern "C" int32_t tanx_conv_process_device(tanx_conv *cv, const float *d_in, si
         }
         schedule_queued(cv, &queued);
     }
+    auto finish = [&](int32_t rc) {
+        // a long call also computes the sums of the blocks after it (one sweep
+        // beside its four or more), a short one leaves them to a call that
+        // needs them: calls of several blocks in a row use none
+        return rc == TANX_OK && nb >= 4 * (size_t)kPassMax ? ensure_sums(cv) : rc;
+    };
     for (; b < nb; b++) {
         if (fuse && cv->nu && !flags) {
             const int take = (int)std::min<size_t>(nb - b, (size_t)nu_call_blocks(cv));
@@ -1999,7 +2005,7 @@ extern "C" int32_t tanx_conv_process_device(tanx_conv *cv, const float *d_in, si
         }
         if (processed) *processed = (b + 1) * B;
     }
-    return flush_heads(cv, hq);
+    return finish(flush_heads(cv, hq));
 }
 
 /* ProcessDirect (ConvolutionImpl.cpp:719-762): time-domain objects only.
