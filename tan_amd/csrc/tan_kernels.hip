@@ -1540,6 +1540,8 @@ __global__ __launch_bounds__(kTickThreads) void k_window(HeadBatchArgs h, TickAr
 // block.  With every input block at hand the transforms are independent
 // (one wave each up to B = 256, C * n of them), the sweep reads each IR and
 // FDL row once for all n outputs, and only three launches follow each other.
+// Every input sample is read before the last launch, the only one that writes
+// outputs: the caller's output may be its input.
 // Calls of 16 blocks, 64 channels x 65,536 taps at B = 256: 28 us, 89 us a
 // launch per four blocks; 8 blocks of 1,024 channels x 131,072 taps with FP16
 // rows: 304 us (5.3 TB/s of rows), 577 us with two sweeps; 4 blocks of 1,024
@@ -1563,6 +1565,10 @@ __global__ __launch_bounds__(kTickThreads) void k_call_spectra(CallArgs a)
             const float *src = m < M / 2 ? prev + 2 * m : cur + 2 * (m - M / 2);
             s0[w][m] = make_float2(src[0], src[1]);
         }
+        if (a.xring) {
+            float *xr = a.xring + ((size_t)c * (a.xmask + 1) + ((a.xslot + j) & a.xmask)) * M;
+            for (int m = tid; m < M; m += NT) xr[m] = cur[m];
+        }
     }
     __syncthreads();
     if (!active) return;
@@ -1581,6 +1587,13 @@ __global__ __launch_bounds__(kTickThreads) void k_call_pass(CallArgs a)
     __shared__ float4 red[pass_red_float4<M, NF, HT, KM>()];
     const int c = blockIdx.x / a.nchunk, j = blockIdx.x - c * a.nchunk;
     if (!a.run[c]) return;
+    // the last block's input is the next call's previous one: kept here, after
+    // k_call_spectra has read the one before the call and before k_call_out
+    // writes outputs, which may lie over the inputs
+    if (j == 0) {
+        const float *last = a.xin + (size_t)c * a.in_stride + (size_t)(a.n - 1) * M;
+        for (int m = threadIdx.x; m < M; m += kTickThreads) a.xprev[(size_t)c * M + m] = last[m];
+    }
     const float *SA = HT == IR_F32 ? nullptr : a.SA + (size_t)c * a.P;
     const float *SB = (HT == IR_F32 || NF == 1) ? nullptr : a.SB + (size_t)c * a.P;
     const int i0 = j * a.pc, i1 = min(a.P, i0 + a.pc);
@@ -1681,19 +1694,11 @@ __global__ __launch_bounds__(kTickThreads) void k_call_out(CallArgs a)
             yo[2 * n + 1] = y[q].y;
         }
     }
-    // the block's spectrum enters the delay line, the last block's input is
-    // the next call's previous one
+    // the block's spectrum enters the delay line
     const float2 *row = a.X + (size_t)item * M;
     float2 *to = a.fdl + ((size_t)c * a.P + ((a.slot + k) & (a.P - 1))) * M;
 #pragma unroll
     for (int q = 0; q < KPT; q++) to[tid + q * NT] = row[tid + q * NT];
-    const float *xi = a.xin + (size_t)c * a.in_stride + (size_t)k * M;
-    if (k == a.n - 1)
-        for (int m = tid; m < M; m += NT) a.xprev[(size_t)c * M + m] = xi[m];
-    if (a.xring) {
-        float *xr = a.xring + ((size_t)c * (a.xmask + 1) + ((a.xslot + k) & a.xmask)) * M;
-        for (int m = tid; m < M; m += NT) xr[m] = xi[m];
-    }
 }
 
 // ---------------------------------------------------------------------------

@@ -1,0 +1,51 @@
+"""Device calls of several blocks: buffers, shapes and orders of calls at which
+the call path and the paths for single blocks have to agree."""
+import numpy as np
+import pytest
+
+import tan_amd as T
+
+pytestmark = pytest.mark.gpu
+UNIFORM = T.TAN_CONVOLUTION_METHOD_FFT_UNIFORM_PARTITIONED
+NONUNIFORM = T.TAN_CONVOLUTION_METHOD_FFT_PARTITIONED_NONUNIFORM
+
+
+def _run(conv, x, y, calls, B, before=None):
+    """Calls of the given lengths on conv (x is y: in place); before: call ->
+    function of the object run before it."""
+    t = 0
+    for i, n in enumerate(calls):
+        if before and i in before:
+            before[i](conv)
+        rc, done = conv.Process(x[:, t * B:(t + n) * B], y[:, t * B:(t + n) * B])
+        assert rc == T.AMF_OK and done == n * B
+        t += n
+    conv.Synchronize()
+    return y.cpu().numpy()
+
+
+def _update(h):
+    def issue(conv):
+        assert conv.UpdateResponseTD(h, h.shape[1]) == T.AMF_OK
+    return issue
+
+
+# waves and whole workgroups per block, a ring of frames, several launches per call
+@pytest.mark.parametrize("method,L,B", [(UNIFORM, 4096, 64), (UNIFORM, 65536, 512), (NONUNIFORM, 16384, 64),
+                                        (NONUNIFORM, 65536, 1024)])
+def test_in_place(gpu_ctx, method, L, B):
+    """Calls whose output is their input's buffer give what separate buffers do."""
+    import torch
+    calls = [4, 8, 1, 8, 40, 3, 16, 2, 24]
+    C, nb = 5, sum(calls)
+    x = torch.from_numpy(T.signals.input_bank(C, nb * B, base_seed=11)).cuda()
+    before = {i: _update(T.signals.ir_bank(C, L, k, base_seed=12)) for k, i in enumerate((0, 3, 6))}
+    ys = []
+    for same in (False, True):
+        conv = T.TANConvolution(gpu_ctx)
+        assert conv.InitGpu(method, L, B, C) == T.AMF_OK
+        xd = x.clone()
+        ys.append(_run(conv, xd, xd if same else torch.zeros_like(xd), calls, B, before))
+        conv.Terminate()
+    assert np.abs(ys[0]).max() > 0.1
+    np.testing.assert_array_equal(ys[0], ys[1])
