@@ -2627,9 +2627,10 @@ __global__ __launch_bounds__(256) void k_td(TdArgs a)
             yo[j] = ya;
         }
     }
-    // the new samples enter the history (this workgroup alone owns channel c)
+    // the new samples enter the history (this workgroup alone owns channel c),
+    // from the window: the output may lie over the input
     float *hw = a.hist + (size_t)c * len;
-    for (int j = tid; j < n; j += nt) hw[(a.pos + j) & mask] = xi[j];
+    for (int j = tid; j < n; j += nt) hw[(a.pos + j) & mask] = w[len - 1 + j];
 }
 
 __global__ void k_td_load(const float *__restrict__ ir, long long stride, long long n, const int *__restrict__ chan,

@@ -8,6 +8,7 @@ import tan_amd as T
 pytestmark = pytest.mark.gpu
 UNIFORM = T.TAN_CONVOLUTION_METHOD_FFT_UNIFORM_PARTITIONED
 NONUNIFORM = T.TAN_CONVOLUTION_METHOD_FFT_PARTITIONED_NONUNIFORM
+TIME_DOMAIN = T.TAN_CONVOLUTION_METHOD_TIME_DOMAIN
 
 
 def _run(conv, x, y, calls, B, before=None):
@@ -32,7 +33,7 @@ def _update(h):
 
 # waves and whole workgroups per block, a ring of frames, several launches per call
 @pytest.mark.parametrize("method,L,B", [(UNIFORM, 4096, 64), (UNIFORM, 65536, 512), (NONUNIFORM, 16384, 64),
-                                        (NONUNIFORM, 65536, 1024)])
+                                        (NONUNIFORM, 65536, 1024), (TIME_DOMAIN, 500, 128)])
 def test_in_place(gpu_ctx, method, L, B):
     """Calls whose output is their input's buffer give what separate buffers do."""
     import torch

@@ -17,6 +17,6 @@ def _run(name, guard="start", fill="0xff", timeout=600, **kw):
     assert p.returncode == 0, (p.returncode, p.stdout[-2000:], p.stderr[-2000:])
 
 
-@pytest.mark.parametrize("method", [0, 1], ids=["uniform", "nonuniform"])
+@pytest.mark.parametrize("method", [0, 1, 2], ids=["uniform", "nonuniform", "time"])
 def test_in_place(sim_built, method):  # noqa: F811
     _run("in_place", method=method)
