@@ -1536,8 +1536,12 @@ static int32_t process_block_kp(tanx_conv *cv, const float *din, long long in_st
 
 // Blocks one CallArgs launch of this object may take: its spectra and partial
 // sums are kept where the passes keep theirs (4 kp maxchunk rows per
-// channel), of which n + (n + 1) * chunks rows per channel are used.
-static int call_blocks_max(const tanx_conv *cv) { return std::min(kPassMax, (4 * cv->kp * cv->maxchunk - 1) / 2); }
+// channel), of which n + (n + 1) * chunks rows per channel are used, and each
+// block has a row of its own in the delay line.
+static int call_blocks_max(const tanx_conv *cv)
+{
+    return std::min(std::min(kPassMax, cv->P), (4 * cv->kp * cv->maxchunk - 1) / 2);
+}
 
 // Least blocks of a device call that take process_call's three launches.  Few
 // blocks of a small object are two launches of batched heads (5 blocks of 3

@@ -62,6 +62,33 @@ def in_place(method=0, L=4096, B=64, C=3):
     assert np.array_equal(ys[0], ys[1])
 
 
+def few_partitions(P=4, kp=8, B=64, C=2):
+    """Objects with fewer partitions than their calls have blocks, a response
+    issued before some calls: as one block per call."""
+    calls = [5, 24, 1, 16, 8, 33, 4, 7]
+    nb, ups = sum(calls), {0: 0, 3: 1, 5: 2}
+    x = T.signals.input_bank(C, nb * B, base_seed=21)
+    irs = [T.signals.ir_bank(C, P * B, k, base_seed=22) for k in range(len(ups))]
+    at = dict(zip(np.cumsum([0] + calls), range(len(calls) + 1)))
+    ctx = T.TANContext(device=0)
+    ys = []
+    for sizes in (calls, [1] * nb):
+        conv = T.TANConvolution(ctx, pass_blocks=kp)
+        assert conv.InitGpu(UNIFORM, P * B, B, C) == T.AMF_OK
+        assert conv.Info()["partitions"] == P
+        xd, yd = simlib.Dev(C, nb * B, x), simlib.Dev(C, nb * B, 0.0)
+        t = 0
+        for n in sizes:
+            if at.get(t) in ups:
+                update(conv, irs[ups[at[t]]])
+            call(conv, xd, yd, t, n, B)
+            t += n
+        ys.append(yd.a.copy())
+    err = float(np.abs(ys[0].astype(np.float64) - ys[1]).max())
+    print(f"P={P} K={kp}: calls vs one block per call {err:.3e}", flush=True)
+    assert np.abs(ys[1]).max() > 0.1 and err <= 2e-6  # outputs up to 3, as in test_gpu_passes.py
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]](**{k: int(v) for k, v in (a.split("=") for a in sys.argv[2:])})
     print("scenario complete", flush=True)

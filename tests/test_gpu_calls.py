@@ -50,3 +50,23 @@ def test_in_place(gpu_ctx, method, L, B):
         conv.Terminate()
     assert np.abs(ys[0]).max() > 0.1
     np.testing.assert_array_equal(ys[0], ys[1])
+
+
+@pytest.mark.parametrize("P,kp,B", [(1, 4, 64), (2, 4, 64), (4, 16, 64), (8, 4, 128), (4, 4, 1024), (8, 12, 512)])
+def test_few_partitions(gpu_ctx, P, kp, B):
+    """Objects with fewer partitions than their calls have blocks, a response
+    issued before some calls: as one block per call."""
+    import torch
+    calls = [5, 24, 1, 16, 8, 33, 4, 7]
+    C, nb = 3, sum(calls)
+    starts = np.cumsum([0] + calls)
+    x = torch.from_numpy(T.signals.input_bank(C, nb * B, base_seed=21)).cuda()
+    ups = {i: _update(T.signals.ir_bank(C, P * B, k, base_seed=22)) for k, i in enumerate((0, 3, 5))}
+    ys = []
+    for sizes, before in ((calls, ups), ([1] * nb, {int(starts[i]): u for i, u in ups.items()})):
+        conv = T.TANConvolution(gpu_ctx, pass_blocks=kp)
+        assert conv.InitGpu(UNIFORM, P * B, B, C) == T.AMF_OK
+        ys.append(_run(conv, x, torch.zeros_like(x), sizes, B, before))
+        conv.Terminate()
+    assert np.abs(ys[1]).max() > 0.1
+    assert np.abs(ys[0].astype(np.float64) - ys[1]).max() <= 2e-6  # outputs up to 3, as in test_gpu_passes.py
