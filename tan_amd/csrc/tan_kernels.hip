@@ -1468,7 +1468,8 @@ __device__ void heads_role(const HeadBatchArgs &h, int c, HeadsSmem<M> &sm)
         const int j = e >> LM, k = e & (M - 1);
         const float2 X = r2c_post<M>(Z + j * M, k, sm.twn);
         sm.x[j][k] = X;
-        h.fdl[((size_t)c * h.P + h.slot[j]) * M + k] = X;
+        // with fewer rows than blocks, a row takes its last block's
+        if (j + h.P >= n) h.fdl[((size_t)c * h.P + h.slot[j]) * M + k] = X;
     }
     __syncthreads();
 #pragma unroll
