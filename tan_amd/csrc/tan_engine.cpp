@@ -1776,6 +1776,7 @@ static int32_t ensure_sums(tanx_conv *cv)
         cv->tread ^= 1;
         const int nf = fill_tail(cv, a);
         cv->tread ^= 1;
+        cv->tail_nchunk = cv->nchunk;  // set_tail_chunks may have come since tail_done
         return launch_timed(cv, cv->t_tail, nf, a, tail_bytes(cv, nf), cv->tail_alg_bytes);
     }
     const long long e = (long long)cv->ticks, c = cv->covered;

@@ -89,6 +89,33 @@ def few_partitions(P=4, kp=8, B=64, C=2):
     assert np.abs(ys[1]).max() > 0.1 and err <= 2e-6  # outputs up to 3, as in test_gpu_passes.py
 
 
+def chunk_changes(method=1, L=32768, B=64, C=3):
+    """The tail chunk count set between a call of several blocks and the next
+    block: as one block per call with the default count."""
+    # (the first call: a non-uniform object's response fades in up to three frames later)
+    calls, chunks = [200, 8, 1, 7, 1, 1, 9, 1, 6, 2, 12, 1], {2: 4, 4: 1, 5: 0, 7: 3, 9: 2, 11: 8}
+    nb = sum(calls)
+    x = T.signals.input_bank(C, nb * B, base_seed=31)
+    h = T.signals.ir_bank(C, L, 0, base_seed=32)
+    ctx = T.TANContext(device=0)
+    ys = []
+    for sizes in (calls, [1] * nb):
+        conv = T.TANConvolution(ctx, nu_multiple=64 if method == 1 else 0)
+        assert conv.InitGpu(METHODS[method], L, B, C) == T.AMF_OK
+        update(conv, h)
+        xd, yd = simlib.Dev(C, nb * B, x), simlib.Dev(C, nb * B, 0.0)
+        t = 0
+        for i, n in enumerate(sizes):
+            if sizes is calls and i in chunks:
+                assert lib.tanx_conv_set_tail_chunks(conv.handle, chunks[i]) == T.AMF_OK
+            call(conv, xd, yd, t, n, B)
+            t += n
+        ys.append(yd.a.copy())
+    err = float(np.abs(ys[0].astype(np.float64) - ys[1]).max())
+    print(f"chunk count changed between calls: {err:.3e}", flush=True)
+    assert np.abs(ys[1]).max() > 0.1 and err <= 2e-6  # outputs up to 3, as in test_gpu_passes.py
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]](**{k: int(v) for k, v in (a.split("=") for a in sys.argv[2:])})
     print("scenario complete", flush=True)

@@ -70,3 +70,31 @@ def test_few_partitions(gpu_ctx, P, kp, B):
         conv.Terminate()
     assert np.abs(ys[1]).max() > 0.1
     assert np.abs(ys[0].astype(np.float64) - ys[1]).max() <= 2e-6  # outputs up to 3, as in test_gpu_passes.py
+
+
+@pytest.mark.parametrize("method,L,B,mult", [(UNIFORM, 32768, 64, 0), (NONUNIFORM, 32768, 64, 64),
+                                             (NONUNIFORM, 65536, 256, 16)])
+def test_chunk_changes(gpu_ctx, method, L, B, mult):
+    """The tail chunk count set between a call of several blocks and the next
+    block: as one block per call with the default count."""
+    import torch
+    # (the first call: a non-uniform object's response fades in up to three frames later)
+    calls, chunks = [200, 8, 1, 7, 1, 1, 9, 1, 6, 2, 12, 1], {2: 4, 4: 1, 5: 0, 7: 3, 9: 2, 11: 8}
+    C, nb = 3, sum(calls)
+    x = torch.from_numpy(T.signals.input_bank(C, nb * B, base_seed=31)).cuda()
+    h = T.signals.ir_bank(C, L, 0, base_seed=32)
+
+    def chunk(n):
+        def issue(conv):
+            assert conv.SetTailChunks(n) == T.AMF_OK
+        return issue
+
+    ys = []
+    for sizes, before in ((calls, {i: chunk(n) for i, n in chunks.items()}), ([1] * nb, None)):
+        conv = T.TANConvolution(gpu_ctx, nu_multiple=mult)
+        assert conv.InitGpu(method, L, B, C) == T.AMF_OK
+        _update(h)(conv)
+        ys.append(_run(conv, x, torch.zeros_like(x), sizes, B, before))
+        conv.Terminate()
+    assert np.abs(ys[1]).max() > 0.1
+    assert np.abs(ys[0].astype(np.float64) - ys[1]).max() <= 2e-6  # outputs up to 3, as in test_gpu_passes.py

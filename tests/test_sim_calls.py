@@ -25,3 +25,8 @@ def test_in_place(sim_built, method):  # noqa: F811
 @pytest.mark.parametrize("P,kp,B", [(1, 4, 64), (2, 4, 64), (4, 16, 64), (8, 4, 64), (4, 4, 1024), (8, 12, 512)])
 def test_few_partitions(sim_built, P, kp, B):  # noqa: F811
     _run("few_partitions", P=P, kp=kp, B=B)
+
+
+@pytest.mark.parametrize("method", [0, 1], ids=["uniform", "nonuniform"])
+def test_chunk_changes(sim_built, method):  # noqa: F811
+    _run("chunk_changes", method=method)
