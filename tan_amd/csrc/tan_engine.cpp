@@ -1637,6 +1637,10 @@ static int32_t process_call(tanx_conv *cv, const float *din, long long in_stride
     const bool small = (size_t)cv->C * cv->P * B * (sizeof(float2) + ir_elem_bytes(cv->irtype)) <= kCachedRowsMax;
     int chunks = std::max(1, std::min((groups + cv->C - 1) / cv->C, cv->P / 16));
     if (small) chunks = std::max(chunks, (cv->P + 63) / 64);
+    // where k_call_pass sums a whole FP32 chunk as one chain (CallFold), chunks
+    // shorter than the object's own: the chain starts with the near partitions
+    // that a head adds last
+    if (cv->irtype == IR_F32 && cv->B > 256 && xb >= 0) chunks = std::max(chunks, cv->nchunk * 3 / 2);
     chunks = std::max(1, std::min(chunks, (rows - done) / outs));
     a.pc = (cv->P + chunks - 1) / chunks;
     a.nchunk = (cv->P + a.pc - 1) / a.pc;

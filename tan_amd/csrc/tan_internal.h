@@ -312,10 +312,11 @@ hipError_t launch_window(int B, int tail_nf, const HeadBatchArgs &h, const TickA
                          hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 // A call's blocks w .. w+n-1 of a uniform object (n <= kPassMax) in three
 // launches, all known at once: the blocks' spectra (k_call_spectra, into X),
-// one sweep over every partition for the n outputs (k_call_pass: partition i
-// of block w+k meets X row k - i, or FDL row w + k - i before the call; it
+// one sweep over partitions 1 .. P-1 for the n outputs (k_call_pass: partition
+// i of block w+k meets X row k - i, or FDL row w + k - i before the call; it
 // also keeps the last input block) and the inverse transforms (k_call_out),
-// which also move X into the FDL ring.  One block of the call may crossfade.
+// which also add partition 0 and move X into the FDL ring.  One block of the
+// call may crossfade.
 struct CallArgs {
     int C, P, n;
     int irtype;

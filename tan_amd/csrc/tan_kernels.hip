@@ -855,18 +855,27 @@ struct SweepRows {
 // dc: the lane's first bin is the packed (DC, Nyquist) element.
 // NF filters: HA for outputs k < kA, HB (NF = 2) for outputs k >= kB; with
 // one filter every output is computed (the caller stores those it wants).
-// FOLD: fold() is called once between the partitions before pf and those from pf on
-// (p0 < pf < p1), to put the sums so far aside; the trips are laid so that
-// one starts at pf and the loads in flight go on across it.
-template <int M, int NF, int HT, bool NT, int KM, bool FOLD, class Fold>
+// SEG = 2: fold() is called once between the partitions before pf and those
+// from pf on (p0 < pf < p1), to put the sums so far aside; the trips are laid
+// so that one starts at pf and the loads in flight go on across it.  SEG = 0:
+// it is called after every kFold partitions but the last.
+template <int NF, int KM, int SEG, int E>
+struct SweepTrip {
+    static constexpr int kBody = NF == 2 ? 4 : KM < 8 || (SEG == 0 && E == 2) ? 8 : KM;  // partitions per loop trip
+    // 12 to 16 partitions, 8 of the long rows (which have fewer)
+    static constexpr int kFold = E == 2 || kBody >= 12 ? kBody : (16 / kBody) * kBody;
+};
+
+template <int M, int NF, int HT, bool NT, int KM, int SEG, class Fold>
 __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA, const char *HB, const float *SA,
                                            const float *SB, int p0, int pf, int p1, int r, bool dc, int kA, int kB,
                                            Bins<PassGeo<M, HT>::E> (&accA)[KM], Bins<PassGeo<M, HT>::E> (&accB)[KM],
                                            Fold fold)
 {
     constexpr int E = PassGeo<M, HT>::E;
-    constexpr int U = PassGeo<M, HT>::U;                  // partitions per stage
-    constexpr int kBody = NF == 2 ? 4 : KM < 8 ? 8 : KM;  // partitions per loop trip
+    constexpr int U = PassGeo<M, HT>::U;  // partitions per stage
+    constexpr int kBody = SweepTrip<NF, KM, SEG, E>::kBody, kFold = SweepTrip<NF, KM, SEG, E>::kFold;
+    constexpr bool FOLD = SEG == 2;
     constexpr size_t kRowBytes = (size_t)M * IrRow<HT>::kBytes;
     static_assert(kBody % U == 0 && KM <= kPassMax, "pass length");
     // entry KM - 1 + q of the window holds the row of partition i + q (row
@@ -914,7 +923,7 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
     };
     load(cur, p0 - lead);
     for (int i = p0 - lead; i < p1; i += kBody) {
-        if (FOLD && i == pf && i > p0) fold();
+        if (SEG == 2 ? i == pf && i > p0 : SEG == 0 && i > p0 && (i - p0) % kFold == 0) fold();
 #pragma unroll
         for (int q0 = 0; q0 < kBody; q0 += U) {
             load(nxt, i + q0 + U);
@@ -966,7 +975,8 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
 // skip is uniform.  The range is cut into SEG * G segments, each summed as
 // one chain; a lane group takes SEG of them in one sweep (its first one's
 // sums wait in LDS, one float2 per output and thread) and an output adds the
-// segments in order.  All threads call it.
+// segments in order.  SEG = 0: one segment per lane group, its chains of
+// kFold partitions each added up there.  All threads call it.
 template <int M, int NF, int HT, bool NT, int KM, int SEG, class Out>
 __device__ __forceinline__ void sweep_outputs(const SweepRows &rows, const char *HA, const char *HB, const float *SA,
                                               const float *SB, int i0, int i1, int pmin, bool dc0, int kA, int kB,
@@ -978,25 +988,32 @@ __device__ __forceinline__ void sweep_outputs(const SweepRows &rows, const char 
                   : Geo::R % 64 == 0 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / Geo::R)
                                      : (int)threadIdx.x / Geo::R;
     const int r = threadIdx.x % Geo::R;
-    constexpr int NS = SEG * Geo::G;
+    constexpr int PG = SEG == 0 ? 1 : SEG, NS = PG * Geo::G;  // segments of a lane group, in all
     const int span = (i1 - i0 + NS - 1) / NS;
-    float2 *sums = reinterpret_cast<float2 *>(red);  // [G][S]
-    float2 *firsts = sums + kTickThreads;            // [outputs][threads]
+    constexpr int E = Geo::E;
+    float2 *sums = reinterpret_cast<float2 *>(red);          // [G][S]
+    float2 *firsts = sums + (Geo::G > 1 ? kTickThreads : 0);  // [outputs][threads][E]
     // filter f's output k: the filters' outputs together are at most KM + 1
-    auto first = [&](int f, int k) { return firsts + (k + f) * kTickThreads; };
+    auto first = [&](int f, int k) { return firsts + (k + f) * kTickThreads * E; };
     Bins<Geo::E> acc[2][KM];
-    const int q0 = min(i1, i0 + g * SEG * span), pf = min(i1, q0 + span), p1 = min(i1, q0 + SEG * span);
+    const int q0 = min(i1, i0 + g * PG * span), pf = min(i1, q0 + span), p1 = min(i1, q0 + PG * span);
     const int p0 = max(q0, pmin);
-    const bool both = SEG == 2 && p0 < pf && pf < p1;
-    pass_sweep<M, NF, HT, NT, KM, SEG == 2>(rows, HA, HB, SA, SB, p0, pf, p1, r, dc0 && r == 0, kA, kB, acc[0], acc[1], [&] {
+    bool both = false;  // LDS holds sums of this group
+    pass_sweep<M, NF, HT, NT, KM, SEG>(rows, HA, HB, SA, SB, p0, pf, p1, r, dc0 && r == 0, kA, kB, acc[0], acc[1], [&] {
 #pragma unroll
         for (int f = 0; f < NF; f++)
 #pragma unroll
             for (int k = 0; k < KM; k++)
                 if (NF == 1 || (f == 0 ? k < kA : k >= kB)) {
-                    first(f, k)[threadIdx.x] = make_float2(acc[f][k].re[0], acc[f][k].im[0]);
-                    acc[f][k].re[0] = acc[f][k].im[0] = 0.f;
+#pragma unroll
+                    for (int e = 0; e < E; e++) {
+                        float2 &to = first(f, k)[threadIdx.x * E + e];
+                        const float2 v = make_float2(acc[f][k].re[e], acc[f][k].im[e]);
+                        to = SEG == 0 && both ? cadd(to, v) : v;
+                        acc[f][k].re[e] = acc[f][k].im[e] = 0.f;
+                    }
                 }
+        both = true;
     });
     // unrolled over the outputs so that every pointer is picked statically
     // (an output pointer indexed at run time would put the whole argument
@@ -1009,22 +1026,27 @@ __device__ __forceinline__ void sweep_outputs(const SweepRows &rows, const char 
             if (!o) continue;
             const Bins<Geo::E> &a = acc[f][k];
             if constexpr (Geo::G == 1) {
-                float2 v = make_float2(a.re[0], a.im[0]);
-                if (both) v = cadd(first(f, k)[threadIdx.x], v);
-                if constexpr (Geo::E == 1) gst(o + r, v);
-                else gst(reinterpret_cast<float4 *>(o) + r, make_float4(v.x, v.y, a.re[1], a.im[1]));
+                float2 v[E];
+#pragma unroll
+                for (int e = 0; e < E; e++) {
+                    v[e] = make_float2(a.re[e], a.im[e]);
+                    if (SEG != 1 && both) v[e] = cadd(first(f, k)[threadIdx.x * E + e], v[e]);
+                }
+                if constexpr (E == 1) gst(o + r, v[0]);
+                else gst(reinterpret_cast<float4 *>(o) + r, make_float4(v[0].x, v[0].y, v[1].x, v[1].y));
             } else {
+                static_assert(SEG == 1 || E == 1, "one bin per lane in LDS");
                 static_assert(Geo::S == M && Geo::G * M == kTickThreads * Geo::E, "pass reduction buffer");
                 // (a group without a second segment: no first one, the sums as they are)
-                if (SEG == 2 && !both) first(f, k)[threadIdx.x] = make_float2(0.f, 0.f);
+                if (SEG != 1 && !both) first(f, k)[threadIdx.x] = make_float2(0.f, 0.f);
 #pragma unroll
                 for (int e = 0; e < Geo::E; e++) sums[g * M + Geo::E * r + e] = make_float2(a.re[e], a.im[e]);
                 __syncthreads();
                 for (int b = threadIdx.x; b < M; b += kTickThreads) {
-                    float2 sum = SEG == 2 ? cadd(first(f, k)[b], sums[b]) : sums[b];
+                    float2 sum = SEG != 1 ? cadd(first(f, k)[b], sums[b]) : sums[b];
 #pragma unroll
                     for (int gg = 1; gg < Geo::G; gg++) {
-                        if constexpr (SEG == 2) sum = cadd(sum, first(f, k)[gg * Geo::R + b]);
+                        if constexpr (SEG != 1) sum = cadd(sum, first(f, k)[gg * Geo::R + b]);
                         sum = cadd(sum, sums[gg * M + b]);
                     }
                     gst(o + b, sum);
@@ -1579,13 +1601,28 @@ __global__ __launch_bounds__(kTickThreads) void k_call_spectra(CallArgs a)
     for (int k = tid; k < M; k += NT) row[k] = r2c_post<M>(Z, k, a.twN);
 }
 
-// NT: streamed rows, a chunk's sums in two chains; otherwise (short chunks of
-// rows that the caches hold) ordinary loads and one chain
+// A chunk of FP32 rows is summed in chains of kFold partitions, added up in
+// LDS: one chain of its 64 to 128 partitions lost what the single blocks'
+// split keeps (16 blocks of 64 channels x 65,536 taps: 3.1e-7 of the output
+// against FP64, 2.3e-7 a block at a time and with the short chains).  Not
+// two-bin lanes with two filters, which the LDS they would need slows (9 blocks
+// of 100 channels x 100,000 taps at B = 512: 226 us, 137 without): their chunks
+// are short instead.  16-bit rows lose 2e-4 by their storage.
+template <int M, int NF, int HT, int KM>
+struct CallFold {
+    using Geo = PassGeo<M, HT>;
+    static constexpr int kSums = (Geo::G > 1 ? kTickThreads / 2 : 0) + (KM + NF - 1) * kTickThreads * Geo::E / 2;
+    static constexpr int SEG = HT == IR_F32 && (NF == 1 || Geo::E == 1) ? 0 : 1;
+    static constexpr int kRed = SEG == 0 && kSums > tail_red_float4<M>() ? kSums : tail_red_float4<M>();  // float4
+};
+
+// NT: streamed rows; otherwise (rows that the caches hold) ordinary loads.
 template <int M, int NF, int HT, bool NT, int KM>
 __global__ __launch_bounds__(kTickThreads) void k_call_pass(CallArgs a)
 {
     using Geo = PassGeo<M, HT>;
-    __shared__ float4 red[pass_red_float4<M, NF, HT, KM>()];
+    using Fold = CallFold<M, NF, HT, KM>;
+    __shared__ float4 red[Fold::kRed];
     const int c = blockIdx.x / a.nchunk, j = blockIdx.x - c * a.nchunk;
     if (!a.run[c]) return;
     // the last block's input is the next call's previous one: kept here, after
@@ -1601,7 +1638,9 @@ __global__ __launch_bounds__(kTickThreads) void k_call_pass(CallArgs a)
     const int kA = NF == 2 ? a.xb + 1 : a.n, kB = NF == 2 ? a.xb : a.n;
     for (int s0 = 0; s0 < M; s0 += Geo::S) {
         const size_t at = (size_t)c * a.P * M + s0;
-        const SweepRows rows = {a.fdl + at, a.X + (size_t)c * a.n * M + s0, a.slot, a.P - 1, a.n};
+        // a block's own spectrum (partition 0) is k_call_out's, so the last
+        // block's serves none of the sums
+        const SweepRows rows = {a.fdl + at, a.X + (size_t)c * a.n * M + s0, a.slot, a.P - 1, a.n - 1};
         const char *HA = reinterpret_cast<const char *>(a.HA) + at * IrRow<HT>::kBytes;
         const char *HB = NF == 2 ? reinterpret_cast<const char *>(a.HB) + at * IrRow<HT>::kBytes : nullptr;
         // this chunk's row of filter f's output k
@@ -1609,11 +1648,23 @@ __global__ __launch_bounds__(kTickThreads) void k_call_pass(CallArgs a)
             if (!(f == 0 ? k < kA : k >= kB && k < a.n)) return nullptr;
             return a.T + (((size_t)c * (a.n + NF - 1) + k + f) * a.nchunk + j) * M + s0;
         };
-        sweep_outputs<M, NF, HT, NT, KM, NT ? Geo::SEG : 1>(rows, HA, HB, SA, SB, i0, i1, 0, s0 == 0, kA, kB, red,
-                                                            out);
+        sweep_outputs<M, NF, HT, NT, KM, Fold::SEG>(rows, HA, HB, SA, SB, i0, i1, 1, s0 == 0, kA, kB, red, out);
     }
 }
 
+// Bin k of partition 0 of channel c
+__device__ __forceinline__ float2 first_partition(int irtype, const void *H, const float *S, int c, int P, int M, int k)
+{
+    if (irtype == IR_F32) return IrRow<IR_F32>::get1(ir_row<IR_F32>(H, c, P, 0, M), k);
+    const float s = gld(S + (size_t)c * P);
+    const float2 h = irtype == IR_F16 ? IrRow<IR_F16>::get1(ir_row<IR_F16>(H, c, P, 0, M), k)
+                                      : IrRow<IR_BF16>::get1(ir_row<IR_BF16>(H, c, P, 0, M), k);
+    return make_float2(h.x * s, h.y * s);
+}
+
+// Adds the block's chunks (each batch of CB loaded and summed together: one
+// chain over 64 chunks would round as often), then, as the heads do, partition
+// 0, whose terms are the largest, and inverts.
 template <int M>
 __global__ __launch_bounds__(kTickThreads) void k_call_out(CallArgs a)
 {
@@ -1634,8 +1685,18 @@ __global__ __launch_bounds__(kTickThreads) void k_call_out(CallArgs a)
     float2 wn[KPT];
 #pragma unroll
     for (int q = 0; q < KPT; q++) wn[q] = a.twN[tid + q * NT];
+    const float2 *row = a.X + (size_t)item * M;
+    float2 *to = a.fdl + ((size_t)c * a.P + ((a.slot + k) & (a.P - 1))) * M;
+    float2 x[KPT];
+#pragma unroll
+    for (int q = 0; q < KPT; q++) x[q] = row[tid + q * NT];
     float2 y[ZP];
     for (int f = 0; f < (two ? 2 : 1); f++) {
+        const bool second = f == 1 || k > a.xb;
+        float2 h0[KPT];
+#pragma unroll
+        for (int q = 0; q < KPT; q++)
+            h0[q] = first_partition(a.irtype, second ? a.HB : a.HA, second ? a.SB : a.SA, c, a.P, M, tid + q * NT);
         // the row of this block's filter: A's up to the crossfade, B's (one further) after it
         const int o = two ? k + f : k + (k > a.xb ? 1 : 0);
         const float2 *T = a.T + ((size_t)c * outs + o) * a.nchunk * M;
@@ -1649,15 +1710,21 @@ __global__ __launch_bounds__(kTickThreads) void k_call_out(CallArgs a)
 #pragma unroll
                 for (int q = 0; q < KPT; q++) t[u][q] = T[(size_t)min(j0 + u, a.nchunk - 1) * M + tid + q * NT];
 #pragma unroll
-            for (int u = 0; u < CB; u++)
+            for (int q = 0; q < KPT; q++) {
+                float2 b = t[0][q];
 #pragma unroll
-                for (int q = 0; q < KPT; q++) {
-                    s[q].x += j0 + u < a.nchunk ? t[u][q].x : 0.f;
-                    s[q].y += j0 + u < a.nchunk ? t[u][q].y : 0.f;
+                for (int u = 1; u < CB; u++) {
+                    b.x += j0 + u < a.nchunk ? t[u][q].x : 0.f;
+                    b.y += j0 + u < a.nchunk ? t[u][q].y : 0.f;
                 }
+                s[q] = cadd(s[q], b);
+            }
         }
 #pragma unroll
-        for (int q = 0; q < KPT; q++) s1[w][tid + q * NT] = s[q];
+        for (int q = 0; q < KPT; q++) {
+            mac2(s[q], x[q], h0[q], tid + q * NT == 0);
+            s1[w][tid + q * NT] = s[q];
+        }
         group_sync<NT>();
 #pragma unroll
         for (int q = 0; q < KPT; q++) s0[w][tid + q * NT] = c2r_pre_w<M>(s1[w], tid + q * NT, wn[q]);
@@ -1696,10 +1763,8 @@ __global__ __launch_bounds__(kTickThreads) void k_call_out(CallArgs a)
         }
     }
     // the block's spectrum enters the delay line
-    const float2 *row = a.X + (size_t)item * M;
-    float2 *to = a.fdl + ((size_t)c * a.P + ((a.slot + k) & (a.P - 1))) * M;
 #pragma unroll
-    for (int q = 0; q < KPT; q++) to[tid + q * NT] = row[tid + q * NT];
+    for (int q = 0; q < KPT; q++) to[tid + q * NT] = x[q];
 }
 
 // ---------------------------------------------------------------------------

@@ -98,3 +98,51 @@ def test_chunk_changes(gpu_ctx, method, L, B, mult):
         conv.Terminate()
     assert np.abs(ys[1]).max() > 0.1
     assert np.abs(ys[0].astype(np.float64) - ys[1]).max() <= 2e-6  # outputs up to 3, as in test_gpu_passes.py
+
+
+# one bin and two per lane, one filter and a crossfade, chunks of one object's and of many channels
+@pytest.mark.parametrize("C,L,B,n,switch", [(64, 65536, 256, 16, False), (256, 65536, 256, 16, False),
+                                            (200, 65536, 128, 9, False), (250, 65536, 256, 12, True),
+                                            (300, 65536, 512, 16, False), (100, 65536, 512, 9, True)])
+def test_error_of_calls(gpu_ctx, C, L, B, n, switch):
+    """Calls of several blocks are no further from FP64 than one block per
+    call.  Both errors are sums of tens of millions of roundings, which vary
+    by a few percent with the order of the sums: 5% is allowed."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(C + n)
+    decay = torch.exp(-torch.arange(L, device="cuda") / 12000.0)
+    irs = [torch.randn(C, L, device="cuda", generator=g) * decay for _ in range(2)]
+    warm = L // B + 4
+    x = torch.empty(C, (warm + n) * B, device="cuda").uniform_(-1, 1, generator=g)
+    ys = [[], []]
+    for way in range(2):
+        conv = T.TANConvolution(gpu_ctx)
+        assert conv.InitGpu(UNIFORM, L, B, C) == T.AMF_OK
+        assert conv.UpdateResponseTD(irs[0], L) == T.AMF_OK
+        y = torch.zeros_like(x)
+        _run(conv, x, y, [warm], B)
+        if switch:
+            assert conv.UpdateResponseTD(irs[1], L) == T.AMF_OK
+        tail = slice(warm * B, None)
+        _run(conv, x[:, tail], y[:, tail], [n] if way == 0 else [1] * n, B)
+        ys[way] = y[:, tail].double()
+        conv.Terminate()
+
+    def exact(h):
+        hist = x[:, -(L + n * B):].double()
+        size = 1 << (hist.shape[1] + L).bit_length()
+        out = torch.empty(C, n * B, dtype=torch.float64, device="cuda")
+        for c in range(0, C, 50):
+            f = torch.fft.rfft(hist[c:c + 50], size) * torch.fft.rfft(h[c:c + 50].double(), size)
+            out[c:c + 50] = torch.fft.irfft(f, size)[:, L:L + n * B]
+        return out
+
+    ref = exact(irs[0])
+    if switch:  # the update is handed off by the first block and crossfades in the third
+        new, at = exact(irs[1]), 2 * B
+        j = torch.arange(B, device="cuda", dtype=torch.float64) / B
+        ref[:, at:at + B] = new[:, at:at + B] * j + ref[:, at:at + B] * (1 - j)
+        ref[:, at + B:] = new[:, at + B:]
+    err = [float((y - ref).norm() / ref.norm()) for y in ys]
+    assert err[1] <= 1e-6
+    assert err[0] <= 1.05 * err[1], err
