@@ -1644,11 +1644,11 @@ static int32_t process_call(tanx_conv *cv, const float *din, long long in_stride
     chunks = std::max(1, std::min(chunks, (rows - done) / outs));
     a.pc = (cv->P + chunks - 1) / chunks;
     a.nchunk = (cv->P + a.pc - 1) / a.pc;
-    // ordinary loads and one chain of sums per chunk while the caches hold the
-    // rows (a chunk's window is filled from rows its neighbour reads too): 16
-    // blocks of 64 channels x 65,536 taps 28 us, 35 us with streaming loads;
-    // larger objects stream (1,024 channels: 268 against 287 us)
-    a.cached = small && a.pc <= 64;
+    // ordinary loads while the caches hold the rows of every live object, as in
+    // the passes; streaming beyond (calls of 16 blocks on 12 objects of 64
+    // channels x 65,536 taps in turn: 32.6 us each with ordinary loads, 29.9
+    // streamed; 1,024 channels: 287 and 268 us)
+    a.cached = cached_rows(cv);
     a.X = cv->T;
     a.T = cv->T + (size_t)cv->C * done * B;
     hipStream_t s = cv->ctx->proc;
