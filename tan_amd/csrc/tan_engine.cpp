@@ -383,7 +383,8 @@ struct tanx_conv {
     uint64_t rows_bytes = 0;
     long long covered = 0;
     // the sums of blocks ticks .. covered are scheduled (porg) but not
-    // computed: process_call leaves them to the next block that needs them
+    // computed: process_call leaves them to the call's end or the next block
+    // that needs them
     bool deferred = false;
     long long porg[2 * kPassMax][2] = {};
     int pchunk[2 * kPassMax][2] = {};
@@ -1004,6 +1005,14 @@ static TickArgs tick_common(tanx_conv *cv)
 // current block alone.
 static int fill_pass(tanx_conv *cv, long long w, long long e, TickArgs &a);
 
+// Blocks of a pass that begins with block e: it ends on the phase grid, its
+// last block c satisfies (c + kphase) % kp == 0, so the next pass runs in that
+// block's launch.
+static int grid_blocks(const tanx_conv *cv, long long e)
+{
+    return (int)(((-(long long)cv->kphase - e) % cv->kp + cv->kp) % cv->kp) + 1;
+}
+
 static int fill_tail(tanx_conv *cv, TickArgs &a)
 {
     if (cv->kp > 1) {
@@ -1047,9 +1056,7 @@ static int fill_pass(tanx_conv *cv, long long w, long long e, TickArgs &a)
         a.kn = 1;
         return 0;
     }
-    // the pass ends on the phase grid: its last block c satisfies
-    // (c + kphase) % kp == 0, so the next pass runs in that block's launch
-    const int kn = (int)(((-(long long)cv->kphase - e) % cv->kp + cv->kp) % cv->kp) + 1;
+    const int kn = grid_blocks(cv, e);
     const long long s_rel = (sw >= e && sw < e + kn) ? sw - e : -1;
     a.nchunk = cv->nchunk;
     a.pc = cv->pc;
@@ -1568,11 +1575,54 @@ static void schedule_queued(tanx_conv *cv, int *queued)
     *queued = 0;
 }
 
+// The part of the pass ring (4 kp pieces of maxchunk rows per channel: a piece
+// per block and filter) that the sums of blocks e .. e + m - 1 leave free,
+// the larger one: its first piece and number of rows.
+static int call_space(const tanx_conv *cv, long long e, int m, int *first)
+{
+    const int pieces = 4 * cv->kp;
+    *first = 0;
+    if (m == 0) return pieces * cv->maxchunk;
+    const int from = 2 * cv->pring(e), to = 2 * cv->pring(e + m - 1) + 1;  // (a switch's second sums are free)
+    if (to < from) {
+        *first = to;
+        return (from - to) * cv->maxchunk;
+    }
+    if (pieces - to > from) *first = to;
+    return std::max(from, pieces - to) * cv->maxchunk;
+}
+
+// Blocks e .. on the pass grid after a call of n blocks whose partial sums the
+// call's sweep can compute (two: with a crossfade), 0 if it can not: outputs
+// that its lanes hold, and sums that leave room for the call's own.
+static int call_ahead(const tanx_conv *cv, int n, long long e, bool two)
+{
+    const int m = grid_blocks(cv, e);
+    int first = 0;
+    const int most = cv->irtype == IR_F32 && cv->B <= 256 && !two ? kSweepMax : kPassMax;
+    return n + m <= most && call_space(cv, e, m, &first) >= 2 * n + 1 ? m : 0;
+}
+
+// Whether a device call of nb blocks takes process_call's launches.  They
+// leave the partial sums of the blocks after the call as every block does: in
+// one sweep with the call's own, or in one more sweep over the rows.  A block
+// at a time is a sweep every kp blocks, so a call of any length, and any mix
+// of calls, sweeps no more than before.
+static bool call_pays(const tanx_conv *cv, size_t nb)
+{
+    const size_t most = (size_t)std::max(1, call_blocks_max(cv));
+    if (std::min(nb, most) < call_blocks_min(cv)) return false;
+    const bool update = cv->pending || cv->ready || cv->delayed;
+    const bool one = nb <= most && call_ahead(cv, (int)nb, (long long)(cv->ticks + nb), update) > 0;
+    return ((nb + most - 1) / most + (one ? 0 : 1)) * (size_t)cv->kp <= nb;
+}
+
 // The next n blocks of a device call of a uniform object with multi-block
 // passes, in three launches (CallArgs).  A call ends before a second
-// crossfade; *advanced is the number of blocks taken.
+// crossfade; *advanced is the number of blocks taken.  whole: they are the
+// call's only ones.
 static int32_t process_call(tanx_conv *cv, const float *din, long long in_stride, float *dout, long long out_stride,
-                            int n, int *advanced, int *queued)
+                            int n, bool whole, int *advanced, int *queued)
 {
     const size_t B = cv->B;
     *advanced = 0;
@@ -1617,7 +1667,6 @@ static int32_t process_call(tanx_conv *cv, const float *din, long long in_stride
         const bool armed = cv->delayed && cv->switch_at == cv->ticks;
         if (xfade || armed || cv->B > kHeadBatchMaxB) schedule_queued(cv, queued);
     }
-    cv->deferred = true;
     *advanced = done;
     a.n = done;
     a.xb = xb >= 0 ? xb : done;
@@ -1633,24 +1682,42 @@ static int32_t process_call(tanx_conv *cv, const float *din, long long in_stride
     // fewer: 16 blocks of 64 channels 30, 35 and 42 us with 256, 512 and 1,024
     // workgroups; 8 blocks with a crossfade 54, 52 and 55 us), of at least 16
     // partitions, as many as the rows hold
-    const int rows = 4 * cv->kp * cv->maxchunk, groups = done > 8 ? 256 : 512;
+    const long long e = (long long)cv->ticks;
+    if (whole && done == n && !cv->delayed) a.ahead = call_ahead(cv, done, e, xb >= 0);
+    int first = 0;
+    const int rows = call_space(cv, e, a.ahead, &first), groups = done > 8 ? 256 : 512;
     const bool small = (size_t)cv->C * cv->P * B * (sizeof(float2) + ir_elem_bytes(cv->irtype)) <= kCachedRowsMax;
     int chunks = std::max(1, std::min((groups + cv->C - 1) / cv->C, cv->P / 16));
     if (small) chunks = std::max(chunks, (cv->P + 63) / 64);
-    // where k_call_pass sums a whole FP32 chunk as one chain (CallFold), chunks
-    // shorter than the object's own: the chain starts with the near partitions
-    // that a head adds last
-    if (cv->irtype == IR_F32 && cv->B > 256 && xb >= 0) chunks = std::max(chunks, cv->nchunk * 3 / 2);
+    // two filters' FP32 chunks are one or two chains (CallFold): shorter than
+    // the object's own chunks, whose chains do not start with the near
+    // partitions (a head adds them last), but no shorter than they need be
+    if (cv->irtype == IR_F32 && xb >= 0)
+        chunks = std::max(chunks, std::min(cv->nchunk * 3 / 2, cv->P / (B <= 256 ? 32 : 8)));
     chunks = std::max(1, std::min(chunks, (rows - done) / outs));
+    if (a.ahead > 0) chunks = std::min(chunks, cv->maxchunk);
     a.pc = (cv->P + chunks - 1) / chunks;
     a.nchunk = (cv->P + a.pc - 1) / a.pc;
+    cv->deferred = a.ahead == 0;
+    if (a.ahead > 0) {
+        // scheduled as by a pass in the launch of the last block
+        TickArgs p{};
+        cv->covered = e - 1;
+        *queued = 0;
+        if (fill_pass(cv, e - 1, e, p) != 1 || p.kn != a.ahead) return TANX_UNEXPECTED;
+        for (long long b = e; b < e + a.ahead; b++) cv->pchunk[cv->pring(b)][0] = a.nchunk;
+        a.sums = cv->T;
+        a.ring0 = cv->pring(e);
+        a.ring = 2 * cv->kp;
+        a.sums_stride = 2 * (size_t)cv->C * cv->maxchunk * B;
+    }
     // ordinary loads while the caches hold the rows of every live object, as in
     // the passes; streaming beyond (calls of 16 blocks on 12 objects of 64
     // channels x 65,536 taps in turn: 32.6 us each with ordinary loads, 29.9
     // streamed; 1,024 channels: 287 and 268 us)
     a.cached = cached_rows(cv);
-    a.X = cv->T;
-    a.T = cv->T + (size_t)cv->C * done * B;
+    a.X = cv->T + (size_t)first * cv->C * cv->maxchunk * B;
+    a.T = a.X + (size_t)cv->C * done * B;
     hipStream_t s = cv->ctx->proc;
     if (cv->timing) {
         hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1766,7 +1833,7 @@ static int32_t process_call_nu(tanx_conv *cv, const float *din, long long in_str
     return TANX_OK;
 }
 
-// Computes the sums process_call left: of the blocks ticks .. covered with
+// Computes the sums process_call and process_call_nu left: of the blocks ticks .. covered with
 // the filters they use now (the switch state that of their scheduling), from
 // the rows before their origin.  Blocks of one filter share their origin.
 static int32_t ensure_sums(tanx_conv *cv)
@@ -1969,27 +2036,21 @@ extern "C" int32_t tanx_conv_process_device(tanx_conv *cv, const float *d_in, si
     HeadQueue hq;
     const bool fuse = cv->fused && !cv->fmode;
     size_t b = 0;
-    const size_t most = (size_t)std::max(1, call_blocks_max(cv));
-    if (fuse && cv->kp > 1 && !flags && std::min(nb, most) >= call_blocks_min(cv)) {
+    if (fuse && cv->kp > 1 && !flags && call_pays(cv, nb)) {
         // windows of equal length
+        const size_t most = (size_t)call_blocks_max(cv);
         const size_t windows = (nb + most - 1) / most, want = (nb + windows - 1) / windows;
         int queued = 0;
         while (b < nb) {
             int took = 0;
             const int32_t rc = process_call(cv, d_in + b * B, (long long)in_stride, d_out + b * B,
-                                            (long long)out_stride, (int)std::min(nb - b, want), &took, &queued);
+                                            (long long)out_stride, (int)std::min(nb - b, want), windows == 1, &took, &queued);
             if (rc != TANX_OK) return rc;
             b += (size_t)took;
             if (processed) *processed = b * B;
         }
         schedule_queued(cv, &queued);
     }
-    auto finish = [&](int32_t rc) {
-        // a long call also computes the sums of the blocks after it (one sweep
-        // beside its four or more), a short one leaves them to a call that
-        // needs them: calls of several blocks in a row use none
-        return rc == TANX_OK && nb >= 4 * (size_t)kPassMax ? ensure_sums(cv) : rc;
-    };
     for (; b < nb; b++) {
         if (fuse && cv->nu && !flags) {
             const int take = (int)std::min<size_t>(nb - b, (size_t)nu_call_blocks(cv));
@@ -2014,7 +2075,9 @@ extern "C" int32_t tanx_conv_process_device(tanx_conv *cv, const float *d_in, si
         }
         if (processed) *processed = (b + 1) * B;
     }
-    return finish(flush_heads(cv, hq));
+    const int32_t rc = flush_heads(cv, hq);
+    // the partial sums of the blocks after the call are part of it
+    return rc == TANX_OK ? ensure_sums(cv) : rc;
 }
 
 /* ProcessDirect (ConvolutionImpl.cpp:719-762): time-domain objects only.

@@ -45,6 +45,7 @@ enum IrType { IR_F32 = 0, IR_F16 = 1, IR_BF16 = 2 };
 inline int ir_elem_bytes(int t) { return t == IR_F32 ? 8 : 4; }
 
 constexpr int kPassMax = 16;     // blocks one tail pass computes partial sums for, at most
+constexpr int kSweepMax = 20;    // outputs of a call's sweep, at most (CallArgs)
 constexpr int kPassDefault = 4;  // the library's choice for IRs of 16 or more partitions
 constexpr int kHeadBatch = 4;    // heads one launch runs together, at most
 // partitions a head adds itself at most: a pass of the launch with heads
@@ -337,6 +338,14 @@ struct CallArgs {
     int xb;                // block (of the n) that crossfades, n without one
     int nchunk, pc;        // partition chunks per channel and partitions per chunk
     int cached;            // nonzero: the sweep reads the rows with ordinary loads
+    // partial sums of the `ahead` blocks after the call, as a pass in the
+    // launch of block w + n - 1 alone leaves them (filter B's with a
+    // crossfade): block w + n + k's, [C][nchunk][B], at sums +
+    // ((ring0 + k) % ring) * sums_stride
+    int ahead;
+    float2 *sums;
+    int ring0, ring;
+    size_t sums_stride;
     // non-uniform objects: frame output added to block k's samples (channel c
     // at zA + c * zstride + k * B, or nullptr), and the input ring (or
     // nullptr): block w + k into slot (xslot + k) & xmask

@@ -861,7 +861,8 @@ struct SweepRows {
 // it is called after every kFold partitions but the last.
 template <int NF, int KM, int SEG, int E>
 struct SweepTrip {
-    static constexpr int kBody = NF == 2 ? 4 : KM < 8 || (SEG == 0 && E == 2) ? 8 : KM;  // partitions per loop trip
+    // partitions per loop trip
+    static constexpr int kBody = NF == 2 ? 4 : KM < 8 || (SEG == 0 && E == 2) ? 8 : KM > kPassMax ? kPassMax : KM;
     // 12 to 16 partitions, 8 of the long rows (which have fewer)
     static constexpr int kFold = E == 2 || kBody >= 12 ? kBody : (16 / kBody) * kBody;
 };
@@ -877,7 +878,7 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
     constexpr int kBody = SweepTrip<NF, KM, SEG, E>::kBody, kFold = SweepTrip<NF, KM, SEG, E>::kFold;
     constexpr bool FOLD = SEG == 2;
     constexpr size_t kRowBytes = (size_t)M * IrRow<HT>::kBytes;
-    static_assert(kBody % U == 0 && KM <= kPassMax, "pass length");
+    static_assert(kBody % U == 0 && KM <= kSweepMax, "pass length");
     // entry KM - 1 + q of the window holds the row of partition i + q (row
     // -(i + q)) for the trip starting at partition i; output k reads the
     // entry k before it
@@ -1563,12 +1564,14 @@ __global__ __launch_bounds__(kTickThreads) void k_window(HeadBatchArgs h, TickAr
 // block.  With every input block at hand the transforms are independent
 // (one wave each up to B = 256, C * n of them), the sweep reads each IR and
 // FDL row once for all n outputs, and only three launches follow each other.
+// The sweep also computes the partial sums of the blocks after the call where
+// the outputs together are few enough.
 // Every input sample is read before the last launch, the only one that writes
 // outputs: the caller's output may be its input.
-// Calls of 16 blocks, 64 channels x 65,536 taps at B = 256: 28 us, 89 us a
+// Calls of 16 blocks, 64 channels x 65,536 taps at B = 256: 32 us, 88 us a
 // launch per four blocks; 8 blocks of 1,024 channels x 131,072 taps with FP16
-// rows: 304 us (5.3 TB/s of rows), 577 us with two sweeps; 4 blocks of 1,024
-// channels x 65,536 taps: 185 us, 222 us before.
+// rows: 316 us (5.1 TB/s of rows), 575 us with two sweeps; 4 blocks of 1,024
+// channels x 65,536 taps: 192 us, 221 us before.
 // ---------------------------------------------------------------------------
 template <int M>
 __global__ __launch_bounds__(kTickThreads) void k_call_spectra(CallArgs a)
@@ -1604,16 +1607,17 @@ __global__ __launch_bounds__(kTickThreads) void k_call_spectra(CallArgs a)
 // A chunk of FP32 rows is summed in chains of kFold partitions, added up in
 // LDS: one chain of its 64 to 128 partitions lost what the single blocks'
 // split keeps (16 blocks of 64 channels x 65,536 taps: 3.1e-7 of the output
-// against FP64, 2.3e-7 a block at a time and with the short chains).  Not
-// two-bin lanes with two filters, which the LDS they would need slows (9 blocks
-// of 100 channels x 100,000 taps at B = 512: 226 us, 137 without): their chunks
-// are short instead.  16-bit rows lose 2e-4 by their storage.
+// against FP64, 2.3e-7 a block at a time and with the short chains).  With two
+// filters that takes registers (12 blocks of 64 channels: 240 VGPRs and 52 us
+// instead of 159 and 39, 16 outputs each): two segments as in a pass, one
+// chain for two-bin lanes, of shorter chunks instead.  16-bit rows lose 2e-4
+// by their storage.
 template <int M, int NF, int HT, int KM>
 struct CallFold {
     using Geo = PassGeo<M, HT>;
+    static constexpr int SEG = NF == 2 ? Geo::SEG : HT == IR_F32 ? 0 : 1;
     static constexpr int kSums = (Geo::G > 1 ? kTickThreads / 2 : 0) + (KM + NF - 1) * kTickThreads * Geo::E / 2;
-    static constexpr int SEG = HT == IR_F32 && (NF == 1 || Geo::E == 1) ? 0 : 1;
-    static constexpr int kRed = SEG == 0 && kSums > tail_red_float4<M>() ? kSums : tail_red_float4<M>();  // float4
+    static constexpr int kRed = SEG != 1 && kSums > tail_red_float4<M>() ? kSums : tail_red_float4<M>();  // float4
 };
 
 // NT: streamed rows; otherwise (rows that the caches hold) ordinary loads.
@@ -1638,14 +1642,21 @@ __global__ __launch_bounds__(kTickThreads) void k_call_pass(CallArgs a)
     const int kA = NF == 2 ? a.xb + 1 : a.n, kB = NF == 2 ? a.xb : a.n;
     for (int s0 = 0; s0 < M; s0 += Geo::S) {
         const size_t at = (size_t)c * a.P * M + s0;
-        // a block's own spectrum (partition 0) is k_call_out's, so the last
-        // block's serves none of the sums
+        // a block's own spectrum (partition 0) is k_call_out's, and the blocks
+        // after the call add the last block's themselves (their heads take
+        // partitions 0 .. k + 1): that one serves none of the sums
         const SweepRows rows = {a.fdl + at, a.X + (size_t)c * a.n * M + s0, a.slot, a.P - 1, a.n - 1};
         const char *HA = reinterpret_cast<const char *>(a.HA) + at * IrRow<HT>::kBytes;
         const char *HB = NF == 2 ? reinterpret_cast<const char *>(a.HB) + at * IrRow<HT>::kBytes : nullptr;
         // this chunk's row of filter f's output k
         auto out = [&](int f, int k) -> float2 * {
-            if (!(f == 0 ? k < kA : k >= kB && k < a.n)) return nullptr;
+            if (k >= a.n) {
+                if (f != NF - 1 || k >= a.n + a.ahead) return nullptr;
+                int r = a.ring0 + k - a.n;
+                if (r >= a.ring) r -= a.ring;
+                return a.sums + r * a.sums_stride + ((size_t)c * a.nchunk + j) * M + s0;
+            }
+            if (!(f == 0 ? k < kA : k >= kB)) return nullptr;
             return a.T + (((size_t)c * (a.n + NF - 1) + k + f) * a.nchunk + j) * M + s0;
         };
         sweep_outputs<M, NF, HT, NT, KM, Fold::SEG>(rows, HA, HB, SA, SB, i0, i1, 1, s0 == 0, kA, kB, red, out);
@@ -3102,7 +3113,17 @@ static hipError_t launch_call_pass(const CallArgs &a, hipStream_t s)
         else if (a.cached) hipLaunchKernelGGL((k_call_pass<M, 1, HT, false, KM>), g, t, 0, s, a); \
         else hipLaunchKernelGGL((k_call_pass<M, 1, HT, true, KM>), g, t, 0, s, a);                \
         break;
-    switch (pass_km(a.n)) {
+    const int outputs = a.n + a.ahead;
+    if (outputs > kPassMax) {
+        if constexpr (PassGeo<M, HT>::E == 1) {
+            if (a.HB) return hipErrorInvalidValue;
+            if (a.cached) hipLaunchKernelGGL((k_call_pass<M, 1, HT, false, kSweepMax>), g, t, 0, s, a);
+            else hipLaunchKernelGGL((k_call_pass<M, 1, HT, true, kSweepMax>), g, t, 0, s, a);
+            return hipGetLastError();
+        }
+        return hipErrorInvalidValue;
+    }
+    switch (pass_km(outputs)) {
         TANX_CALL_KM(4) TANX_CALL_KM(8) TANX_CALL_KM(12) TANX_CALL_KM(16)
     default:
         return hipErrorInvalidValue;
@@ -3403,7 +3424,7 @@ static hipError_t launch_call_m(const CallArgs &a, hipStream_t s, hipEvent_t ev0
 
 hipError_t launch_call(int B, const CallArgs &a, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
 {
-    if (a.n < 1 || a.n > kPassMax || a.n > a.P || a.nchunk < 1 || (a.HB == nullptr) != (a.xb >= a.n) || a.xb < 0)
+    if (a.n < 1 || a.n > kPassMax || a.n > a.P || a.ahead < 0 || a.n + a.ahead > kSweepMax || a.nchunk < 1 || (a.HB == nullptr) != (a.xb >= a.n) || a.xb < 0)
         return hipErrorInvalidValue;
     switch (B) {
     case 64: return launch_call_m<64>(a, s, ev0, ev1);

@@ -146,3 +146,24 @@ def test_error_of_calls(gpu_ctx, C, L, B, n, switch):
     err = [float((y - ref).norm() / ref.norm()) for y in ys]
     assert err[1] <= 1e-6
     assert err[0] <= 1.05 * err[1], err
+
+
+@pytest.mark.parametrize("opt", [{}, {"pass_blocks": 8}, {"pass_blocks": 12}, {"nu_multiple": 16}])
+def test_next_block(gpu_ctx, opt):
+    """A call leaves the sums of the block after it computed: that block is
+    one launch, whatever the call's length."""
+    import torch
+    L, B, C = 65536, 256, 3
+    conv = T.TANConvolution(gpu_ctx, **opt)
+    assert conv.InitGpu(NONUNIFORM if "nu_multiple" in opt else UNIFORM, L, B, C) == T.AMF_OK
+    _update(T.signals.ir_bank(C, L, 0, base_seed=61))(conv)
+    assert conv.EnableTiming(True) == T.AMF_OK
+    x = torch.rand(C, 70 * B, device="cuda")
+    y = torch.empty_like(x)
+    for n in (1, 2, 4, 5, 8, 11, 16, 17, 24, 64, 70):
+        _run(conv, x, y, [n], B)
+        conv.ReadTiming(reset=True)
+        _run(conv, x, y, [1], B)
+        t = conv.ReadTiming(reset=True)
+        assert t["head_launches"] + t["tail_launches"] == 1, (n, t)
+    conv.Terminate()

@@ -30,3 +30,19 @@ def test_few_partitions(sim_built, P, kp, B):  # noqa: F811
 @pytest.mark.parametrize("method", [0, 1], ids=["uniform", "nonuniform"])
 def test_chunk_changes(sim_built, method):  # noqa: F811
     _run("chunk_changes", method=method)
+
+
+@pytest.mark.parametrize("kp,precision", [(0, 0), (2, 0), (4, 0), (4, 1), (7, 0), (8, 2), (12, 0), (16, 0)])
+def test_mixed_uniform(sim_built, kp, precision):  # noqa: F811
+    for seed in (1, 2):
+        _run("mixed", seed=seed, kp=kp, precision=precision)
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_mixed_nonuniform(sim_built, seed):  # noqa: F811
+    _run("mixed", seed=seed, method=1)
+
+
+@pytest.mark.parametrize("method,kp", [(0, 0), (0, 8), (0, 12), (1, 0)])
+def test_next_block(sim_built, method, kp):  # noqa: F811
+    _run("next_block", method=method, kp=kp)
