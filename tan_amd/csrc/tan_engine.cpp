@@ -1552,11 +1552,11 @@ static int call_blocks_max(const tanx_conv *cv)
 
 // Least blocks of a device call that take process_call's three launches.  Few
 // blocks of a small object are two launches of batched heads (5 blocks of 3
-// channels x 4,096 taps: 13.4 us, 14.9 us in three launches; 6 blocks: 16.6
-// against 15.2 us), but a pass over many rows costs more than a launch (5 blocks of 64
-// channels x 65,536 taps: 30.6 against 25.4 us), and heads above
-// kHeadBatchMaxB are a launch each (4 blocks of 64 channels x 16,384 taps at
-// B = 1024: 47.2 against 26.5 us).
+// channels x 4,096 taps: 13.4 us, 14.9 us in three launches; 6 blocks: 16.0
+// against 13.7 us), but a pass over many rows costs more than a launch (5 blocks of 64
+// channels x 65,536 taps: 29.4 against 24.3 us), and heads above
+// kHeadBatchMaxB are a launch each (4 blocks of 64 channels x 65,536 taps at
+// B = 1024: 57.3 against 31.0 us).
 static size_t call_blocks_min(const tanx_conv *cv)
 {
     const size_t rows = (size_t)cv->C * cv->P * cv->B * (sizeof(float2) + ir_elem_bytes(cv->irtype));
@@ -1607,7 +1607,10 @@ static int call_ahead(const tanx_conv *cv, int n, long long e, bool two)
 // leave the partial sums of the blocks after the call as every block does: in
 // one sweep with the call's own, or in one more sweep over the rows.  A block
 // at a time is a sweep every kp blocks, so a call of any length, and any mix
-// of calls, sweeps no more than before.
+// of calls, sweeps no more than that.  1,024 channels x 65,536 taps, a call
+// and a single block in turn: 4 and 1 blocks 275 to 252 us, 400 when the
+// single block had to compute its sums; 8 and 1 blocks 485 to 278 us (434);
+// that single block 27 us (193).
 static bool call_pays(const tanx_conv *cv, size_t nb)
 {
     const size_t most = (size_t)std::max(1, call_blocks_max(cv));
@@ -1979,9 +1982,10 @@ static int32_t process_host_block(tanx_conv *cv, const float *const *in, float *
     for (int ch = 0; ch < cv->C; ch++) std::memcpy(cv->hin + ch * B, in[ch] + off, B * sizeof(float));
     hipStream_t s = cv->ctx->proc;
     // the head reads and writes the pinned blocks itself: a transfer before and
-    // one after it cost more than its few PCIe round trips (2 channels at
-    // B = 1024: 36.4 to 32.4 us, 31 channels 161 to 136 us, 1 channel at B = 64
-    // 27.1 to 22.0 us; input by a fetch launch, output direct: 34.9, 141, 25.4)
+    // one after it cost more than its few PCIe round trips, whatever the size (1
+    // channel at B = 64 20.8 to 17.8 us, 31 at B = 1024 55.5 to 31.1, 512 at B = 256
+    // 90.9 to 61.5, 1,024 at B = 1024, 8 MB in all, 384 to 356; input by a fetch
+    // launch, output direct: slower than this at 1, 2 and 31 channels)
     int32_t rc = process_block(cv, cv->hin, (long long)B, cv->hout, (long long)B, n, flags, false);
     if (rc != TANX_OK) return rc;
     TANX_CHECK(hipEventRecord(cv->ev_out, s));

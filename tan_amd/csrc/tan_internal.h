@@ -418,6 +418,15 @@ struct RoomEar {
     float late_scale;
     int late_total;
 };
+// d / 340, the IEEE quotient's bits for every float from 2^-31 to 2^37 (the few
+// below round to sample 0 either way): the quotient by the rounded
+// reciprocal, corrected by its remainder (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990).
+__host__ __device__ inline float div340(float d)
+{
+    const float rc = 1.0f / 340.0f, q = d * rc;
+    return fmaf(fmaf(-340.0f, q, d), rc, q);
+}
 constexpr int kRoomWindow = 8192;  // output samples per late-image window (32 KB of LDS)
 // RoomEar of the left (out[0]) and right (out[1]) ear; AMF_RESULT value.
 int32_t room_ears(const tanx_room *room, const tanx_source *source, const tanx_listener *ears, int fs, int len,

@@ -2086,9 +2086,10 @@ __global__ __launch_bounds__(256) void k_ir_transform_rows_group(const IrArgs *_
 // t holds the points t + s N/16, s < 16, and the last stage leaves the
 // results in the same places, so global memory is read and written straight
 // from registers, coalesced.  (Radix-4 stages that go through LDS each time
-// made five of it, and two buffers: 2,000 points of 1,000 channels took 9.6
-// us as 1,000 workgroups of four waves, now one wave each; TANFFT of 12
-// channels x 2^18 points 83 to 45 us.)
+// made five of it, and two buffers: TANFFT of 12 channels x 2^18 points 83 to
+// 44 us.  2,048-point real transforms of 1,000 channels are no faster as one
+// wave each than as workgroups of four, 9.6 and 9.7 us: one wave per SIMD
+// waits for its own loads and stores.)
 // ---------------------------------------------------------------------------
 template <bool INV>
 __device__ __forceinline__ float2 mul_ni(float2 v)  // v W_4 (forward -i, inverse +i)

@@ -176,16 +176,6 @@ __device__ __forceinline__ ImageParams image_params(const RoomEar &E)
     return p;
 }
 
-// d / 340, the IEEE quotient's bits (checked for every float from 2^-31 to
-// 2^37; the few below round to sample 0 either way): the quotient by the
-// rounded reciprocal, corrected by its remainder (Markstein, "Computation of
-// elementary functions on the IBM RISC System/6000 processor", 1990).
-__device__ __forceinline__ float div340(float d)
-{
-    const float rc = 1.0f / 340.0f, q = d * rc;
-    return fmaf(fmaf(-340.0f, q, d), rc, q);
-}
-
 // Late images of one window of kRoomWindow output samples [w0, w0 +
 // kRoomWindow), w0 = wstart + window * kRoomWindow, and one slice of the
 // image lattice's rows (iy, iz): the images arriving in the window lie in a
