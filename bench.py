@@ -959,10 +959,11 @@ PMC_JSON = os.path.join(ROOT, "profiles", "pmc_traffic_k_group_tick_rt.json")
 
 
 PROFILE_LEGS = {
-    "c2": ("k_window_64ch_65536taps_b256.txt",
+    "c2": ("calls_64ch_65536taps_b256.txt",
            "one 64-channel object x 65,536 taps, B = 256, 2,000 blocks in calls of 50 blocks, a fresh IR "
-           "every 50 blocks (the c2_64ch leg): fused launches of up to 4 heads with the 4-block pass after "
-           "them, tail chunks pinned to 8; the object's rows (100 MB) stay in the Infinity Cache"),
+           "every 50 blocks (the c2_64ch leg): three launches per 13 blocks (spectra, one sweep, inverse "
+           "transforms) and one pass for the blocks after the call, its tail chunks pinned to 8; the object's "
+           "rows (100 MB) stay in the Infinity Cache"),
     "serving": ("k_group_tick_serving.txt",
                 "the served mixed workload (Poisson sessions, 20/s, mean life 30 s, 1-16 channels, IR "
                 "8,192-524,288 taps, B = 256, an IR update every 10-100 blocks; about 620 sessions / 5,300 "
@@ -996,6 +997,20 @@ def profile_leg(T, torch, leg):
     log(f"profile leg {leg} done")
 
 
+def profile_case(torch, name, passes=60):
+    """One listed case of perf/cases.py: after a tensor addition that marks
+    the end of its preparation, `passes` passes over three states in turn."""
+    from perf import cases
+    case = next(c for c in cases.listed() if c["name"] == name)
+    states = [cases.prepare(case, k) for k in range(3)]
+    torch.zeros(7, device="cuda").add_(1.0)
+    torch.cuda.synchronize()
+    for i in range(passes):
+        cases.run(states[i % 3])
+    torch.cuda.synchronize()
+    log(f"profile case {name} done")
+
+
 def summarize_trace(run_dir, leg):
     """Writes profiles/<leg's file> from the kernel statistics of a traced
     `bench.py --profile-run --profile-leg <leg>` under run_dir/prof_<leg>."""
@@ -1009,7 +1024,7 @@ def summarize_trace(run_dir, leg):
     for r in stats:
         if float(r["Percentage"]) < 0.05:
             continue
-        lines.append(f"{r['Name'].split('(')[0].replace('void ', '')[:64]:64s} {int(r['Calls']):6d} "
+        lines.append(f"{r['Name'].replace('(anonymous namespace)::', '').split('(')[0].replace('void ', '')[:64]:64s} {int(r['Calls']):6d} "
                      f"{float(r['AverageNs']) / 1e3:10.1f} {float(r['MinNs']) / 1e3:10.1f} "
                      f"{float(r['MaxNs']) / 1e3:10.1f} {float(r['Percentage']):7.2f}")
     out = os.path.join(ROOT, "profiles", name)
@@ -1099,7 +1114,7 @@ def summarize_profiles(run_dir, groups):
              "staggered, with its crossfade); the first ticks include cold caches (the Max column).", "",
              f"{'kernel':64s} {'calls':>6s} {'avg us':>10s} {'min us':>10s} {'max us':>10s} {'% time':>7s}"]
     for r in stats:
-        lines.append(f"{r['Name'].split('(')[0].replace('void ', '')[:64]:64s} {int(r['Calls']):6d} "
+        lines.append(f"{r['Name'].replace('(anonymous namespace)::', '').split('(')[0].replace('void ', '')[:64]:64s} {int(r['Calls']):6d} "
                      f"{float(r['AverageNs']) / 1e3:10.1f} {float(r['MinNs']) / 1e3:10.1f} "
                      f"{float(r['MaxNs']) / 1e3:10.1f} {float(r['Percentage']):7.2f}")
     lines += ["", f"Group kernels per tick: {gt_ns / PROFILE_TICKS / 1e3:.1f} us (all k_group_tick and "
@@ -1149,6 +1164,8 @@ def main():
                          "--summarize-profiles: which summary to write")
     ap.add_argument("--serving-only", action="store_true",
                     help="run the serving legs alone and print their rows as one JSON line (no headline)")
+    ap.add_argument("--profile-case", type=str, default="",
+                    help="with --profile-run: this listed case of perf/cases.py instead of a leg")
     ap.add_argument("--profile-run", action="store_true",
                     help="short fixed workload for rocprofv3 counter passes; prints no JSON")
     args = ap.parse_args()
@@ -1171,7 +1188,9 @@ def main():
     import tan_amd as T
     T.load_library()
     if args.profile_run:
-        if args.profile_leg == "rt":
+        if args.profile_case:
+            profile_case(torch, args.profile_case)
+        elif args.profile_leg == "rt":
             profile_run(T, torch, args.rt_groups or PROFILE_GROUPS)
         else:
             profile_leg(T, torch, args.profile_leg)
@@ -1227,8 +1246,8 @@ def main():
         c2 = {"channels": C, "blocks": 2000, "ir_updates": 40, "wall_ms": dt * 1e3,
               "rt_channels_throughput": C * 2000 * B / FS / dt, "ms_per_update_period": dt / 40 * 1e3,
               "pass_blocks": info.get("pass_blocks"), "tail_chunks": info.get("tail_chunks"),
-              "k_window_avg_us": pass_us,
-              "k_window_alg_GBps": kt["tail_alg_bytes"] / (kt["tail_ms"] * 1e-3) / 1e9 if kt["tail_ms"] else None,
+              "launches_avg_us": pass_us,
+              "launches_alg_GBps": kt["tail_alg_bytes"] / (kt["tail_ms"] * 1e-3) / 1e9 if kt["tail_ms"] else None,
               "kernel_us_per_block": (kt["head_ms"] + kt["tail_ms"]) * 1e3 / kt["blocks"],
               "note": "64-channel rows (~100 MB) stay in the Infinity Cache; not an HBM figure"}
         log(f"  {c2['rt_channels_throughput']:.0f} real-time channels of throughput at 64 channels")

@@ -222,9 +222,12 @@ int32_t tanx_conv_process(tanx_conv *conv, const float *const *in, float *const 
                           size_t n, const uint32_t *flags, size_t *processed);
 /* Device-memory variant (stands in for Process(cl_mem[], cl_mem[])):
  * channel c reads block b at d_in + c * in_stride + b * block and writes
- * d_out + c * out_stride + b * block.  Asynchronous: ordered on the
- * library's process stream; use tanx_conv_synchronize before reading d_out
- * on the host. */
+ * d_out + c * out_stride + b * block; d_out may be d_in.  Asynchronous:
+ * ordered on the library's process stream; use tanx_conv_synchronize before
+ * reading d_out on the host.  A call of several blocks may add the
+ * partitions of each output in another order than a block at a time does
+ * (other bits within the same error against FP64); like a block, it ends with
+ * the partial sums of the next block computed. */
 int32_t tanx_conv_process_device(tanx_conv *conv, const float *d_in, size_t in_stride,
                                  float *d_out, size_t out_stride, size_t n,
                                  const uint32_t *flags, size_t *processed);
@@ -328,13 +331,16 @@ int32_t tanx_conv_set_tail_chunks(tanx_conv *conv, uint32_t chunks);
 int32_t tanx_conv_autotune(tanx_conv *conv, uint32_t *chunks, double *us_per_block);
 /* Device-memory Process runs each block's head and the next block's tail
  * multiply-accumulate in one launch (default 1); 0 launches them separately
- * as the host-memory path does.  Results are identical either way. */
+ * as the host-memory path does.  Results are identical either way for calls
+ * of one block; when fused, a call of several takes them together where it
+ * can, which adds the partitions in another order. */
 int32_t tanx_conv_set_fused(tanx_conv *conv, uint32_t fused);
 /* Device-memory Process over two or more blocks (no channel flags, fused,
  * timing off) replays a captured hipGraph of one tick launch per block,
  * whose arguments come from a descriptor array copied once per batch of up
- * to 64 blocks (default 1); 0 launches each block directly.  Results are
- * identical either way. */
+ * to 64 blocks; 0 (the default) launches each block directly.  It applies to
+ * objects without multi-block passes or frames, whose results are identical
+ * either way. */
 int32_t tanx_conv_set_graph(tanx_conv *conv, uint32_t use_graph);
 /* Kernel timing: when enabled, HIP events are recorded on the process
  * stream around every launch.  "head" counts launches that carry the head
