@@ -2243,10 +2243,28 @@ __device__ __forceinline__ void st_pair(float *p, float2 v, bool al8)
     }
 }
 
-// Transforms of 64..2,048 complex points: workgroups of one wave (two at
+// Transforms of 128..2,048 complex points: workgroups of one wave (two at
 // 2,048 points), 1,024 / M channels each.  M is the complex size (N for
 // complex directions, N/2 for real ones).
 constexpr int fft_threads_of(int M) { return M / 16 > 64 ? M / 16 : 64; }
+
+// Whether a transform runs in registers (k_fft) or through LDS (k_fft_lds).
+// In registers a lane does sixteen points' work on its own, which pays once
+// there are many waves, or stages; the real forward directions also unpack in
+// that lane.  Kernel times in us, LDS and registers: complex 64 points of
+// 1,000 channels 3.4 and 4.3, 128 points 3.8 and 4.0 (4,096 channels 5.2 and
+// 4.9), 256 points of 1,000 channels 4.8 and 4.1; real inverse 2 x 256 points
+// of 64 and 1,000 channels 4.8 and 4.9, 5.6 and 5.2, 2 x 1,024 points 6.0 both
+// and 9.5 and 8.5; real forward 2 x 128 points of 1,000 channels 4.2 and 6.5, 2
+// x 512 points of 1,000 and 4,096 channels 6.9 and 8.0, 16.3 and 12.1, 2 x 2,048
+// points of 64 and 1,000 channels 7.7 and 7.9, 19 and 14.
+static bool fft_in_regs(int mode, int M, int channels)
+{
+    const long long points = (long long)channels * M;
+    if (mode == 2 || mode == 4) return M >= 256 && points >= 1000000;
+    if (mode < 2) return M >= 256 || (M == 128 && points >= 3 << 16);
+    return M >= 1024 || (M >= 256 && points >= 3 << 16);
+}
 
 template <int M>
 __global__ __launch_bounds__(fft_threads_of(M)) void k_fft(FftArgs a, int channels, bool al8)
@@ -2330,9 +2348,11 @@ __global__ __launch_bounds__(fft_threads_of(M)) void k_fft(FftArgs a, int channe
     for (int s = 0; s < 16; s++) st_pair(out + 2 * (t + s * NT), make_float2(x[s].x * sc, x[s].y * sc), al8);
 }
 
-// Fewer than 64 complex points: one workgroup per channel
+// One workgroup per channel, radix-4 stages through LDS: transforms of fewer
+// than 64 complex points, and those that leave the device mostly idle
+// (fft_in_regs)
 template <int M>
-__global__ __launch_bounds__(M / 4 > 64 ? (M / 4 < 1024 ? M / 4 : 1024) : 64) void k_fft_small(FftArgs a)
+__global__ __launch_bounds__(M / 4 > 64 ? (M / 4 < 1024 ? M / 4 : 1024) : 64) void k_fft_lds(FftArgs a)
 {
     __shared__ float2 s0[M > 1 ? M : 2], s1[M > 1 ? M : 2], s2[M > 1 ? M : 2];
     const int c = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
@@ -2559,7 +2579,7 @@ __global__ __launch_bounds__(256) void k_fft4_c2r_pre(const float *in, long long
 // ---------------------------------------------------------------------------
 // Time-domain convolution (see TdArgs), 256 threads, window and filters in LDS.
 //
-// A lane computes R consecutive outputs: eight taps (two float4 of the
+// A lane computes R = 1, 2 or 4 consecutive outputs: eight taps (two float4 of the
 // filter, the same for every lane) against a window of R + 7 samples kept in
 // registers, of which eight are new per step.  At R = 4 a step is 32
 // multiply-adds on two ds_read_b128 of samples; one output per lane read 16
@@ -2597,7 +2617,10 @@ __device__ __forceinline__ void td_dot(const float *w0, const float *h, int taps
         const float hv[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
 #pragma unroll
         for (int t = R - 2; t >= 0; t--) win[t + 8] = win[t];
-        if constexpr (R % 4 == 0) {
+        if constexpr (R == 1) {
+#pragma unroll
+            for (int t = 0; t < 8; t++) win[t] = (w - k)[t];
+        } else if constexpr (R % 4 == 0) {
 #pragma unroll
             for (int t = 0; t < 8; t += 4) {
                 const float4 v = *reinterpret_cast<const float4 *>(w - k + t);
@@ -2669,11 +2692,13 @@ __global__ __launch_bounds__(256) void k_td(TdArgs a)
     const float step = (float)(1.0 / (double)a.B);
     const float *w0 = w + len - 1 - f0;
     // the lanes beyond those that the n outputs need share the taps: slice s of
-    // the 2^ls slices (of at least 128 taps) sums taps from s * per on, which
-    // shortens the lanes' chains (7 channels x 1,070 taps, B = 64: 20.9 to 8.3 us)
+    // the 2^ls slices (of at least 128 taps, 64 at one output per lane) sums
+    // taps from s * per on, which shortens the lanes' chains (7 channels x 1,070
+    // taps, B = 64: 20.9 to 8.3 us)
+    constexpr int kSlice = R == 1 ? 64 : 128;
     const int lanes = (n + R - 1) / R;
     int ls = 0;
-    while (ls < 3 && (lanes << (ls + 1)) <= nt && (taps >> (ls + 1)) >= 128) ls++;
+    while (ls < 3 && (lanes << (ls + 1)) <= nt && (taps >> (ls + 1)) >= kSlice) ls++;
     const int per = ((taps + 7) / 8 + (1 << ls) - 1) / (1 << ls) * 8;
     float *part = hb + (a.Hb ? len : 0);  // [2 filters][slices][n] partial sums
     const int sl = ls == 0 ? 0 : tid / lanes, k0 = min(taps, sl * per), cnt = min(per, taps - k0);
@@ -2823,29 +2848,28 @@ __global__ __launch_bounds__(64 * kDftWaves) void k_dft_mfma(const float *__rest
 // Sum of the channels in channel order (the reference's order), channel c at
 // ins[c] (LIST: device pointer list) or at in + c * stride.  A block of audio
 // is a few hundred samples, so the sum is one lane's chain of loads: the
-// channels' samples are loaded kMixBatch at a time (one memory round trip)
-// and then added in order, on workgroups of one wave that spread over the
-// compute units: 2.9 instead of 8.8 us for 32 channels of 256 samples.
-constexpr int kMixBatch = 16, kMixThreads = 64;
-
-template <bool LIST>
-__global__ __launch_bounds__(kMixThreads) void k_mix(const float *const *__restrict__ ins,
-                                                     const float *__restrict__ in, long long stride, int channels,
-                                                     long long n, float *__restrict__ out)
+// channels' samples are loaded BATCH at a time (one memory round trip) and
+// then added in order: 2.2 us for 32 channels of 256 samples, 4.7 a channel at
+// a time, 22.7 and 25.5 us for 10^6 samples.  The smallest of 2, 4, 8 and 16
+// that holds the channels (16 beyond): loading a single channel's samples
+// sixteen times took 7.7 us at 10^6, 3.4 twice.
+template <bool LIST, int BATCH>
+__global__ __launch_bounds__(256) void k_mix(const float *const *__restrict__ ins, const float *__restrict__ in,
+                                             long long stride, int channels, long long n, float *__restrict__ out)
 {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
         float acc = 0.f;
-        for (int c0 = 0; c0 < channels; c0 += kMixBatch) {
-            float v[kMixBatch];
+        for (int c0 = 0; c0 < channels; c0 += BATCH) {
+            float v[BATCH];
             // channels past the last one load it again, unused
 #pragma unroll
-            for (int u = 0; u < kMixBatch; u++) {
+            for (int u = 0; u < BATCH; u++) {
                 const int c = min(c0 + u, channels - 1);
                 if constexpr (LIST) v[u] = gld(ins[c] + i);
                 else v[u] = in[(size_t)c * stride + i];
             }
 #pragma unroll
-            for (int u = 0; u < kMixBatch; u++)
+            for (int u = 0; u < BATCH; u++)
                 if (c0 + u < channels) acc = c0 + u == 0 ? v[u] : acc + v[u];
         }
         out[i] = acc;
@@ -3579,18 +3603,26 @@ hipError_t launch_fft(int channels, const FftArgs &a, hipStream_t s)
     const bool real = a.mode >= 2;
     const int M = real ? (1 << (a.log2len - 1)) : (1 << a.log2len);
     if (M > kFftLdsMax) return launch_fft4(channels, a, s);
+    if (!fft_in_regs(a.mode, M, channels)) {
+        switch (M) {
+#define TANX_FFT_CASE(V) case V: hipLaunchKernelGGL(k_fft_lds<V>, dim3(channels), dim3(fft_threads(V)), 0, s, a); break;
+            TANX_FFT_CASE(1) TANX_FFT_CASE(2) TANX_FFT_CASE(4) TANX_FFT_CASE(8) TANX_FFT_CASE(16) TANX_FFT_CASE(32)
+            TANX_FFT_CASE(64) TANX_FFT_CASE(128) TANX_FFT_CASE(256) TANX_FFT_CASE(512) TANX_FFT_CASE(1024)
+            TANX_FFT_CASE(2048)
+#undef TANX_FFT_CASE
+        default:
+            return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    }
     const bool al8 = ((reinterpret_cast<uintptr_t>(a.in) | reinterpret_cast<uintptr_t>(a.out)) & 7) == 0 && a.stride % 2 == 0;
     switch (M) {
-#define TANX_FFT_CASE(V) case V: hipLaunchKernelGGL(k_fft_small<V>, dim3(channels), dim3(64), 0, s, a); break;
-        TANX_FFT_CASE(1) TANX_FFT_CASE(2) TANX_FFT_CASE(4) TANX_FFT_CASE(8) TANX_FFT_CASE(16) TANX_FFT_CASE(32)
-#undef TANX_FFT_CASE
 #define TANX_FFT_CASE(V)                                                                                       \
     case V:                                                                                                    \
         hipLaunchKernelGGL(k_fft<V>, dim3((unsigned)((channels * (V / 16) + fft_threads_of(V) - 1) / fft_threads_of(V))), \
                            dim3(fft_threads_of(V)), 0, s, a, channels, al8);                                   \
         break;
-        TANX_FFT_CASE(64) TANX_FFT_CASE(128) TANX_FFT_CASE(256) TANX_FFT_CASE(512) TANX_FFT_CASE(1024)
-        TANX_FFT_CASE(2048)
+        TANX_FFT_CASE(128) TANX_FFT_CASE(256) TANX_FFT_CASE(512) TANX_FFT_CASE(1024) TANX_FFT_CASE(2048)
 #undef TANX_FFT_CASE
     default:
         return hipErrorInvalidValue;
@@ -3606,9 +3638,14 @@ hipError_t launch_td(const TdArgs &a, hipStream_t s, hipEvent_t ev0, hipEvent_t 
     // per filter: 8 slices of the outputs that fill the workgroup)
     const size_t filters = a.Hb ? 2 : 1;
     const size_t smem = sizeof(float) * ((size_t)a.len + a.B + kTdPad + filters * ((size_t)a.len + 1024));
-    // four outputs per lane once their waves cover the chip's 1,024 SIMDs, two below
+    // four outputs per lane once their waves cover the chip's 1,024 SIMDs, two
+    // below; one where a channel has so little to do that more would leave most
+    // of its wave idle (64 taps, n = 64: 2,048 channels 4.9 us, 7.4 at four, 4.6
+    // before there were several; 64 channels 3.7, 4.3 at two, 3.7; 256 taps: 7.7,
+    // 10.7, 7.9 and 4.3, 5.0, 5.3)
     const long long waves4 = (long long)a.C * ((a.n + 255) / 256);
-    if (waves4 >= 1024) hipExtLaunchKernelGGL((k_td<4>), dim3(a.C), dim3(256), smem, s, ev0, ev1, 0, a);
+    if ((long long)a.n * a.len <= 64 * 256) hipExtLaunchKernelGGL((k_td<1>), dim3(a.C), dim3(256), smem, s, ev0, ev1, 0, a);
+    else if (waves4 >= 1024) hipExtLaunchKernelGGL((k_td<4>), dim3(a.C), dim3(256), smem, s, ev0, ev1, 0, a);
     else hipExtLaunchKernelGGL((k_td<2>), dim3(a.C), dim3(256), smem, s, ev0, ev1, 0, a);
     return hipGetLastError();
 }
@@ -3642,13 +3679,23 @@ static unsigned io_blocks(long long n)
     return (unsigned)(b < 1 ? 1 : b);
 }
 
+template <int BATCH>
+static void launch_mix_batch(const float *const *d_ins, const float *d_in, long long stride, int channels, long long n,
+                             float *d_out, hipStream_t s)
+{
+    const dim3 g(io_blocks(n)), t(256);
+    if (d_ins) hipLaunchKernelGGL((k_mix<true, BATCH>), g, t, 0, s, d_ins, d_in, stride, channels, n, d_out);
+    else hipLaunchKernelGGL((k_mix<false, BATCH>), g, t, 0, s, d_ins, d_in, stride, channels, n, d_out);
+}
+
 hipError_t launch_mix(const float *const *d_ins, const float *d_in, long long stride, int channels, long long n,
                       float *d_out, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    const dim3 g((unsigned)std::min<long long>((n + kMixThreads - 1) / kMixThreads, 16384)), t(kMixThreads);
-    if (d_ins) hipLaunchKernelGGL((k_mix<true>), g, t, 0, s, d_ins, d_in, stride, channels, n, d_out);
-    else hipLaunchKernelGGL((k_mix<false>), g, t, 0, s, d_ins, d_in, stride, channels, n, d_out);
+    if (channels <= 2) launch_mix_batch<2>(d_ins, d_in, stride, channels, n, d_out, s);
+    else if (channels <= 4) launch_mix_batch<4>(d_ins, d_in, stride, channels, n, d_out, s);
+    else if (channels <= 8) launch_mix_batch<8>(d_ins, d_in, stride, channels, n, d_out, s);
+    else launch_mix_batch<16>(d_ins, d_in, stride, channels, n, d_out, s);
     return hipGetLastError();
 }
 
