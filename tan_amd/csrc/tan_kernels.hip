@@ -856,7 +856,7 @@ struct SweepRows {
 // NF filters: HA for outputs k < kA, HB (NF = 2) for outputs k >= kB; with
 // one filter every output is computed (the caller stores those it wants).
 // SEG = 2: fold() is called once between the partitions before pf and those
-// from pf on (p0 < pf < p1), to put the sums so far aside; the trips are laid
+// from pf on (p0 < pf < p1), to put the sums so far aside; the stages are laid
 // so that one starts at pf and the loads in flight go on across it.  SEG = 0:
 // it is called after every kFold partitions but the last.
 template <int NF, int KM, int SEG, int E>
@@ -883,8 +883,8 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
     // -(i + q)) for the trip starting at partition i; output k reads the
     // entry k before it
     Bins<E> win[KM - 1 + kBody];
-    // partitions the first trip skips
-    const int lead = FOLD && pf > p0 && pf < p1 ? (kBody - (pf - p0) % kBody) % kBody : 0;
+    // partitions the first stage skips
+    const int lead = FOLD && pf > p0 && pf < p1 ? (U - (pf - p0) % U) % U : 0;
 #pragma unroll
     for (int k = 0; k < KM; k++)
 #pragma unroll
@@ -894,7 +894,7 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
         }
     // the rows before partition p0 that its outputs reach back to
 #pragma unroll
-    for (int t = 0; t < KM - 1 + (FOLD ? kBody : 0); t++) {
+    for (int t = 0; t < KM - 1 + (FOLD ? U : 0); t++) {
 #pragma unroll
         for (int e = 0; e < E; e++) win[t].re[e] = win[t].im[e] = 0.f;
         const int back = KM - 1 + lead - t;  // entry t: partition p0 - back
@@ -924,9 +924,10 @@ __device__ __forceinline__ void pass_sweep(const SweepRows &rows, const char *HA
     };
     load(cur, p0 - lead);
     for (int i = p0 - lead; i < p1; i += kBody) {
-        if (SEG == 2 ? i == pf && i > p0 : SEG == 0 && i > p0 && (i - p0) % kFold == 0) fold();
+        if (SEG == 0 && i > p0 && (i - p0) % kFold == 0) fold();
 #pragma unroll
         for (int q0 = 0; q0 < kBody; q0 += U) {
+            if (FOLD && i + q0 == pf && pf > p0 && pf < p1) fold();
             load(nxt, i + q0 + U);
             // the loads stay before the products (moved to their use they would not
             // be in flight: 38 instead of 28 us in the call of 16 blocks below)
