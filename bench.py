@@ -946,11 +946,11 @@ def profile_run(T, torch, ngroups):
 
 
 PROFILE_CMDS = {
-    "trace": "rocprofv3 --kernel-trace --stats --output-format csv -d <repo>/gpurun_out/prof_rt -o run -- "
+    "trace": "rocprofv3 --kernel-trace --stats --output-format csv -d <out>/prof_rt -o run -- "
              "python3 <repo>/bench.py --profile-run --rt-groups {g}",
-    "fetch": "rocprofv3 --pmc FETCH_SIZE --output-format csv -d <repo>/gpurun_out/pmc_fetch -o run -- "
+    "fetch": "rocprofv3 --pmc FETCH_SIZE --output-format csv -d <out>/pmc_fetch -o run -- "
              "python3 <repo>/bench.py --profile-run --rt-groups {g}",
-    "write": "rocprofv3 --pmc WRITE_SIZE --output-format csv -d <repo>/gpurun_out/pmc_write -o run -- "
+    "write": "rocprofv3 --pmc WRITE_SIZE --output-format csv -d <out>/pmc_write -o run -- "
              "python3 <repo>/bench.py --profile-run --rt-groups {g}",
 }
 PROFILE_TICKS = 200
@@ -1018,7 +1018,7 @@ def summarize_trace(run_dir, leg):
     name, what = PROFILE_LEGS[leg]
     stats = list(csv.DictReader(open(os.path.join(run_dir, f"prof_{leg}", "run_kernel_stats.csv"))))
     cmd = (f"cd /tmp && export TMPDIR=/tmp && rocprofv3 --kernel-trace --stats --output-format csv -d "
-           f"<repo>/gpurun_out/prof_{leg} -o run -- python3 <repo>/bench.py --profile-run --profile-leg {leg}")
+           f"<out>/prof_{leg} -o run -- python3 <repo>/bench.py --profile-run --profile-leg {leg}")
     lines = [f"# Kernel trace: {what}", "", "Command (from the repository root on the GPU box):", "  " + cmd, "",
              f"{'kernel':64s} {'calls':>6s} {'avg us':>10s} {'min us':>10s} {'max us':>10s} {'% time':>7s}"]
     for r in stats:
